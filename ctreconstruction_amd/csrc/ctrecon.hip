@@ -6,7 +6,8 @@
 //   dd_forward_kernel           one wavefront per (2 views, 4 detector columns, 63 rows)
 //   dd_forward_zslab_kernel     z-slab views (non-circular geometries), FP64 loops per cell
 //   bp_geometry_kernel          per-view backprojection constants, FP64 -> FP32
-//   dd_backproject_tile_kernel  one workgroup per 16 x 16 x ZC voxel tile, windows in LDS
+//   dd_backproject_tile_kernel  one workgroup per 16 x 16 x ZC voxel tile and view split, windows in LDS
+//   bp_reduce_kernel            sums the view splits' partial volumes in a fixed order
 //   adj_geometry_kernel         per-view constants of the inverse central projection
 //   adj_rowprefix_kernel        row prefix sums of projections times path length
 //   dd_adjoint_kernel           exact transpose of the forward projector, gathered per voxel
@@ -1379,12 +1380,21 @@ __device__ inline void bp_column_view(const BpView& v, const float* __restrict__
 
 // KIND: kBpFast writes the volume and sets flags[tile][view] for every view it leaves (in
 // part or whole) to kBpRest, which adds those contributions; kBpAll does everything.
+// blockIdx.y is the view split: split s takes the views [s * views_per, (s + 1) * views_per) of
+// its tile and, where there is more than one, writes its sums to its own copy of the volume in
+// `parts`, which bp_reduce_kernel adds up in split order (see bp_split).
 template <int ZC, int KIND>
 __global__ void __launch_bounds__(256) dd_backproject_tile_kernel(
     const float* __restrict__ q, float* __restrict__ vol, const float* __restrict__ vt,
-    uint8_t* __restrict__ flags, int nx, int ny, int nz, int nu, int nv, int n_views, float x0,
-    float y0, float z0, float dx, float dy, float dz, int curved, float scale, float zero_tol,
-    int accumulate, int tiles_x, int tiles_y, int tiles_z) {
+    uint8_t* __restrict__ flags, float* __restrict__ parts, int nx, int ny, int nz, int nu, int nv,
+    int all_views, int views_per, float x0, float y0, float z0, float dx, float dy, float dz, int curved,
+    float scale, float zero_tol, int accumulate, int tiles_x, int tiles_y, int tiles_z) {
+    // from here on the split's views are views 0 .. n_views - 1
+    const int view_first = blockIdx.y * views_per;
+    const int n_views = min(views_per, all_views - view_first);
+    q += (size_t)view_first * nv * nu;
+    vt += (size_t)view_first * kBpViewStride;
+    if (gridDim.y > 1) vol = parts + (size_t)blockIdx.y * nx * ny * nz;
     __shared__ float win[2][kWinCap + kMaxUTaps - 1];
     __shared__ int4 wring[kWinRing];
     __shared__ float scan_lds[(kMaxRows + 3) * 256];
@@ -1397,7 +1407,7 @@ __global__ void __launch_bounds__(256) dd_backproject_tile_kernel(
     const int tx = t % tiles_x;
     const int ty = (t / tiles_x) % tiles_y;
     const int tz = t / (tiles_x * tiles_y);
-    uint8_t* __restrict__ tflags = (KIND == kBpAll) ? nullptr : flags + (size_t)t * n_views;
+    uint8_t* __restrict__ tflags = (KIND == kBpAll) ? nullptr : flags + (size_t)t * all_views + view_first;
     if constexpr (KIND == kBpRest) {
         // nothing left for this tile: done
         int any = 0;
@@ -1562,6 +1572,20 @@ __global__ void __launch_bounds__(256) dd_backproject_tile_kernel(
         else
             vol[idx] = accumulate ? vol[idx] + acc[i] : acc[i];
     }
+}
+
+// vol = (accumulate ? vol : 0) + the splits' partial volumes, in split order (deterministic).
+// One 16-byte load per split and thread where the volume's size and address allow it (W = 4).
+template <int W>
+__global__ void __launch_bounds__(256) bp_reduce_kernel(const float* __restrict__ parts, float* __restrict__ vol,
+                                                        size_t n, int splits, int accumulate) {
+    typedef float vec __attribute__((ext_vector_type(W)));
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * W;
+    if (i >= n) return;
+    vec sum = *reinterpret_cast<const vec*>(parts + i);
+    for (int s = 1; s < splits; ++s) sum += *reinterpret_cast<const vec*>(parts + (size_t)s * n + i);
+    vec* out = reinterpret_cast<vec*>(vol + i);
+    *out = accumulate ? *out + sum : sum;
 }
 
 __global__ void __launch_bounds__(256) fill_zero_kernel(uint32_t* __restrict__ p, size_t n) {
@@ -2342,11 +2366,111 @@ size_t bp_tiles(const ctr_geometry* g) {
            ((g->nz + kBpZC - 1) / kBpZC);
 }
 
+// workspace of the FDK backprojection without view splits, and the offset of the splits' volumes
+size_t bp_base_bytes(const ctr_geometry* g) {
+    return align_up((size_t)g->n_views * kBpViewStride * sizeof(float), 256) +
+           align_up(bp_tiles(g) * g->n_views, 256);
+}
+
+// View splits of the FDK backprojection.  A tile's views are a serial chain, and a volume of few
+// tiles leaves most of the 256 CUs (five groups each) idle: 32 tiles at 64^3 took 617 us, one per
+// CU at 256^2 x 1 took 1012 us.  Below kBpTargetGroups tiles the views are therefore shared out to
+// so many groups per tile that about kBpTargetGroups run, each summing into its own copy of the
+// volume, added up by bp_reduce_kernel: 98 and 592 us there, 1.91 -> 1.38 ms at 151 x 163 x 107 x
+// 241 views, 4.16 -> 3.89 ms at 256^3 x 360 views (2048 tiles: a nearly empty last wave).  2560 and
+// 10240 groups are up to 10 % slower on those than 5120 (too few in flight; more copies to add).
+// A split keeps at least kBpMinViews views (64^3 x 90: 98 us with 4, 116 with 8, 160 with 16).  The
+// copies take at most kBpTargetGroups tiles' worth of memory (168 MB).
+constexpr int kBpTargetGroups = 5120;
+constexpr int kBpMinViews = 4;
+
+struct BpSplit {
+    int splits, views_per;
+    size_t bytes;  // workspace with the splits' partial volumes
+};
+
+// the split of a problem whose workspace may take `budget` bytes
+BpSplit bp_split(const ctr_geometry* g, size_t budget) {
+    const long long tiles = (long long)bp_tiles(g);
+    const size_t part = (size_t)g->nx * g->ny * g->nz * sizeof(float);
+    const size_t base = bp_base_bytes(g);
+    long long want = std::min<long long>((kBpTargetGroups + tiles - 1) / tiles, g->n_views / kBpMinViews);
+    const size_t room = budget > base + 256 ? (budget - base - 256) / part : 0;
+    if (room < (size_t)std::max<long long>(want, 1)) want = (long long)room;
+    want = std::max<long long>(want, 1);
+    BpSplit sp;
+    sp.views_per = (int)((g->n_views + want - 1) / want);
+    sp.views_per += sp.views_per & 1;  // the kernel takes views in pairs
+    sp.splits = (g->n_views + sp.views_per - 1) / sp.views_per;
+    sp.bytes = base + (sp.splits > 1 ? align_up(sp.splits * part, 256) : 0);
+    return sp;
+}
+
 size_t ctr_dd_backproject_workspace_bytes(const ctr_geometry* g, int mode) {
     if (check_geometry(g)) return 0;
     if (mode == CTR_BP_ADJOINT) return adj_layout(g).total;
-    return align_up((size_t)g->n_views * kBpViewStride * sizeof(float), 256) +
-           align_up(bp_tiles(g) * g->n_views, 256);
+    return bp_split(g, SIZE_MAX).bytes;
+}
+
+// The FDK backprojection's launches: per-view constants, the passes over every tile and view split,
+// and, with more than one split, the sum of the splits.
+static int bp_fdk(const ctr_geometry* g, const double* angles, const float* proj, float* vol, int mode, float scale,
+                  float zero_tol, int accumulate, void* workspace, const BpSplit& sp, hipStream_t s) {
+    int st = CTR_OK;
+    float* vt = (float*)workspace;
+    hipLaunchKernelGGL(bp_geometry_kernel, dim3((g->n_views + 255) / 256), dim3(256), 0, s, *g,
+                       angles, vt, mode);
+    if ((st = status_from_hip(hipGetLastError()))) return st;
+    // voxel centres: ReconCenter + (i - (n-1)/2) * d with d = (dx, -dy, -dz)
+    const float x0 = (float)(g->recon_center[0] - (g->nx - 1) / 2.0 * g->dx);
+    const float y0 = (float)(g->recon_center[1] + (g->ny - 1) / 2.0 * g->dy);
+    const float z0 = (float)(g->recon_center[2] + (g->nz - 1) / 2.0 * g->dz);
+    constexpr int ZC = kBpZC;
+    float* parts = (float*)((char*)workspace + bp_base_bytes(g));
+    const int pass_acc = sp.splits > 1 ? 0 : accumulate;
+    auto finish = [&]() -> int {
+        if (hipGetLastError() != hipSuccess) return CTR_ERR_HIP;
+        if (sp.splits == 1) return CTR_OK;
+        const size_t n = (size_t)g->nx * g->ny * g->nz;
+        if (n % 4 == 0 && (reinterpret_cast<uintptr_t>(vol) & 15) == 0)
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(bp_reduce_kernel<4>), dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0,
+                               s, parts, vol, n, sp.splits, accumulate);
+        else
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(bp_reduce_kernel<1>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
+                               parts, vol, n, sp.splits, accumulate);
+        return status_from_hip(hipGetLastError());
+    };
+    const int tiles_x = (g->nx + kTileX - 1) / kTileX;
+    const int tiles_y = (g->ny + kTileY - 1) / kTileY;
+    const int tiles_z = (g->nz + ZC - 1) / ZC;
+    const long long tiles = (long long)tiles_x * tiles_y * tiles_z;
+    if (tiles >= 2147483647LL) return CTR_ERR_INVALID;
+    const int curved = g->detector_shape == CTR_DETECTOR_CURVED ? 1 : 0;
+    const float fdx = (float)g->dx, fdy = (float)(-g->dy), fdz = (float)(-g->dz);
+    // weight zeroing, a volume of one z chunk (a slice through the source height, as in a 2D
+    // fan, is on neither side of it), or a caller's request for one pass (zero_tol < 0): the
+    // general kernel does every view
+    if (zero_tol != 0.0f || tiles_z == 1) {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(dd_backproject_tile_kernel<ZC, kBpAll>), dim3((unsigned)tiles, sp.splits),
+                           dim3(256), 0, s, proj, vol, vt, (uint8_t*)nullptr, parts, g->nx, g->ny, g->nz, g->nu,
+                           g->nv, g->n_views, sp.views_per, x0, y0, z0, fdx, fdy, fdz, curved, scale, zero_tol, pass_acc,
+                           tiles_x, tiles_y, tiles_z);
+        return finish();
+    }
+    // fast pass over the common case, then the (tile, view) pairs it left
+    uint8_t* flags = (uint8_t*)workspace + align_up((size_t)g->n_views * kBpViewStride * sizeof(float), 256);
+    const size_t flag_words = align_up((size_t)tiles * g->n_views, 256) / 4;
+    hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)std::min<size_t>((flag_words + 255) / 256, 65536)),
+                       dim3(256), 0, s, (uint32_t*)flags, flag_words);
+    if ((st = status_from_hip(hipGetLastError()))) return st;
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(dd_backproject_tile_kernel<ZC, kBpFast>), dim3((unsigned)tiles, sp.splits),
+                       dim3(256), 0, s, proj, vol, vt, flags, parts, g->nx, g->ny, g->nz, g->nu, g->nv, g->n_views,
+                       sp.views_per, x0, y0, z0, fdx, fdy, fdz, curved, scale, zero_tol, pass_acc, tiles_x, tiles_y, tiles_z);
+    if ((st = status_from_hip(hipGetLastError()))) return st;
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(dd_backproject_tile_kernel<ZC, kBpRest>), dim3((unsigned)tiles, sp.splits),
+                       dim3(256), 0, s, proj, vol, vt, flags, parts, g->nx, g->ny, g->nz, g->nu, g->nv, g->n_views,
+                       sp.views_per, x0, y0, z0, fdx, fdy, fdz, curved, scale, zero_tol, pass_acc, tiles_x, tiles_y, tiles_z);
+    return finish();
 }
 
 int ctr_dd_backproject(const ctr_geometry* g, const double* angles, const int32_t* branch,
@@ -2387,46 +2511,7 @@ int ctr_dd_backproject(const ctr_geometry* g, const double* angles, const int32_
                            g->detector_shape == CTR_DETECTOR_CURVED ? 1 : 0, scale, 1e-6f, accumulate);
         return status_from_hip(hipGetLastError());
     }
-    float* vt = (float*)workspace;
-    hipLaunchKernelGGL(bp_geometry_kernel, dim3((g->n_views + 255) / 256), dim3(256), 0, s, *g,
-                       angles, vt, mode);
-    if ((st = status_from_hip(hipGetLastError()))) return st;
-    // voxel centres: ReconCenter + (i - (n-1)/2) * d with d = (dx, -dy, -dz)
-    const float x0 = (float)(g->recon_center[0] - (g->nx - 1) / 2.0 * g->dx);
-    const float y0 = (float)(g->recon_center[1] + (g->ny - 1) / 2.0 * g->dy);
-    const float z0 = (float)(g->recon_center[2] + (g->nz - 1) / 2.0 * g->dz);
-    constexpr int ZC = kBpZC;
-    const int tiles_x = (g->nx + kTileX - 1) / kTileX;
-    const int tiles_y = (g->ny + kTileY - 1) / kTileY;
-    const int tiles_z = (g->nz + ZC - 1) / ZC;
-    const long long tiles = (long long)tiles_x * tiles_y * tiles_z;
-    if (tiles >= 2147483647LL) return CTR_ERR_INVALID;
-    const int curved = g->detector_shape == CTR_DETECTOR_CURVED ? 1 : 0;
-    const float fdx = (float)g->dx, fdy = (float)(-g->dy), fdz = (float)(-g->dz);
-    // weight zeroing, a volume of one z chunk (a slice through the source height, as in a 2D
-    // fan, is on neither side of it), or a caller's request for one pass (zero_tol < 0): the
-    // general kernel does every view
-    if (zero_tol != 0.0f || tiles_z == 1) {
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(dd_backproject_tile_kernel<ZC, kBpAll>), dim3((unsigned)tiles),
-                           dim3(256), 0, s, proj, vol, vt, (uint8_t*)nullptr, g->nx, g->ny, g->nz, g->nu,
-                           g->nv, g->n_views, x0, y0, z0, fdx, fdy, fdz, curved, scale, zero_tol, accumulate,
-                           tiles_x, tiles_y, tiles_z);
-        return status_from_hip(hipGetLastError());
-    }
-    // fast pass over the common case, then the (tile, view) pairs it left
-    uint8_t* flags = (uint8_t*)workspace + align_up((size_t)g->n_views * kBpViewStride * sizeof(float), 256);
-    const size_t flag_words = align_up((size_t)tiles * g->n_views, 256) / 4;
-    hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)std::min<size_t>((flag_words + 255) / 256, 65536)),
-                       dim3(256), 0, s, (uint32_t*)flags, flag_words);
-    if ((st = status_from_hip(hipGetLastError()))) return st;
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(dd_backproject_tile_kernel<ZC, kBpFast>), dim3((unsigned)tiles),
-                       dim3(256), 0, s, proj, vol, vt, flags, g->nx, g->ny, g->nz, g->nu, g->nv, g->n_views,
-                       x0, y0, z0, fdx, fdy, fdz, curved, scale, zero_tol, accumulate, tiles_x, tiles_y, tiles_z);
-    if ((st = status_from_hip(hipGetLastError()))) return st;
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(dd_backproject_tile_kernel<ZC, kBpRest>), dim3((unsigned)tiles),
-                       dim3(256), 0, s, proj, vol, vt, flags, g->nx, g->ny, g->nz, g->nu, g->nv, g->n_views,
-                       x0, y0, z0, fdx, fdy, fdz, curved, scale, zero_tol, accumulate, tiles_x, tiles_y, tiles_z);
-    return status_from_hip(hipGetLastError());
+    return bp_fdk(g, angles, proj, vol, mode, scale, zero_tol, accumulate, workspace, bp_split(g, SIZE_MAX), s);
 }
 
 int ctr_dd_backproject_static(const ctr_geometry* g, const double* angles, const float* proj,
@@ -2435,14 +2520,15 @@ int ctr_dd_backproject_static(const ctr_geometry* g, const double* angles, const
     int st = check_geometry(g);
     if (st) return st;
     if (mode != CTR_BP_FDK_REF && mode != CTR_BP_FDK_EDGE) return CTR_ERR_UNSUPPORTED;
-    const size_t need = ctr_dd_backproject_workspace_bytes(g, mode);
-    if (need > kStaticScratchBytes) return CTR_ERR_SCRATCH;
+    // as many view splits as the array holds beside the table and the flags (none if need be)
+    if (bp_base_bytes(g) > kStaticScratchBytes) return CTR_ERR_SCRATCH;
+    if (!angles || !proj || !vol) return CTR_ERR_INVALID;
     void* ws = nullptr;
     if ((st = static_scratch(&ws))) return st;
     // the same launches as ctr_dd_backproject: the per-view table is written by a kernel and
     // the flags are cleared by a fill kernel on `stream` before use
-    return ctr_dd_backproject(g, angles, nullptr, proj, vol, mode, scale, zero_tol, accumulate, ws,
-                              need, stream);
+    return bp_fdk(g, angles, proj, vol, mode, scale, zero_tol, accumulate, ws, bp_split(g, kStaticScratchBytes),
+                  (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -140,11 +140,13 @@ int ctr_dd_backproject(const ctr_geometry* g, const double* angles, const int32_
 /* No counterpart in the reference: ctr_dd_backproject (modes CTR_BP_FDK_REF and
  * CTR_BP_FDK_EDGE) without a workspace argument, for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
- * Its scratch (the per-view table and the per-(tile, view) flags) lives in a static 32 MiB
- * device array, one per GPU, held until the process ends; problems needing more
- * (ctr_dd_backproject_workspace_bytes(g, mode) > 32 MiB, e.g. above about 1000 views at 512^3)
+ * Its scratch (the per-view table, the per-(tile, view) flags and, as far as they fit, the
+ * partial volumes of a small problem's view splits) lives in a static 32 MiB device array, one per
+ * GPU, held until the process ends; problems whose table and flags need more (64 bytes per view
+ * plus one byte per 16 x 16 x 32 voxel tile and view, e.g. above about 2000 views at 512^3)
  * return CTR_ERR_SCRATCH, and CTR_BP_ADJOINT returns CTR_ERR_UNSUPPORTED.  It allocates
- * nothing and launches the same kernels as ctr_dd_backproject.  Every call on one GPU shares
+ * nothing and launches the same kernels as ctr_dd_backproject (with fewer view splits where the
+ * partial volumes do not all fit: the same sums in another order).  Every call on one GPU shares
  * that GPU's array: calls that overlap in time on one GPU (other streams, other threads) race
  * and must be serialised by the caller.  The current device must be the one `stream` and the
  * buffers belong to. */
