@@ -907,26 +907,29 @@ __global__ void bp_geometry_kernel(ctr_geometry g, const double* __restrict__ an
 // are assigned so that each XCD holds contiguous z-chunks, whose windows share detector rows in
 // that XCD's L2.  A window larger than the LDS buffer is gathered from global memory.
 constexpr int kTileX = 16, kTileY = 16;
-#ifndef CTR_BP_WIN_CAP
-#define CTR_BP_WIN_CAP 1024
-#endif
-constexpr int kWinCap = CTR_BP_WIN_CAP;  // floats per LDS window buffer
-#ifndef CTR_BP_WIN_RING
-#define CTR_BP_WIN_RING 64
-#endif
-constexpr int kWinRing = CTR_BP_WIN_RING;  // views in the LDS ring of detector windows (power of 2)
-constexpr int kMaxUTaps = 3;           // u taps held in registers (more are looped)
-constexpr int kPrefetch = (kWinCap + 255) / 256;  // window cells per thread
-#ifndef CTR_BP_ZC
-#define CTR_BP_ZC 32
-#endif
-#ifndef CTR_BP_MAX_ROWS
-#define CTR_BP_MAX_ROWS 19
-#endif
-constexpr int kBpZC = CTR_BP_ZC;            // voxels along z per work-item (and tile)
-constexpr int kBpSub = 16;                  // voxels per sub-chunk: the unit of one row integral
-static_assert(kBpZC % kBpSub == 0, "a work-item's voxels split into whole sub-chunks");
-constexpr int kMaxRows = CTR_BP_MAX_ROWS;   // rows per sub-chunk on the row-integral path
+constexpr int kWinRing = 64;                // views in the LDS ring of detector windows (power of 2)
+constexpr int kMaxRows = 19;                // rows per sub-chunk on the row-integral path
+
+// Shape of a work-item's share: ZC voxels along z in sub-chunks of SUB (the unit of one row
+// integral), CAP floats per LDS detector window, TAPS u taps held in registers.  A sub-chunk's rows
+// must fit the row-integral table (kMaxRows) and a tile's detector window its LDS buffer, so SUB
+// and ZC shrink and CAP grows as the detector gets finer against the voxels; bp_choose has the rule.
+// LDS leaves room for five groups per CU with the first shape, four with the next three, two with
+// the last, and the registers for as many.  Measured, with one shape (the first) before: 256^3 x 360
+// views of 1024 x 768 cells, 1.9 cells per voxel, 80.6 -> 9.7 ms (Fine); 320 x 320 x 200 x 480 views,
+// 1.2 cells, 81.4 -> 11.2 ms (Medium; Fine 12.6); 192 x 192 x 100 x 300, 1.05 cells, 3.15 -> 1.42 ms
+// (Medium; Fine 1.50); 128^3 x 180, 1.0 cells, 0.51 -> 0.42 ms (Whole; Medium 0.52).  2048-cell windows
+// for Whole: 136 registers, three groups per CU, 18 % slower on a 151 x 163 x 107 helix.
+template <int ZC_, int SUB_, int CAP_, int TAPS_>
+struct BpShape {
+    static constexpr int ZC = ZC_, SUB = SUB_, CAP = CAP_, TAPS = TAPS_;
+    static_assert(ZC % SUB == 0, "a work-item's voxels split into whole sub-chunks");
+};
+using BpCoarse = BpShape<32, 16, 1024, 3>;  // up to about one detector cell per voxel, plain volumes
+using BpWhole = BpShape<32, 16, 1280, 3>;   // the same with larger windows
+using BpMedium = BpShape<24, 12, 2048, 4>;  // up to about 1.4
+using BpFine = BpShape<16, 8, 2048, 5>;     // up to about two
+using BpFinest = BpShape<8, 4, 4096, 8>;    // up to about four
 
 struct BpView {
     float c, s, Sx, Sy, Sz, Au, Bu, Av, Bv, R;
@@ -984,17 +987,17 @@ __device__ inline void tile_window(const BpView& v, float xa, float xb, float ya
 }
 
 // 0: window empty (skip the view), 1: staged in LDS, 2: too large, gather from global memory
+template <int CAP>
 __device__ inline int window_mode(int wvn, int wun) {
     if (wvn <= 0 || wun <= 0) return 0;
-    return (wvn * wun <= kWinCap) ? 1 : 2;
+    return (wvn * wun <= CAP) ? 1 : 2;
 }
 
 // Work split of the backprojection (kind): the fast pass (kBpFast) handles the common case
-// only -- LDS window, z chunk on one side of the source (affine footprints), at most kMaxRows
-// rows and kMaxUTaps columns, slowly varying footprint heights, no weight zeroing -- and
-// reports every (work-item, view) it
-// leaves; the completing pass (kBpRest) does exactly those; kBpAll does everything.  Keeping
-// the rare cases out of the fast pass keeps its register count, and so its occupancy, low.
+// only -- LDS window, at most kMaxRows rows and TAPS columns, no weight zeroing -- and reports
+// every (work-item, view) it leaves; the completing pass (kBpRest) does exactly those; kBpAll
+// does everything.  Keeping the rare cases out of the fast pass keeps its register count, and so
+// its occupancy, low.
 constexpr int kBpFast = 0, kBpAll = 1, kBpRest = 2;
 
 // Footprint of a voxel column for one view: the four corners (+-hx, +-hy) rotated into the
@@ -1059,6 +1062,30 @@ __device__ inline BpChunk bp_chunk(const BpView& v, const BpColumn& col, float Z
     return ch;
 }
 
+// The same ends for a chunk on either side of the source height: smn = (e - hz) r1 is the smaller of
+// its values at r = rmin and rmax, smx = (e + hz) r2 the larger, so the low end is the smaller and
+// the high end the larger of two affine forms, which also holds for a chunk on one side.
+struct BpPiece {
+    float Alo[2], Dlo[2], Ahi[2], Dhi[2];
+    __device__ inline float lo(float fi) const { return fminf(fmaf(fi, Dlo[0], Alo[0]), fmaf(fi, Dlo[1], Alo[1])); }
+    __device__ inline float hi(float fi) const { return fmaxf(fmaf(fi, Dhi[0], Ahi[0]), fmaf(fi, Dhi[1], Ahi[1])); }
+};
+
+__device__ inline BpPiece bp_piece(const BpView& v, float rmin, float rmax, float Z0, float dz, float hz) {
+    BpPiece p;
+    const float e0 = v.Sz - Z0;
+    const bool g1_high = v.Bv > 0.0f;
+    const float el = g1_high ? e0 + hz : e0 - hz, eh = g1_high ? e0 - hz : e0 + hz;
+    const float B[2] = {v.Bv * rmin, v.Bv * rmax};
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        p.Alo[k] = fmaf(-B[k], el, v.Av);
+        p.Ahi[k] = fmaf(-B[k], eh, v.Av);
+        p.Dlo[k] = p.Dhi[k] = B[k] * dz;
+    }
+    return p;
+}
+
 // Row-integral table of a work-item (its LDS column `scan`, stride 256 floats): entry m holds
 // C at row boundary ks - 1 + m, so entries 0 and 1 are 0 (boundaries ks - 1 and ks), entry j + 2
 // the integral of rows ks .. ks + j, and entry nr + 2 repeats the total.  A lookup at
@@ -1070,14 +1097,15 @@ __device__ inline float bp_lookup(const float* __restrict__ scan, float x) {
     return fmaf(__builtin_amdgcn_fractf(x), b - a, a);
 }
 
-// The row integral of nr window rows from `rp` (stride `stride`), u-filtered with three taps
+// The row integral of nr window rows from `rp` (stride `stride`), u-filtered with NT taps
 // (weight 0 past the footprint; the window buffers are zero-initialised and padded, so such
 // reads stay finite) and times W, into the table above.  The tap weights `wa` come with W
-// folded in (wa[t] = wu[t] * W), so a row is three FMAs into the running sum, taps in the order
-// 2, 1, 0 (every pass accumulates a row this way).  Two rows per step.
-__device__ inline void bp_row_integral3(const float* __restrict__ rp, int stride, int nr, const float (&wa)[kMaxUTaps],
-                                        float* __restrict__ scan) {
-    const float a0 = wa[0], a1 = wa[1], a2 = wa[2];
+// folded in (wa[t] = wu[t] * W), so a row is NT FMAs into the running sum, taps from the last to
+// the first (every pass accumulates a row this way).  Two rows per step.
+template <int NT, int TAPS>
+__device__ inline void bp_row_integral(const float* __restrict__ rp, int stride, int nr, const float (&wa)[TAPS],
+                                       float* __restrict__ scan) {
+    static_assert(NT <= TAPS, "taps held");
     float csum = 0.0f;
     scan[0] = 0.0f;
     scan[256] = 0.0f;
@@ -1086,27 +1114,47 @@ __device__ inline void bp_row_integral3(const float* __restrict__ rp, int stride
     const float* const pair_end = rp + __mul24(nr & ~1, stride);
     while (rp != pair_end) {
         const float* rq = rp + stride;
-        const float p0 = rp[0], p1 = rp[1], p2 = rp[2];
-        const float q0 = rq[0], q1 = rq[1], q2 = rq[2];
-        csum = fmaf(a0, p0, fmaf(a1, p1, fmaf(a2, p2, csum)));
+        float p[NT], q[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) p[t] = rp[t];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) q[t] = rq[t];
+#pragma unroll
+        for (int t = NT - 1; t >= 0; --t) csum = fmaf(wa[t], p[t], csum);
         sp[256] = csum;
-        csum = fmaf(a0, q0, fmaf(a1, q1, fmaf(a2, q2, csum)));
+#pragma unroll
+        for (int t = NT - 1; t >= 0; --t) csum = fmaf(wa[t], q[t], csum);
         sp[512] = csum;
         sp += 512;
         rp += 2 * stride;
     }
     if (nr & 1) {
-        csum = fmaf(a0, rp[0], fmaf(a1, rp[1], fmaf(a2, rp[2], csum)));
+#pragma unroll
+        for (int t = NT - 1; t >= 0; --t) csum = fmaf(wa[t], rp[t], csum);
         sp[256] = csum;
     }
     scan[(nr + 2) * 256] = csum;
 }
 
-// The voxels of a sub-chunk (acc[OFF .. OFF+kBpSub-1]) with affine footprints from the row
+// The same with as many taps (at least 3) as the wavefront's widest footprint needs.
+template <int TAPS, int NT = 3>
+__device__ inline void bp_rows(const float* __restrict__ rp, int stride, int nr, int ntaps, const float (&wa)[TAPS],
+                               float* __restrict__ scan) {
+    if constexpr (NT == TAPS) {
+        bp_row_integral<TAPS>(rp, stride, nr, wa, scan);
+    } else {
+        if (!__any(ntaps > NT))
+            bp_row_integral<NT>(rp, stride, nr, wa, scan);
+        else
+            bp_rows<TAPS, (NT + 2 < TAPS && TAPS > 5) ? NT + 2 : NT + 1 >= TAPS ? TAPS : NT + 1>(rp, stride, nr, ntaps, wa, scan);
+    }
+}
+
+// The voxels of a sub-chunk (acc[OFF .. OFF+SUB-1]) with affine footprints from the row
 // integral: C between row boundaries is linear.  With CLAMP, v - (ks - 1) is clamped to
 // [1, nr + 1], which gives C = 0 below and the total above (rows outside the detector or the
-// window contribute nothing).  Without it the footprints of all kBpSub voxels must lie inside
-// the table's rows (bp_sub_rows' `inside`: the sub-chunk is whole and its rows were not cut by
+// window contribute nothing).  Without it the footprints of all SUB voxels must lie inside
+// the table's rows (bp_sub_rows' `inside`: its rows were not cut by
 // the detector or the window); the clamp then never binds, so both ways give the same sums.
 // Without EXACT, 1/(hi - lo) of voxel i comes from a quadratic in t = i - 7.5 (the sub-chunk's
 // middle): the footprint height is affine in i, h_i = h_m (1 + t e) with e the fraction it
@@ -1125,21 +1173,21 @@ __device__ inline bool bp_series_ok(const BpColumn& col) {
     return 2.0f * (col.rmax - col.rmin) <= kSeriesRel * (col.rmax + col.rmin);
 }
 
-template <int OFF, bool CLAMP, bool EXACT, int ZC>
+template <int OFF, int SUB, bool CLAMP, bool EXACT, int ZC>
 __device__ inline void bp_voxels_affine(const BpChunk& ch, int ks, int nr, const float* __restrict__ scan,
                                         float (&acc)[ZC]) {
-    static_assert(OFF + kBpSub <= ZC, "sub-chunk inside the work-item");
+    static_assert(OFF + SUB <= ZC, "sub-chunk inside the work-item");
     const float base = (float)(ks - 1), top = (float)(nr + 1);
     const float alo = ch.Alo - base, ahi = ch.Ahi - base;
     // 1/h_i = rm + t c1 + t^2 c2 with t = i - 7.5, rm = 1/h(7.5), e = (Dhi - Dlo) rm,
     // c1 = -rm e, c2 = rm e^2
-    constexpr float kMid = 0.5f * (float)(kBpSub - 1);
+    constexpr float kMid = 0.5f * (float)(SUB - 1);
     const float dD = ch.Dhi - ch.Dlo;
     const float rm = EXACT ? 0.0f : __builtin_amdgcn_rcpf(fmaf(kMid, dD, ahi - alo));
     const float e = dD * rm;
     const float c1 = -(rm * e), c2 = -(c1 * e);
 #pragma unroll
-    for (int i = 0; i < kBpSub; ++i) {
+    for (int i = 0; i < SUB; ++i) {
         const float lo = fmaf((float)i, ch.Dlo, alo), hi = fmaf((float)i, ch.Dhi, ahi);
         const float t = (float)i - kMid;
         float rinv;
@@ -1153,59 +1201,89 @@ __device__ inline void bp_voxels_affine(const BpChunk& ch, int ks, int nr, const
     }
 }
 
-// z of the first voxel of sub-chunk h of a work-item whose first voxel is at Z0: every pass
-// derives its sub-chunks from this, so they round them alike
-__device__ inline float bp_sub_z0(float Z0, float dz, int h) { return fmaf((float)(kBpSub * h), dz, Z0); }
-
-// Rows [ks, ks + nr - 1] (clamped to the detector and to the rows [row0, row0 + nrows) of the
-// source) that the n voxels of an affine sub-chunk touch: the ends move monotonically with i,
-// so the range comes from the end voxels.  `inside`: the sub-chunk is whole and nothing was cut.
-__device__ inline void bp_sub_rows(const BpChunk& ch, int n, int row0, int nrows, int nv, int& ks, int& nr,
-                                   bool& inside) {
-    const float fL = (float)(n - 1);
-    const float lo0 = fmaf(0.0f, ch.Dlo, ch.Alo), hi0 = fmaf(0.0f, ch.Dhi, ch.Ahi);
-    const float loL = fmaf(fL, ch.Dlo, ch.Alo), hiL = fmaf(fL, ch.Dhi, ch.Ahi);
-    const int klo = (int)floorf(fminf(lo0, loL)), khi = (int)floorf(fmaxf(hi0, hiL));
-    ks = max(max(klo, 0), row0);
-    const int ke = min(min(khi, nv - 1), row0 + nrows - 1);
-    nr = ke - ks + 1;
-    inside = n == kBpSub && ks == klo && ke == khi;
-}
-
-// Calls f(integral_constant<int, h>) for every sub-chunk h of a ZC-voxel work-item.
-template <int ZC, int H = 0, typename F>
-__device__ inline void bp_for_subs(F&& f) {
-    if constexpr (H * kBpSub < ZC) {
-        f(std::integral_constant<int, H>{});
-        bp_for_subs<ZC, H + 1>(f);
+// The same for any sub-chunk: ends of either side of the source height, clamped to the table's
+// rows, a reciprocal per voxel (about six more instructions per voxel than the affine form).
+template <int OFF, int SUB, int ZC>
+__device__ inline void bp_voxels_general(const BpPiece& pc, int ks, int nr, const float* __restrict__ scan,
+                                         float (&acc)[ZC]) {
+    const float base = (float)(ks - 1), top = (float)(nr + 1);
+#pragma unroll
+    for (int i = 0; i < SUB; ++i) {
+        const float lo = pc.lo((float)i) - base, hi = pc.hi((float)i) - base;
+        const float xl = __builtin_amdgcn_fmed3f(lo, 1.0f, top), xh = __builtin_amdgcn_fmed3f(hi, 1.0f, top);
+        acc[OFF + i] = fmaf(bp_lookup(scan, xh) - bp_lookup(scan, xl), __builtin_amdgcn_rcpf(hi - lo), acc[OFF + i]);
     }
 }
 
-// The fast pass (kBpFast): the common case only -- window in LDS, sub-chunk on one side of the
-// source height, at most kMaxRows rows and kMaxUTaps columns, a footprint height that changes
-// slowly enough along z for the series normaliser (bp_series_ok), no weight zeroing (the
-// host runs this pass only with zero_tol = 0).  The column's u-footprint, u-weights and FDK weight are
-// worked out once per view for all ZC voxels; every sub-chunk then builds its own row integral.
+// z of the first voxel of sub-chunk h of a work-item whose first voxel is at Z0: every pass
+// derives its sub-chunks from this, so they round them alike
+template <int SUB>
+__device__ inline float bp_sub_z0(float Z0, float dz, int h) { return fmaf((float)(SUB * h), dz, Z0); }
+
+// Rows [ks, ks + nr - 1] (clamped to the detector and to the rows [row0, row0 + nrows) of the
+// source) that the first n voxels of a sub-chunk touch: the ends move monotonically with i,
+// so the range comes from the end voxels.  `inside`: nothing was cut.
+__device__ inline void bp_sub_rows(const BpView& v, const BpColumn& col, const BpChunk& ch, float Z0, float dz,
+                                   float hz, int n, int row0, int nrows, int nv, int& ks, int& nr, bool& inside) {
+    const float fL = (float)(n - 1);
+    float rlo, rhi;
+    if (ch.lin) {
+        rlo = fminf(fmaf(0.0f, ch.Dlo, ch.Alo), fmaf(fL, ch.Dlo, ch.Alo));
+        rhi = fmaxf(fmaf(0.0f, ch.Dhi, ch.Ahi), fmaf(fL, ch.Dhi, ch.Ahi));
+    } else {
+        const BpPiece pc = bp_piece(v, col.rmin, col.rmax, Z0, dz, hz);
+        rlo = fminf(pc.lo(0.0f), pc.lo(fL));
+        rhi = fmaxf(pc.hi(0.0f), pc.hi(fL));
+    }
+    const int klo = (int)floorf(rlo), khi = (int)floorf(rhi);
+    ks = max(max(klo, 0), row0);
+    const int ke = min(min(khi, nv - 1), row0 + nrows - 1);
+    nr = ke - ks + 1;
+    inside = ks == klo && ke == khi;
+}
+
+// Calls f(integral_constant<int, h>) for every sub-chunk h of a ZC-voxel work-item.
+template <int ZC, int SUB, int H = 0, typename F>
+__device__ inline void bp_for_subs(F&& f) {
+    if constexpr (H * SUB < ZC) {
+        f(std::integral_constant<int, H>{});
+        bp_for_subs<ZC, SUB, H + 1>(f);
+    }
+}
+
+// The fast pass (kBpFast): the common case only -- window in LDS, at most kMaxRows rows and TAPS
+// columns, no weight zeroing (the host runs this pass only with zero_tol = 0).  The column's
+// u-footprint, u-weights and FDK weight are worked out once per view for all ZC voxels; every
+// sub-chunk then builds its own row integral.  A last sub-chunk with fewer voxels than SUB is treated
+// as whole: the voxels past the volume's end are summed and not stored.
+// Without GENERAL the pass takes only plain sub-chunks: seen whole (not cut by the detector or the
+// window), on one side of the source height and with a footprint height that changes slowly enough
+// for the series normaliser.  With it, such sub-chunks of a wavefront take the short voxel loop (with a
+// reciprocal per voxel) and the others the general one.  The general loop costs the coarse shape
+// 29 registers, and with them the fifth wavefront per SIMD, so it is left out where the host sees
+// that (nearly) every sub-chunk is plain (bp_choose).
 // Returns true when it leaves a sub-chunk of this (work-item, view) to the completing pass,
-// which decides from the same bp_column / bp_chunk values.
-template <int ZC>
+// which decides from the same bp_column / bp_sub_rows values.
+template <typename S, bool GENERAL>
 __device__ inline bool bp_column_view_fast(const BpView& v, const float* __restrict__ win, int stride,
                                            int row0, int nrows, int col0, int ncols, float X, float Y,
                                            float Z0, float dz, float hx, float hy, float hz, int nz_left,
                                            int curved, float scale, int nu, int nv, float* __restrict__ scan,
-                                           float (&acc)[ZC]) {
+                                           float (&acc)[S::ZC]) {
+    constexpr int SUB = S::SUB, TAPS = S::TAPS;
     const BpColumn col = bp_column(v, X, Y, hx, hy, curved);
     // taps inside the detector and the window
     const int kus = max(max(col.ku0, 0), col0), kue = min(min(col.ku1, nu - 1), col0 + ncols - 1);
     if (kus > kue) return false;
-    const bool taps_ok = kue - kus + 1 <= kMaxUTaps;
+    const int ntaps = kue - kus + 1;
+    const bool taps_ok = ntaps <= TAPS;
     // overlap of each tap with [ulo, uhi] over the footprint width (python/GPUFuncs_pycuda.py:
     // 427-438 without zeroing); a footprint inside one cell weighs 1
     const float inv_u = __builtin_amdgcn_rcpf(col.uhi - col.ulo);
     const float fk = (float)kus;
-    float wu[kMaxUTaps];
+    float wu[TAPS];
 #pragma unroll
-    for (int j = 0; j < kMaxUTaps; ++j) {
+    for (int j = 0; j < TAPS; ++j) {
         const float k = fk + (float)j;
         const float w = (fminf(col.uhi, k + 1.0f) - fmaxf(col.ulo, k)) * inv_u;
         wu[j] = (kus + j <= kue) ? fmaxf(w, 0.0f) : 0.0f;
@@ -1214,44 +1292,50 @@ __device__ inline bool bp_column_view_fast(const BpView& v, const float* __restr
     const bool series_ok = bp_series_ok(col);
     const float dd = v.R - col.yr0;
     const float W = scale * (v.R * v.R) * __builtin_amdgcn_rcpf(dd * dd);
-    float wa[kMaxUTaps];
+    float wa[TAPS];
 #pragma unroll
-    for (int j = 0; j < kMaxUTaps; ++j) wa[j] = wu[j] * W;
+    for (int j = 0; j < TAPS; ++j) wa[j] = wu[j] * W;
     const float* wp = win + (kus - col0);
     bool left = false;
-    bp_for_subs<ZC>([&](auto hc) {
+    bp_for_subs<S::ZC, SUB>([&](auto hc) {
         constexpr int h = decltype(hc)::value;
-        const int n = min(kBpSub, nz_left - kBpSub * h);
-        if (n <= 0) return;
-        const BpChunk ch = bp_chunk<kBpSub>(v, col, bp_sub_z0(Z0, dz, h), dz, hz);
-        if (!ch.lin) {
-            left = true;
-            return;
-        }
+        if (nz_left <= SUB * h) return;
+        const float Z0h = bp_sub_z0<SUB>(Z0, dz, h);
+        const BpChunk ch = bp_chunk<SUB>(v, col, Z0h, dz, hz);
         int ks, nr;
         bool inside;
-        bp_sub_rows(ch, n, row0, nrows, nv, ks, nr, inside);
+        bp_sub_rows(v, col, ch, Z0h, dz, hz, SUB, row0, nrows, nv, ks, nr, inside);
         if (nr <= 0) return;
-        if (nr > kMaxRows || !taps_ok || !inside || !series_ok) {
+        const bool plain = ch.lin && inside && (GENERAL || series_ok);
+        if (nr > kMaxRows || !taps_ok || (!GENERAL && !plain)) {
             left = true;
             return;
         }
         // window offsets fit 24 bits: a full-rate multiply (the 32-bit one is quarter rate)
-        bp_row_integral3(wp + __mul24(ks - row0, stride), stride, nr, wa, scan);
-        bp_voxels_affine<kBpSub * h, false, false>(ch, ks, nr, scan, acc);
+        bp_rows<TAPS>(wp + __mul24(ks - row0, stride), stride, nr, ntaps, wa, scan);
+        if (!GENERAL || !__any(!plain)) {
+            bp_voxels_affine<SUB * h, SUB, false, GENERAL>(ch, ks, nr, scan, acc);
+        } else if constexpr (GENERAL) {
+            // opaque copies: keeps this loop's footprints from being computed before the branch,
+            // where they would cost the common loop its registers
+            float rmin = col.rmin, rmax = col.rmax;
+            asm volatile("" : "+v"(rmin), "+v"(rmax));
+            bp_voxels_general<SUB * h, SUB>(bp_piece(v, rmin, rmax, Z0h, dz, hz), ks, nr, scan, acc);
+        }
     });
     return left;
 }
 
 // The completing pass (kBpRest: every (work-item, view, sub-chunk) the fast pass left, and
 // nothing else) and the single pass over all cases (kBpAll).
-template <int ZC, bool FROM_LDS, int KIND>
+template <typename S, bool FROM_LDS, int KIND, bool GENERAL>
 __device__ inline void bp_column_view(const BpView& v, const float* __restrict__ src, int stride,
                                       int row0, int nrows, int col0, int ncols, float X, float Y,
                                       float Z0, float dz, float hx, float hy, float hz, int nz_left,
                                       int curved, float scale, float zero_tol, int nu, int nv,
-                                      bool window_in_lds, float* __restrict__ scan, float (&acc)[ZC]) {
+                                      bool window_in_lds, float* __restrict__ scan, float (&acc)[S::ZC]) {
     static_assert(KIND == kBpAll || KIND == kBpRest, "the fast pass has its own function");
+    constexpr int SUB = S::SUB, TAPS = S::TAPS;
     const BpColumn col = bp_column(v, X, Y, hx, hy, curved);
     const float ulo = col.ulo, uhi = col.uhi;
     const int ku0 = col.ku0, ku1 = col.ku1;
@@ -1259,98 +1343,61 @@ __device__ inline void bp_column_view(const BpView& v, const float* __restrict__
     const int kus = max(max(ku0, 0), col0), kue = min(min(ku1, nu - 1), col0 + ncols - 1);
     if (kus > kue) return;
     const float inv_u = __builtin_amdgcn_rcpf(uhi - ulo);
-    float wu[kMaxUTaps];
+    float wu[TAPS];
 #pragma unroll
-    for (int j = 0; j < kMaxUTaps; ++j) {
+    for (int j = 0; j < TAPS; ++j) {
         const int ku = kus + j;
         wu[j] = (ku <= kue) ? dd_weight(ku, ku0, ku1, ulo, uhi, inv_u, zero_tol) : 0.0f;
     }
     const float dd = v.R - col.yr0;
     const float W = scale * (v.R * v.R) * __builtin_amdgcn_rcpf(dd * dd);
-    float wa[kMaxUTaps];
+    float wa[TAPS];
 #pragma unroll
-    for (int j = 0; j < kMaxUTaps; ++j) wa[j] = wu[j] * W;
-    const float rmin = col.rmin, rmax = col.rmax;
+    for (int j = 0; j < TAPS; ++j) wa[j] = wu[j] * W;
     const int cbase = kus - col0;
     const int ntaps = kue - kus + 1;
-    bp_for_subs<ZC>([&](auto hc) {
+    bp_for_subs<S::ZC, SUB>([&](auto hc) {
         constexpr int h = decltype(hc)::value;
-        constexpr int OFF = kBpSub * h;
-        const int n = min(kBpSub, nz_left - kBpSub * h);
+        constexpr int OFF = SUB * h;
+        const int n = min(SUB, nz_left - SUB * h);
         if (n <= 0) return;
-        const float Z0h = bp_sub_z0(Z0, dz, h);
-        const BpChunk ch = bp_chunk<kBpSub>(v, col, Z0h, dz, hz);
-        const bool lin = ch.lin;
-        auto foot = [&](float fi, float& lo, float& hi) {
-            if (lin) {
-                lo = fmaf(fi, ch.Dlo, ch.Alo);
-                hi = fmaf(fi, ch.Dhi, ch.Ahi);
-            } else {
-                const float e = v.Sz - fmaf(fi, dz, Z0h);
-                const float ep = e + hz, em = e - hz;
-                const float smx = ep * (ep >= 0.0f ? rmax : rmin);
-                const float smn = em * (em >= 0.0f ? rmin : rmax);
-                const float g1 = fmaf(-v.Bv, smn, v.Av), g2 = fmaf(-v.Bv, smx, v.Av);
-                lo = fminf(g1, g2);
-                hi = fmaxf(g1, g2);
-            }
-        };
+        const float Z0h = bp_sub_z0<SUB>(Z0, dz, h);
+        const BpChunk ch = bp_chunk<SUB>(v, col, Z0h, dz, hz);
         int ks, nr;
-        bool inside = false;
-        if (lin) {
-            bp_sub_rows(ch, n, row0, nrows, nv, ks, nr, inside);
-        } else {
-            // the ends move monotonically with i, so the range comes from the end voxels
-            float lo0, hi0, loL, hiL;
-            foot(0.0f, lo0, hi0);
-            foot((float)(n - 1), loL, hiL);
-            const float rlo = fminf(lo0, loL), rhi = fmaxf(hi0, hiL);
-            ks = max(max((int)floorf(rlo), 0), row0);
-            const int ke = min(min((int)floorf(rhi), nv - 1), row0 + nrows - 1);
-            nr = ke - ks + 1;
-        }
-        if (nr <= 0) return;
+        bool inside;
         if constexpr (KIND == kBpRest) {
             // the sub-chunks the fast pass did
-            const bool common = window_in_lds && lin && inside && nr <= kMaxRows && ntaps <= kMaxUTaps &&
-                                zero_tol <= 0.0f && bp_series_ok(col);
-            if (common) return;
+            bp_sub_rows(v, col, ch, Z0h, dz, hz, SUB, row0, nrows, nv, ks, nr, inside);
+            const bool plain = ch.lin && inside && bp_series_ok(col);
+            if (window_in_lds && nr <= kMaxRows && ntaps <= TAPS && (GENERAL || plain)) return;
         }
+        bp_sub_rows(v, col, ch, Z0h, dz, hz, n, row0, nrows, nv, ks, nr, inside);
+        if (nr <= 0) return;
+        const BpPiece pc = bp_piece(v, col.rmin, col.rmax, Z0h, dz, hz);
         if (zero_tol <= 0.0f && nr <= kMaxRows) {
             const float* rp = src + (FROM_LDS ? __mul24(ks - row0, stride) : (size_t)(ks - row0) * stride) + cbase;
-            if (FROM_LDS && !__any(ntaps > kMaxUTaps)) {
-                bp_row_integral3(rp, stride, nr, wa, scan);
+            if (FROM_LDS && !__any(ntaps > TAPS)) {
+                bp_rows<TAPS>(rp, stride, nr, ntaps, wa, scan);
             } else {
-                // taps from the last to the first, each weight times W, as bp_row_integral3 does
-                // (the same sums for at most three taps)
+                // taps from the last to the first, each weight times W, as bp_row_integral does
+                // (the same sums for at most TAPS taps)
                 float csum = 0.0f;
                 scan[0] = 0.0f;
                 scan[256] = 0.0f;
                 for (int j = 0; j < nr; ++j) {
-                    for (int t = ntaps - 1; t >= kMaxUTaps; --t)
+                    for (int t = ntaps - 1; t >= TAPS; --t)
                         csum = fmaf(dd_weight(kus + t, ku0, ku1, ulo, uhi, inv_u, zero_tol) * W, rp[t], csum);
 #pragma unroll
-                    for (int t = kMaxUTaps - 1; t >= 0; --t) csum = fmaf(wa[t], rp[min(t, ntaps - 1)], csum);
+                    for (int t = TAPS - 1; t >= 0; --t) csum = fmaf(wa[t], rp[min(t, ntaps - 1)], csum);
                     scan[(j + 2) * 256] = csum;
                     rp += stride;
                 }
                 scan[(nr + 2) * 256] = csum;
             }
-            if (lin) {
-                bp_voxels_affine<OFF, true, true>(ch, ks, nr, scan, acc);
-            } else {
-                const float base = (float)(ks - 1), top = (float)(nr + 1);
-#pragma unroll
-                for (int i = 0; i < kBpSub; ++i) {
-                    float lo, hi;
-                    foot((float)i, lo, hi);
-                    lo -= base;
-                    hi -= base;
-                    const float xl = __builtin_amdgcn_fmed3f(lo, 1.0f, top), xh = __builtin_amdgcn_fmed3f(hi, 1.0f, top);
-                    acc[OFF + i] = fmaf(bp_lookup(scan, xh) - bp_lookup(scan, xl), __builtin_amdgcn_rcpf(hi - lo),
-                                        acc[OFF + i]);
-                }
-            }
+            if (ch.lin)
+                bp_voxels_affine<OFF, SUB, true, true>(ch, ks, nr, scan, acc);
+            else
+                bp_voxels_general<OFF, SUB>(pc, ks, nr, scan, acc);
             return;
         }
         // explicit per-row weights (zeroing of small weights, or a sub-chunk over more than
@@ -1361,15 +1408,14 @@ __device__ inline void bp_column_view(const BpView& v, const float* __restrict__
             const float* row = src + (size_t)(k - row0) * stride + cbase;
             float rk = 0.0f;
 #pragma unroll
-            for (int j = 0; j < kMaxUTaps; ++j) rk = fmaf(wu[j], row[min(j, ntaps - 1)], rk);
-            for (int j = kMaxUTaps; j < ntaps; ++j)
+            for (int j = 0; j < TAPS; ++j) rk = fmaf(wu[j], row[min(j, ntaps - 1)], rk);
+            for (int j = TAPS; j < ntaps; ++j)
                 rk = fmaf(dd_weight(kus + j, ku0, ku1, ulo, uhi, inv_u, zero_tol), row[j], rk);
             rk *= W;
             const float fk = (float)k, fk1 = (float)(k + 1);
 #pragma unroll
-            for (int i = 0; i < kBpSub; ++i) {
-                float vlo, vhi;
-                foot((float)i, vlo, vhi);
+            for (int i = 0; i < SUB; ++i) {
+                const float vlo = pc.lo((float)i), vhi = pc.hi((float)i);
                 float w = (fminf(vhi, fk1) - fmaxf(vlo, fk)) * __builtin_amdgcn_rcpf(vhi - vlo);
                 w = (w < zero_tol || w < 0.0f) ? 0.0f : w;
                 acc[OFF + i] = fmaf(w, rk, acc[OFF + i]);
@@ -1383,7 +1429,8 @@ __device__ inline void bp_column_view(const BpView& v, const float* __restrict__
 // blockIdx.y is the view split: split s takes the views [s * views_per, (s + 1) * views_per) of
 // its tile and, where there is more than one, writes its sums to its own copy of the volume in
 // `parts`, which bp_reduce_kernel adds up in split order (see bp_split).
-template <int ZC, int KIND>
+// GENERAL: the fast pass takes every sub-chunk that fits (bp_column_view_fast).
+template <int ZC, int KIND, typename S, bool GENERAL>
 __global__ void __launch_bounds__(256) dd_backproject_tile_kernel(
     const float* __restrict__ q, float* __restrict__ vol, const float* __restrict__ vt,
     uint8_t* __restrict__ flags, float* __restrict__ parts, int nx, int ny, int nz, int nu, int nv,
@@ -1395,7 +1442,9 @@ __global__ void __launch_bounds__(256) dd_backproject_tile_kernel(
     q += (size_t)view_first * nv * nu;
     vt += (size_t)view_first * kBpViewStride;
     if (gridDim.y > 1) vol = parts + (size_t)blockIdx.y * nx * ny * nz;
-    __shared__ float win[2][kWinCap + kMaxUTaps - 1];
+    static_assert(ZC == S::ZC, "the shape's z extent");
+    constexpr int kPrefetch = (S::CAP + 255) / 256;  // window cells per thread
+    __shared__ float win[2][S::CAP + S::TAPS - 1];
     __shared__ int4 wring[kWinRing];
     __shared__ float scan_lds[(kMaxRows + 3) * 256];
     float* scan = scan_lds + threadIdx.x;
@@ -1428,7 +1477,8 @@ __global__ void __launch_bounds__(256) dd_backproject_tile_kernel(
     const float ya0 = fmaf((float)(ty * kTileY), dy, y0);
     const float yb0 = fmaf((float)min(ty * kTileY + kTileY - 1, ny - 1), dy, y0);
     const float za0 = Z0;
-    const float zb0 = fmaf((float)(iz0 + nz_left - 1), dz, z0);
+    // whole in z where the fast pass, which takes a last sub-chunk as whole, reads the window
+    const float zb0 = fmaf((float)(iz0 + (KIND == kBpAll ? nz_left : ZC) - 1), dz, z0);
     const float xa = fminf(xa0, xb0) - hx, xb = fmaxf(xa0, xb0) + hx;
     const float ya = fminf(ya0, yb0) - hy, yb = fmaxf(ya0, yb0) + hy;
     const float za = fminf(za0, zb0) - hz, zb = fmaxf(za0, zb0) + hz;
@@ -1465,14 +1515,14 @@ __global__ void __launch_bounds__(256) dd_backproject_tile_kernel(
     fill_windows(0, kWinRing);
     __syncthreads();
     auto fetch = [&](int view, int v0, int vn, int u0, int un, float (&pf)[kPrefetch]) {
-        if (window_mode(vn, un) != 1) return;
+        if (window_mode<S::CAP>(vn, un) != 1) return;
         if constexpr (KIND == kBpRest) {  // only the views the fast pass left
             if (view >= n_views || !tflags[view]) return;
         }
         const float* qn = q + (size_t)view * nv * nu + (size_t)v0 * nu + u0;
         // element e = threadIdx.x + 256 p of the window is (row r, column c); step by 256.
         // floor((e + 1/2) / un) in FP32: the quotient is at least 0.5/un from an integer and
-        // its rounding error below 3e-5/un, so the floor is exact (e <= 256, un <= kWinCap)
+        // its rounding error below 3e-5/un, so the floor is exact (e <= 256, un <= 4096)
         const float inv_un = __builtin_amdgcn_rcpf((float)un);
         int r = (int)(((float)threadIdx.x + 0.5f) * inv_un);
         int c = (int)threadIdx.x - __mul24(r, un);
@@ -1489,7 +1539,7 @@ __global__ void __launch_bounds__(256) dd_backproject_tile_kernel(
         }
     };
     auto put = [&](float* buf, int view, int vn, int un, const float (&pf)[kPrefetch]) {
-        if (window_mode(vn, un) != 1) return;
+        if (window_mode<S::CAP>(vn, un) != 1) return;
         if constexpr (KIND == kBpRest) {
             if (view >= n_views || !tflags[view]) return;
         }
@@ -1506,7 +1556,7 @@ __global__ void __launch_bounds__(256) dd_backproject_tile_kernel(
     int w0[2], wn[2], wu[2], wun[2];
     for (int k = 0; k < 2; ++k) {
         window_of(k, w0[k], wn[k], wu[k], wun[k]);
-        if (window_mode(wn[k], wun[k]) == 1) {
+        if (window_mode<S::CAP>(wn[k], wun[k]) == 1) {
             for (int e = threadIdx.x; e < wn[k] * wun[k]; e += 256)
                 win[k][e] = q[(size_t)k * nv * nu + (size_t)(w0[k] + e / wun[k]) * nu + wu[k] + e % wun[k]];
         }
@@ -1525,7 +1575,7 @@ __global__ void __launch_bounds__(256) dd_backproject_tile_kernel(
 #pragma unroll 1
         for (int k = 0; k < 2; ++k) {
             const int vw = view + k;
-            const int mode = window_mode(wn[k], wun[k]);
+            const int mode = window_mode<S::CAP>(wn[k], wun[k]);
             if (vw >= n_views || mode == 0) continue;
             if constexpr (KIND == kBpRest) {
                 if (!tflags[vw]) continue;
@@ -1536,18 +1586,18 @@ __global__ void __launch_bounds__(256) dd_backproject_tile_kernel(
                     continue;
                 }
                 if (!active) continue;
-                if (bp_column_view_fast<ZC>(load_view(vt, vw), win[k], wun[k], w0[k], wn[k], wu[k], wun[k], X, Y,
+                if (bp_column_view_fast<S, GENERAL>(load_view(vt, vw), win[k], wun[k], w0[k], wn[k], wu[k], wun[k], X, Y,
                                             Z0, dz, hx, hy, hz, nz_left, curved, scale, nu, nv, scan, acc))
                     tflags[vw] = 1;
             } else {
                 if (!active) continue;
                 const BpView cur = load_view(vt, vw);
                 if (mode == 1) {
-                    bp_column_view<ZC, true, KIND>(cur, win[k], wun[k], w0[k], wn[k], wu[k], wun[k], X, Y,
+                    bp_column_view<S, true, KIND, GENERAL>(cur, win[k], wun[k], w0[k], wn[k], wu[k], wun[k], X, Y,
                                                    Z0, dz, hx, hy, hz, nz_left, curved, scale, zero_tol, nu, nv,
                                                    true, scan, acc);
                 } else {
-                    bp_column_view<ZC, false, KIND>(cur, q + (size_t)vw * nv * nu, nu, 0, nv, 0, nu, X, Y, Z0,
+                    bp_column_view<S, false, KIND, GENERAL>(cur, q + (size_t)vw * nv * nu, nu, 0, nv, 0, nu, X, Y, Z0,
                                                     dz, hx, hy, hz, nz_left, curved, scale, zero_tol, nu, nv,
                                                     false, scan, acc);
                 }
@@ -2140,6 +2190,202 @@ int static_scratch(void** out) {
     return CTR_OK;
 }
 
+// Adjoint workspace: the forward projector's tables and row table (no volume tables), the
+// per-view adjoint constants, then the row-prefix table Y[view][column][nvp].
+struct AdjLayout {
+    size_t tabs_off, rows_off, at_off, yl_off, total;
+};
+
+// entries per column of the adjoint's row-prefix table: breakpoints e = 0 .. nv and a copy
+// of the total, so that the pair (k, k+1) around any point of [0, nv] is inside the column
+int adj_prefix_stride(int nv) { return nv + 2; }
+
+AdjLayout adj_layout(const ctr_geometry* g) {
+    AdjLayout L;
+    L.tabs_off = 0;
+    L.rows_off = align_up((size_t)fp_view_stride(g->nu) * g->n_views * 4, 256);
+    L.at_off = align_up(L.rows_off + (size_t)(2 * g->nv + 1) * 4, 256);
+    L.yl_off = align_up(L.at_off + (size_t)g->n_views * kAdjViewStride * 4, 256);
+    L.total = align_up(L.yl_off + (size_t)g->n_views * g->nu * adj_prefix_stride(g->nv) * 4, 256);
+    return L;
+}
+
+// Work shape of the FDK backprojection (BpCoarse, BpFine, BpFinest) and whether its fast pass holds
+// the general voxel loop, from what one voxel, one sub-chunk and one tile project to.
+//
+// The common-case pass needs a sub-chunk's rows in its table, a footprint's columns in registers
+// and a tile's window in LDS; what does not fit is left to the completing pass, which gathers from
+// global memory at about a twentieth of the speed.  The smaller sub-chunks and tiles cost more
+// set-up per voxel, so the first shape that fits is taken.
+enum BpKind { kShapeCoarse, kShapeWhole, kShapeMedium, kShapeFine, kShapeFinest };
+
+template <typename S>
+bool bp_shape_fits(const ctr_geometry* g, double cells_u, double cells_v, double spread, double closest) {
+    const double diag = sqrt(g->dx * g->dx + g->dy * g->dy);
+    // a voxel's widest footprint crosses at most floor(w) + 2 columns
+    if (floor(diag * cells_u) + 2.0 > S::TAPS) return false;
+    if (ceil((S::SUB * g->dz * cells_v + spread) * closest) + 1.0 > kMaxRows) return false;
+    const double cols = kTileX * diag * cells_u + 4.0;
+    const double rows = S::ZC * g->dz * cells_v + kTileX * spread + 4.0;
+    return cols * rows <= S::CAP;
+}
+
+BpKind bp_choose(const ctr_geometry* g) {
+    const double rx = 0.5 * g->nx * g->dx + fabs(g->recon_center[0]), ry = 0.5 * g->ny * g->dy + fabs(g->recon_center[1]);
+    const double reach = sqrt(rx * rx + ry * ry), sy = g->source_init[1];
+    const double span = fabs(sy - g->detector_init[1]);
+    // half-way out towards the source, where most voxels see at most this magnification
+    const double near = sy - 0.5 * reach, nearest = sy - reach;
+    if (!(nearest > 0.0)) return kShapeWhole;
+    const double cells_u = (g->detector_shape == CTR_DETECTOR_FLAT ? span / g->du : g->sdd / g->du) / near;
+    const double cells_v = span / g->dv / near;
+    const double z_reach = 0.5 * g->nz * g->dz + fabs(g->recon_center[2] - g->source_init[2]);
+    const double diag = sqrt(g->dx * g->dx + g->dy * g->dy);
+    // rows that a column's footprint moves by across one voxel at the volume's z end
+    const double spread = z_reach * diag / near * cells_v;
+    // plain sub-chunks throughout: a circular scan whose source height falls between two
+    // sub-chunks, a detector that sees the whole volume, voxels small enough for the series
+    const double from_top = (g->recon_center[2] + 0.5 * g->nz * g->dz - g->source_init[2]) / (BpCoarse::SUB * g->dz);
+    const bool between = from_top <= 0.0 || from_top >= (double)((g->nz + BpCoarse::SUB - 1) / BpCoarse::SUB) ||
+                         fabs(from_top - round(from_top)) < 1e-6;
+    const double v_reach = z_reach / nearest * span / g->dv + fabs(g->det_offset[1]) / g->dv + 2.0;
+    const bool plain = diag / nearest <= kSeriesRel && g->helical == 0.0 && between && v_reach <= 0.5 * g->nv &&
+                       g->nz % BpCoarse::SUB == 0;
+    if (plain && bp_shape_fits<BpCoarse>(g, cells_u, cells_v, spread, near / nearest)) return kShapeCoarse;
+    if (g->nz > BpMedium::ZC && bp_shape_fits<BpWhole>(g, cells_u, cells_v, spread, near / nearest)) return kShapeWhole;
+    if (g->nz > BpFine::ZC && bp_shape_fits<BpMedium>(g, cells_u, cells_v, spread, near / nearest)) return kShapeMedium;
+    return bp_shape_fits<BpFine>(g, cells_u, cells_v, spread, near / nearest) ? kShapeFine : kShapeFinest;
+}
+
+// calls f(shape) with the chosen shape's type
+template <typename F>
+auto bp_with_shape(BpKind k, F&& f) {
+    switch (k) {
+        case kShapeCoarse: return f(BpCoarse{});
+        case kShapeWhole: return f(BpWhole{});
+        case kShapeMedium: return f(BpMedium{});
+        case kShapeFine: return f(BpFine{});
+        default: return f(BpFinest{});
+    }
+}
+
+// FDK backprojection workspace: per-view constants, one flag byte per (tile, view), then the view
+// splits' partial volumes
+size_t bp_tiles(const ctr_geometry* g, BpKind shape) {
+    const int zc = bp_with_shape(shape, [](auto sh) { return (int)decltype(sh)::ZC; });
+    return (size_t)((g->nx + kTileX - 1) / kTileX) * ((g->ny + kTileY - 1) / kTileY) * ((g->nz + zc - 1) / zc);
+}
+
+// without view splits: per-view constants and flags
+size_t bp_base_bytes(const ctr_geometry* g, BpKind shape) {
+    return align_up((size_t)g->n_views * kBpViewStride * sizeof(float), 256) +
+           align_up(bp_tiles(g, shape) * g->n_views, 256);
+}
+
+// View splits of the FDK backprojection.  A tile's views are a serial chain, and a volume of few
+// tiles leaves most of the 256 CUs (five groups each) idle: 32 tiles at 64^3 took 617 us, one per
+// CU at 256^2 x 1 took 1012 us.  Below kBpTargetGroups tiles the views are therefore shared out to
+// so many groups per tile that about kBpTargetGroups run, each summing into its own copy of the
+// volume, added up by bp_reduce_kernel: 98 and 592 us there, 1.91 -> 1.38 ms at 151 x 163 x 107 x
+// 241 views, 4.16 -> 3.89 ms at 256^3 x 360 views (2048 tiles: a nearly empty last wave).  2560 and
+// 10240 groups are up to 10 % slower on those than 5120 (too few in flight; more copies to add).
+// A split keeps at least kBpMinViews views (64^3 x 90: 98 us with 4, 116 with 8, 160 with 16).  The
+// copies take at most kBpTargetGroups tiles' worth of memory (168 MB).
+constexpr int kBpTargetGroups = 5120;
+constexpr int kBpMinViews = 4;
+
+struct BpPlan {
+    BpKind shape;
+    int splits, views_per;
+    size_t base, bytes;  // workspace without and with the splits' partial volumes
+};
+
+// the plan of a problem whose workspace may take `budget` bytes
+BpPlan bp_plan(const ctr_geometry* g, size_t budget) {
+    BpPlan p;
+    p.shape = bp_choose(g);
+    // no shape has fewer flags than this
+    if (bp_base_bytes(g, p.shape) > budget) p.shape = kShapeWhole;
+    const long long tiles = (long long)bp_tiles(g, p.shape);
+    const size_t part = (size_t)g->nx * g->ny * g->nz * sizeof(float);
+    p.base = bp_base_bytes(g, p.shape);
+    long long want = std::min<long long>((kBpTargetGroups + tiles - 1) / tiles, g->n_views / kBpMinViews);
+    const size_t room = budget > p.base + 256 ? (budget - p.base - 256) / part : 0;
+    if (room < (size_t)std::max<long long>(want, 1)) want = (long long)room;
+    want = std::max<long long>(want, 1);
+    p.views_per = (int)((g->n_views + want - 1) / want);
+    p.views_per += p.views_per & 1;  // the kernel takes views in pairs
+    p.splits = (g->n_views + p.views_per - 1) / p.views_per;
+    p.bytes = p.base + (p.splits > 1 ? align_up(p.splits * part, 256) : 0);
+    return p;
+}
+
+// The launches of one shape: the single pass over all cases, or the fast pass over the common
+// case and then the (tile, view) pairs it left.
+template <typename S>
+hipError_t bp_passes(const ctr_geometry* g, const BpPlan& p, bool one_pass, const float* proj, float* vol,
+                            const float* vt, uint8_t* flags, float* parts, float scale, float zero_tol, int accumulate,
+                            hipStream_t s) {
+    // voxel centres: ReconCenter + (i - (n-1)/2) * d with d = (dx, -dy, -dz)
+    const float x0 = (float)(g->recon_center[0] - (g->nx - 1) / 2.0 * g->dx);
+    const float y0 = (float)(g->recon_center[1] + (g->ny - 1) / 2.0 * g->dy);
+    const float z0 = (float)(g->recon_center[2] + (g->nz - 1) / 2.0 * g->dz);
+    const int tiles_x = (g->nx + kTileX - 1) / kTileX;
+    const int tiles_y = (g->ny + kTileY - 1) / kTileY;
+    const int tiles_z = (g->nz + S::ZC - 1) / S::ZC;
+    const int curved = g->detector_shape == CTR_DETECTOR_CURVED ? 1 : 0;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles_x * tiles_y * tiles_z), p.splits), dim3(256), 0, s, proj, vol,
+                           vt, flags, parts, g->nx, g->ny, g->nz, g->nu, g->nv, g->n_views, p.views_per, x0, y0, z0,
+                           (float)g->dx, (float)(-g->dy), (float)(-g->dz), curved, scale, zero_tol, accumulate, tiles_x,
+                           tiles_y, tiles_z);
+        return hipGetLastError();
+    };
+    constexpr int ZC = S::ZC;
+    if (one_pass) return launch(dd_backproject_tile_kernel<ZC, kBpAll, S, true>);
+    constexpr bool kGeneral = !std::is_same<S, BpCoarse>::value;
+    const hipError_t e = launch(dd_backproject_tile_kernel<ZC, kBpFast, S, kGeneral>);
+    return e != hipSuccess ? e : launch(dd_backproject_tile_kernel<ZC, kBpRest, S, kGeneral>);
+}
+
+// The FDK backprojection's launches: per-view constants, the passes over every tile and view split,
+// and, with more than one split, the sum of the splits.
+int bp_fdk(const ctr_geometry* g, const double* angles, const float* proj, float* vol, int mode, float scale,
+                  float zero_tol, int accumulate, void* workspace, const BpPlan& p, hipStream_t s) {
+    int st = CTR_OK;
+    const size_t tiles = bp_tiles(g, p.shape);
+    if (tiles >= 2147483647u) return CTR_ERR_INVALID;
+    float* vt = (float*)workspace;
+    hipLaunchKernelGGL(bp_geometry_kernel, dim3((g->n_views + 255) / 256), dim3(256), 0, s, *g,
+                       angles, vt, mode);
+    if ((st = status_from_hip(hipGetLastError()))) return st;
+    uint8_t* flags = (uint8_t*)workspace + align_up((size_t)g->n_views * kBpViewStride * sizeof(float), 256);
+    float* parts = (float*)((char*)workspace + p.base);
+    // weight zeroing, a single slice (a 2D fan's, at the source height), or a caller's request for
+    // one pass (zero_tol < 0): the general kernel does every view
+    const bool one_pass = zero_tol != 0.0f || g->nz == 1;
+    if (!one_pass) {
+        const size_t flag_words = align_up(tiles * g->n_views, 256) / 4;
+        hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)std::min<size_t>((flag_words + 255) / 256, 65536)),
+                           dim3(256), 0, s, (uint32_t*)flags, flag_words);
+        if ((st = status_from_hip(hipGetLastError()))) return st;
+    }
+    const hipError_t e = bp_with_shape(p.shape, [&](auto sh) {
+        return bp_passes<decltype(sh)>(g, p, one_pass, proj, vol, vt, flags, parts, scale, zero_tol,
+                                       p.splits > 1 ? 0 : accumulate, s);
+    });
+    if (e != hipSuccess) return CTR_ERR_HIP;
+    if (p.splits == 1) return CTR_OK;
+    const size_t n = (size_t)g->nx * g->ny * g->nz;
+    if (n % 4 == 0 && (reinterpret_cast<uintptr_t>(vol) & 15) == 0)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(bp_reduce_kernel<4>), dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s,
+                           parts, vol, n, p.splits, accumulate);
+    else
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(bp_reduce_kernel<1>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
+                           parts, vol, n, p.splits, accumulate);
+    return status_from_hip(hipGetLastError());
+}
+
 }  // namespace
 
 // ==========================================================================================
@@ -2340,137 +2586,10 @@ int ctr_pixel_filter(const ctr_geometry* g, const double* spectrum, const float*
                                             (float)(1.0 / N), 1));
 }
 
-// Adjoint workspace: the forward projector's tables and row table (no volume tables), the
-// per-view adjoint constants, then the row-prefix table Y[view][column][nvp].
-struct AdjLayout {
-    size_t tabs_off, rows_off, at_off, yl_off, total;
-};
-
-// entries per column of the adjoint's row-prefix table: breakpoints e = 0 .. nv and a copy
-// of the total, so that the pair (k, k+1) around any point of [0, nv] is inside the column
-int adj_prefix_stride(int nv) { return nv + 2; }
-
-AdjLayout adj_layout(const ctr_geometry* g) {
-    AdjLayout L;
-    L.tabs_off = 0;
-    L.rows_off = align_up((size_t)fp_view_stride(g->nu) * g->n_views * 4, 256);
-    L.at_off = align_up(L.rows_off + (size_t)(2 * g->nv + 1) * 4, 256);
-    L.yl_off = align_up(L.at_off + (size_t)g->n_views * kAdjViewStride * 4, 256);
-    L.total = align_up(L.yl_off + (size_t)g->n_views * g->nu * adj_prefix_stride(g->nv) * 4, 256);
-    return L;
-}
-
-// FDK backprojection workspace: per-view constants, then one flag byte per (tile, view)
-size_t bp_tiles(const ctr_geometry* g) {
-    return (size_t)((g->nx + kTileX - 1) / kTileX) * ((g->ny + kTileY - 1) / kTileY) *
-           ((g->nz + kBpZC - 1) / kBpZC);
-}
-
-// workspace of the FDK backprojection without view splits, and the offset of the splits' volumes
-size_t bp_base_bytes(const ctr_geometry* g) {
-    return align_up((size_t)g->n_views * kBpViewStride * sizeof(float), 256) +
-           align_up(bp_tiles(g) * g->n_views, 256);
-}
-
-// View splits of the FDK backprojection.  A tile's views are a serial chain, and a volume of few
-// tiles leaves most of the 256 CUs (five groups each) idle: 32 tiles at 64^3 took 617 us, one per
-// CU at 256^2 x 1 took 1012 us.  Below kBpTargetGroups tiles the views are therefore shared out to
-// so many groups per tile that about kBpTargetGroups run, each summing into its own copy of the
-// volume, added up by bp_reduce_kernel: 98 and 592 us there, 1.91 -> 1.38 ms at 151 x 163 x 107 x
-// 241 views, 4.16 -> 3.89 ms at 256^3 x 360 views (2048 tiles: a nearly empty last wave).  2560 and
-// 10240 groups are up to 10 % slower on those than 5120 (too few in flight; more copies to add).
-// A split keeps at least kBpMinViews views (64^3 x 90: 98 us with 4, 116 with 8, 160 with 16).  The
-// copies take at most kBpTargetGroups tiles' worth of memory (168 MB).
-constexpr int kBpTargetGroups = 5120;
-constexpr int kBpMinViews = 4;
-
-struct BpSplit {
-    int splits, views_per;
-    size_t bytes;  // workspace with the splits' partial volumes
-};
-
-// the split of a problem whose workspace may take `budget` bytes
-BpSplit bp_split(const ctr_geometry* g, size_t budget) {
-    const long long tiles = (long long)bp_tiles(g);
-    const size_t part = (size_t)g->nx * g->ny * g->nz * sizeof(float);
-    const size_t base = bp_base_bytes(g);
-    long long want = std::min<long long>((kBpTargetGroups + tiles - 1) / tiles, g->n_views / kBpMinViews);
-    const size_t room = budget > base + 256 ? (budget - base - 256) / part : 0;
-    if (room < (size_t)std::max<long long>(want, 1)) want = (long long)room;
-    want = std::max<long long>(want, 1);
-    BpSplit sp;
-    sp.views_per = (int)((g->n_views + want - 1) / want);
-    sp.views_per += sp.views_per & 1;  // the kernel takes views in pairs
-    sp.splits = (g->n_views + sp.views_per - 1) / sp.views_per;
-    sp.bytes = base + (sp.splits > 1 ? align_up(sp.splits * part, 256) : 0);
-    return sp;
-}
-
 size_t ctr_dd_backproject_workspace_bytes(const ctr_geometry* g, int mode) {
     if (check_geometry(g)) return 0;
     if (mode == CTR_BP_ADJOINT) return adj_layout(g).total;
-    return bp_split(g, SIZE_MAX).bytes;
-}
-
-// The FDK backprojection's launches: per-view constants, the passes over every tile and view split,
-// and, with more than one split, the sum of the splits.
-static int bp_fdk(const ctr_geometry* g, const double* angles, const float* proj, float* vol, int mode, float scale,
-                  float zero_tol, int accumulate, void* workspace, const BpSplit& sp, hipStream_t s) {
-    int st = CTR_OK;
-    float* vt = (float*)workspace;
-    hipLaunchKernelGGL(bp_geometry_kernel, dim3((g->n_views + 255) / 256), dim3(256), 0, s, *g,
-                       angles, vt, mode);
-    if ((st = status_from_hip(hipGetLastError()))) return st;
-    // voxel centres: ReconCenter + (i - (n-1)/2) * d with d = (dx, -dy, -dz)
-    const float x0 = (float)(g->recon_center[0] - (g->nx - 1) / 2.0 * g->dx);
-    const float y0 = (float)(g->recon_center[1] + (g->ny - 1) / 2.0 * g->dy);
-    const float z0 = (float)(g->recon_center[2] + (g->nz - 1) / 2.0 * g->dz);
-    constexpr int ZC = kBpZC;
-    float* parts = (float*)((char*)workspace + bp_base_bytes(g));
-    const int pass_acc = sp.splits > 1 ? 0 : accumulate;
-    auto finish = [&]() -> int {
-        if (hipGetLastError() != hipSuccess) return CTR_ERR_HIP;
-        if (sp.splits == 1) return CTR_OK;
-        const size_t n = (size_t)g->nx * g->ny * g->nz;
-        if (n % 4 == 0 && (reinterpret_cast<uintptr_t>(vol) & 15) == 0)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(bp_reduce_kernel<4>), dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0,
-                               s, parts, vol, n, sp.splits, accumulate);
-        else
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(bp_reduce_kernel<1>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                               parts, vol, n, sp.splits, accumulate);
-        return status_from_hip(hipGetLastError());
-    };
-    const int tiles_x = (g->nx + kTileX - 1) / kTileX;
-    const int tiles_y = (g->ny + kTileY - 1) / kTileY;
-    const int tiles_z = (g->nz + ZC - 1) / ZC;
-    const long long tiles = (long long)tiles_x * tiles_y * tiles_z;
-    if (tiles >= 2147483647LL) return CTR_ERR_INVALID;
-    const int curved = g->detector_shape == CTR_DETECTOR_CURVED ? 1 : 0;
-    const float fdx = (float)g->dx, fdy = (float)(-g->dy), fdz = (float)(-g->dz);
-    // weight zeroing, a volume of one z chunk (a slice through the source height, as in a 2D
-    // fan, is on neither side of it), or a caller's request for one pass (zero_tol < 0): the
-    // general kernel does every view
-    if (zero_tol != 0.0f || tiles_z == 1) {
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(dd_backproject_tile_kernel<ZC, kBpAll>), dim3((unsigned)tiles, sp.splits),
-                           dim3(256), 0, s, proj, vol, vt, (uint8_t*)nullptr, parts, g->nx, g->ny, g->nz, g->nu,
-                           g->nv, g->n_views, sp.views_per, x0, y0, z0, fdx, fdy, fdz, curved, scale, zero_tol, pass_acc,
-                           tiles_x, tiles_y, tiles_z);
-        return finish();
-    }
-    // fast pass over the common case, then the (tile, view) pairs it left
-    uint8_t* flags = (uint8_t*)workspace + align_up((size_t)g->n_views * kBpViewStride * sizeof(float), 256);
-    const size_t flag_words = align_up((size_t)tiles * g->n_views, 256) / 4;
-    hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)std::min<size_t>((flag_words + 255) / 256, 65536)),
-                       dim3(256), 0, s, (uint32_t*)flags, flag_words);
-    if ((st = status_from_hip(hipGetLastError()))) return st;
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(dd_backproject_tile_kernel<ZC, kBpFast>), dim3((unsigned)tiles, sp.splits),
-                       dim3(256), 0, s, proj, vol, vt, flags, parts, g->nx, g->ny, g->nz, g->nu, g->nv, g->n_views,
-                       sp.views_per, x0, y0, z0, fdx, fdy, fdz, curved, scale, zero_tol, pass_acc, tiles_x, tiles_y, tiles_z);
-    if ((st = status_from_hip(hipGetLastError()))) return st;
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(dd_backproject_tile_kernel<ZC, kBpRest>), dim3((unsigned)tiles, sp.splits),
-                       dim3(256), 0, s, proj, vol, vt, flags, parts, g->nx, g->ny, g->nz, g->nu, g->nv, g->n_views,
-                       sp.views_per, x0, y0, z0, fdx, fdy, fdz, curved, scale, zero_tol, pass_acc, tiles_x, tiles_y, tiles_z);
-    return finish();
+    return bp_plan(g, SIZE_MAX).bytes;
 }
 
 int ctr_dd_backproject(const ctr_geometry* g, const double* angles, const int32_t* branch,
@@ -2511,7 +2630,7 @@ int ctr_dd_backproject(const ctr_geometry* g, const double* angles, const int32_
                            g->detector_shape == CTR_DETECTOR_CURVED ? 1 : 0, scale, 1e-6f, accumulate);
         return status_from_hip(hipGetLastError());
     }
-    return bp_fdk(g, angles, proj, vol, mode, scale, zero_tol, accumulate, workspace, bp_split(g, SIZE_MAX), s);
+    return bp_fdk(g, angles, proj, vol, mode, scale, zero_tol, accumulate, workspace, bp_plan(g, SIZE_MAX), s);
 }
 
 int ctr_dd_backproject_static(const ctr_geometry* g, const double* angles, const float* proj,
@@ -2521,13 +2640,13 @@ int ctr_dd_backproject_static(const ctr_geometry* g, const double* angles, const
     if (st) return st;
     if (mode != CTR_BP_FDK_REF && mode != CTR_BP_FDK_EDGE) return CTR_ERR_UNSUPPORTED;
     // as many view splits as the array holds beside the table and the flags (none if need be)
-    if (bp_base_bytes(g) > kStaticScratchBytes) return CTR_ERR_SCRATCH;
+    if (bp_base_bytes(g, kShapeCoarse) > kStaticScratchBytes) return CTR_ERR_SCRATCH;
     if (!angles || !proj || !vol) return CTR_ERR_INVALID;
     void* ws = nullptr;
     if ((st = static_scratch(&ws))) return st;
     // the same launches as ctr_dd_backproject: the per-view table is written by a kernel and
     // the flags are cleared by a fill kernel on `stream` before use
-    return bp_fdk(g, angles, proj, vol, mode, scale, zero_tol, accumulate, ws, bp_split(g, kStaticScratchBytes),
+    return bp_fdk(g, angles, proj, vol, mode, scale, zero_tol, accumulate, ws, bp_plan(g, kStaticScratchBytes),
                   (hipStream_t)stream);
 }
 

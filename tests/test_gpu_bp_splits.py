@@ -62,3 +62,42 @@ def test_workspace_covers_the_splits(dev):
     dummy = ctypes.c_void_p(16)  # never dereferenced: the size check fails first
     assert lib.ctr_dd_backproject(ctypes.byref(g), dummy, dummy, dummy, dummy, 0, 1.0, 0.0, 0, dummy, need - 1,
                                   None) == N.CTR_ERR_WORKSPACE
+
+
+def _check(dev, p, mode="ref", tol=TOL):
+    g = O.Geometry(p)
+    geom = ctr.ScanGeometry(p)
+    q = np.random.default_rng(5).random((g.nview, g.nv, g.nu)).astype(np.float32)
+    ref = O.backproject(g, q, mode)
+    qd = torch.from_numpy(q).to(dev)
+    peak = np.abs(ref).max()
+    two = ctr.dd_backproject(qd, geom, mode=mode).cpu().numpy()
+    one = ctr.dd_backproject(qd, geom, mode=mode, zero_tol=-1.0).cpu().numpy()
+    assert np.abs(two - ref).max() <= tol * peak
+    assert np.abs(one - ref).max() <= tol * peak
+
+
+# detector cells per voxel (at the magnification of 1.5): below, at and above the edges of the work
+# shapes (about 1, 1.4, 2 and 4), and beyond the last one (gathers from global memory)
+@pytest.mark.parametrize("cells", [0.5, 0.95, 1.05, 1.12, 1.35, 1.45, 1.95, 2.1, 3.9, 4.3, 7.0])
+@pytest.mark.parametrize("nz", [7, 17, 40])
+def test_every_work_shape_matches_the_oracle(dev, cells, nz):
+    cell = 0.75 / cells  # 0.5 mm voxels
+    _check(dev, make_params(NumberOfImage=[18, 17, nz], NumberOfViews=5, StartAngle=0.3, EndAngle=0.3 + 2 * np.pi,
+                            NumberOfDetectorPixels=[int(30 / cell), int((nz + 4) * 0.75 / cell) + 2],
+                            DetectorPixelSize=[cell, cell]))
+
+
+# sub-chunks that straddle the source height (at voxel centres and edges, and moving along a helix),
+# that the detector cuts, and that hold fewer voxels than their shape's; coarse voxels (no series)
+@pytest.mark.parametrize("nz", [1, 2, 15, 16, 24, 25, 31, 33, 48])
+@pytest.mark.parametrize("kind", ["centred", "shifted", "helix", "cut", "coarse_curved"])
+def test_ragged_and_straddling_sub_chunks_match_the_oracle(dev, nz, kind):
+    kw = {"centred": {}, "shifted": dict(ReconCenter=[0.4, -0.3, 0.25 * nz + 0.13]),
+          "helix": dict(Pitch=0.4, EndAngle=4 * np.pi, NumberOfViews=9),
+          "cut": dict(NumberOfDetectorPixels=[22, 12]),
+          "coarse_curved": dict(ImagePixelSpacing=[3.0, 3.0, 3.0], DetectorPixelSize=[5.0, 5.0],
+                                DetectorShape="Curved", NumberOfDetectorPixels=[40, 30])}[kind]
+    base = dict(NumberOfImage=[19, 18, nz], NumberOfViews=5, NumberOfDetectorPixels=[26, 44], StartAngle=0.2,
+                EndAngle=0.2 + 2 * np.pi)
+    _check(dev, make_params(**{**base, **kw}), "edge" if kind == "cut" else "ref")
