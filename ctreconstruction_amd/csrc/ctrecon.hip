@@ -10,7 +10,8 @@
 //   bp_reduce_kernel            sums the view splits' partial volumes in a fixed order
 //   adj_geometry_kernel         per-view constants of the inverse central projection
 //   adj_rowprefix_kernel        row prefix sums of projections times path length
-//   dd_adjoint_kernel           exact transpose of the forward projector, gathered per voxel
+//   adj_tile_kernel             detector windows of every (view, column tile)
+//   dd_adjoint_kernel           exact transpose of the forward projector, gathered per voxel, windows in LDS
 //   spectrum_kernel             filter magnitude from the Ram-Lak cosine series, FP64
 //   twiddle_kernel              Stockham twiddles, stage-major, FP64 -> FP32
 //   fdk_filter_kernel           cosine weight + LDS Stockham FFT convolution, two rows per FFT
@@ -1664,11 +1665,27 @@ __global__ void __launch_bounds__(256) fill_zero_kernel(uint32_t* __restrict__ p
 // sgn(nuB tt) o_a / w_a (Y(e(kc + 1)) - Y(e(kc))) with Y the linear interpolation of the
 // row prefix Y_e = sum_{k < e} y_k L_k (adj_rowprefix_kernel): one table lookup per voxel
 // boundary instead of a walk over rows.
+//
+// Organisation: a workgroup owns a 16 x 16 x TZ voxel tile and a share of the views (splits, as in
+// the FDK backprojection).  Per view the part of Y that the tile projects to (its window: the
+// candidate columns of its corners, and the row edges its z range covers at the magnifications of
+// those columns) is fetched two views ahead into registers and written to one of two LDS buffers
+// while the other is read, one barrier per view, together with the footprint lines and slab
+// fractions of the window's columns.  Rows off the detector hold the end values of Y, so a lookup
+// needs no clamp.  adj_tile_kernel works the windows out per (view, column tile); a window too
+// large for LDS is gathered from global memory after the other views.
 constexpr int kAdjViewStride = 16;
-#ifndef CTR_ADJ_ZC
-#define CTR_ADJ_ZC 16
-#endif
-constexpr int kAdjZChunk = CTR_ADJ_ZC;  // voxels along z per work-item
+constexpr int kAdjCols = 127;  // most window columns
+
+// Work shape: TZ voxels per work-item, CAP floats per LDS window: fewer voxels where the detector is
+// finer (adj_choose: the tallest whose windows fit).  Bound by VALU issue (eight instructions and one
+// two-word LDS read per voxel boundary and candidate column, 2-3 columns per voxel).  Measured
+// against one 8-byte gather from the texture path per boundary: 128^3 x 180 views 1154 -> 234 us,
+// 256^3 x 60 views 1808 -> 525 us.
+template <int TZ_, int CAP_>
+struct AdjShape {
+    static constexpr int TZ = TZ_, CAP = CAP_;
+};
 
 // Per-view constants (FP64 -> FP32):
 //   [0] branch  [1] Pt: source transverse index coordinate  [2] Ps: source slab coordinate
@@ -1770,73 +1787,308 @@ __global__ void __launch_bounds__(256) adj_rowprefix_kernel(const float* __restr
     }
 }
 
-// One work-item per voxel column chunk of kAdjZChunk voxels.  Per view and candidate detector
-// column the rows that reach the chunk are walked once; each row's z footprint (the forward
-// projector's own fma of the same table values) is overlapped with every voxel of the chunk.
-__global__ void __launch_bounds__(256) dd_adjoint_kernel(
-    const float* __restrict__ Y, float* __restrict__ vol, const float* __restrict__ tabs,
-    const float* __restrict__ at, int nx, int ny, int nz, int nu, int nv, int nvp, int n_views,
-    int stride, int curved, float scale, float zero_tol, int accumulate) {
-    const int ix = blockIdx.x * blockDim.x + threadIdx.x;
-    const int iy = blockIdx.y * blockDim.y + threadIdx.y;
-    const int iz0 = blockIdx.z * kAdjZChunk;
-    if (ix >= nx || iy >= ny) return;
-    const int nzc = min(kAdjZChunk, nz - iz0);
-    float acc[kAdjZChunk];
+// Window of a (view, 16 x 16 column tile) pair: candidate columns j0 .. j0 + |nc| - 1 (nc = 0: none)
+// and the range of 1/t, the magnification of the columns' centre rays, over the tile's slabs.
+// nc < 0: some z slab's window does not fit the LDS buffer.
+struct AdjTile {
+    int j0, nc;
+    float rt_lo, rt_hi;
+};
+
+// Row-edge window of the z range [z0, z0 + tz]: edges k0 .. k0 + rows - 1 hold the pairs around
+// every boundary's edge coordinate, with an edge to spare on either side for rounding.
+__device__ inline void adj_rows(const AdjTile& w, float gam, float nuA, float inuB, float z0, float tz, int& k0, int& rows) {
+    const float off = -nuA * inuB, c1 = z0 - gam, c2 = z0 + tz - gam, d1 = w.rt_lo * inuB, d2 = w.rt_hi * inuB;
+    const float e1 = fmaf(c1, d1, off), e2 = fmaf(c1, d2, off), e3 = fmaf(c2, d1, off), e4 = fmaf(c2, d2, off);
+    k0 = (int)floorf(fminf(fminf(e1, e2), fminf(e3, e4))) - 1;
+    rows = (int)floorf(fmaxf(fmaxf(e1, e2), fmaxf(e3, e4))) + 3 - k0;
+}
+
+// odd LDS row pitch: columns of a window start in different banks
+__device__ inline int adj_pitch(int rows) { return rows | 1; }
+
+// One thread per (view, column tile).  The edge coordinate is monotone along every line of the
+// (slab, transverse) plane in front of the source, so its extremes over the tile are at its
+// corners; t is affine in the slab for each column.  A tile that is not wholly in front of the
+// source (its depth, affine over the tile, changes sign between corners, or its slabs reach the
+// source's) has no such window and takes the gather path.
+__global__ void adj_tile_kernel(AdjTile* __restrict__ tw, const float* __restrict__ tabs, const float* __restrict__ at,
+                                int nx, int ny, int nz, int nu, int n_views, int stride, int curved, int tiles_x,
+                                int n_tiles, int tz, int slabs, int cap) {
+    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= n_views * n_tiles) return;
+    const int view = idx / n_tiles, t = idx - view * n_tiles;
+    const int x0 = (t % tiles_x) * kTileX, y0 = (t / tiles_x) * kTileY;
+    const int x1 = min(x0 + kTileX, nx) - 1, y1 = min(y0 + kTileY, ny) - 1;
+    const float* A = at + (size_t)view * kAdjViewStride;
+    const float* T = tabs + (size_t)view * stride;
+    const int br = (int)A[0];
+    AdjTile w = {0, 0, 0.0f, 0.0f};
+    if (br == CTR_BRANCH_X || br == CTR_BRANCH_Y) {
+        const bool xs = br == CTR_BRANCH_X;
+        const float n0 = (float)(xs ? x0 : y0), n1 = (float)(xs ? x1 : y1);
+        const float k0 = (float)(xs ? y0 : x0), k1 = (float)((xs ? y1 : x1) + 1);
+        float lo = 3.0e38f, hi = -3.0e38f, dlo = 3.0e38f, dhi = -3.0e38f;
 #pragma unroll
-    for (int i = 0; i < kAdjZChunk; ++i) acc[i] = 0.0f;
-    const float tol = zero_tol;
-    const float fz0 = (float)iz0, fnv = (float)nv;
-    for (int view = 0; view < n_views; ++view) {
+        for (int c = 0; c < 4; ++c) {
+            const float tk = (c & 1) ? k1 : k0, n = (c & 2) ? n1 : n0;
+            const float e = adj_edge_coord(A, tk, n, curved);
+            const float depth = (tk - A[1]) * A[3] * A[5] - A[4] * (n - A[2]);
+            lo = fminf(lo, e);
+            hi = fmaxf(hi, e);
+            dlo = fminf(dlo, depth);
+            dhi = fmaxf(dhi, depth);
+        }
+        const bool beside = (A[2] > n0 - 1.0f && A[2] < n1 + 1.0f) || !(dlo * dhi > 0.0f);
+        const int j0 = beside ? 0 : max((int)floorf(lo - 0.02f), 0);
+        const int j1 = beside ? nu - 1 : min((int)floorf(hi + 0.02f), nu - 1);
+        if (j0 <= j1) {
+            w.j0 = j0;
+            w.nc = j1 - j0 + 1;
+            float rlo = 3.0e38f, rhi = -3.0e38f;
+            for (int j = j0; j <= j1; ++j) {
+                const float t0 = T[2 * nu + 2 + j], dt = T[3 * nu + 2 + j];
+                const float r0 = __builtin_amdgcn_rcpf(fmaf(dt, n0, t0)), r1 = __builtin_amdgcn_rcpf(fmaf(dt, n1, t0));
+                rlo = fminf(rlo, fminf(r0, r1));
+                rhi = fmaxf(rhi, fmaxf(r0, r1));
+            }
+            w.rt_lo = rlo;
+            w.rt_hi = rhi;
+            // the span of a slab's edges grows with its distance from the source height, so the
+            // first or the last slab has the largest (two rows for the others' rounding)
+            int most = 0;
+            for (int e = 0; e < 2; ++e) {
+                int first, rows;
+                adj_rows(w, T[6 * nu + 2], A[11], A[12], (float)((e ? slabs - 1 : 0) * tz), (float)tz, first, rows);
+                most = max(most, rows);
+            }
+            if (beside || w.nc > kAdjCols || most > cap || adj_pitch(most + 2) * w.nc > cap) w.nc = -w.nc;
+        }
+    }
+    tw[idx] = w;
+}
+
+// One column's share of a work-item's voxels: boundary c of the volume has the edge coordinate
+// (c - gam) de + off, which is evaluated from the start of its group of 16 voxels whatever the
+// shape, so that every shape rounds it alike: next to a ray that only grazes the volume (and whose
+// SART weight is therefore huge) a boundary's rounding is visible in the result.
+template <int TZ, typename F>
+__device__ inline void adj_chunk(int iz0, float gam, float off, float de, float kap, F&& lookup, float (&acc)[TZ]) {
+    constexpr int G = TZ < 16 ? TZ : 16;
+#pragma unroll
+    for (int h = 0; h < TZ; h += G) {
+        const int first = (iz0 + h) & ~15;
+        const float eb = fmaf((float)first - gam, de, off);
+        const float f0 = TZ < 16 ? (float)(iz0 - first) : 0.0f;
+        float prev = lookup(TZ < 16 ? fmaf(f0, de, eb) : eb);
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+            const float here = lookup(fmaf(f0 + (float)(i + 1), de, eb));
+            acc[h + i] = fmaf(kap, here - prev, acc[h + i]);
+            prev = here;
+        }
+    }
+}
+
+// vol = (accumulate ? vol : 0) + scale * A^T y of the split's views (blockIdx.y), or that into the
+// split's volume in `parts` (added up by bp_reduce_kernel).
+template <typename S>
+__global__ void __launch_bounds__(256) dd_adjoint_kernel(
+    const float* __restrict__ Y, float* __restrict__ vol, float* __restrict__ parts, const float* __restrict__ tabs,
+    const float* __restrict__ at, const AdjTile* __restrict__ tw, int nx, int ny, int nz, int nu, int nv, int nvp,
+    int all_views, int views_per, int stride, int curved, float scale, float tol, int accumulate, int tiles_x,
+    int tiles_y, int tiles_z) {
+    constexpr int TZ = S::TZ, CAP = S::CAP, kPre = (CAP + 255) / 256;
+    __shared__ float win[2][CAP];
+    __shared__ float4 cols[2][kAdjCols + 1];  // per column edge: footprint line (at, per slab), slab fraction (at, per slab)
+    const int view0 = blockIdx.y * views_per, n_views = min(views_per, all_views - view0);
+    if (gridDim.y > 1) vol = parts + (size_t)blockIdx.y * nx * ny * nz;
+    // XCD-aware tile order: workgroup b runs on XCD b % 8; give each XCD a contiguous range
+    const int n_tiles = tiles_x * tiles_y, T = n_tiles * tiles_z;
+    const int b = blockIdx.x, xcd = b & 7, local = b >> 3, qd = T >> 3, rm = T & 7;
+    const int tl = (xcd < rm) ? xcd * (qd + 1) + local : rm * (qd + 1) + (xcd - rm) * qd + local;
+    const int tile = tl % n_tiles, tid = threadIdx.x;
+    // each wavefront takes an 8 x 8 quadrant of the tile's columns
+    const int lx = (tid & 7) | ((tid >> 3) & 8), ly = ((tid >> 3) & 7) | ((tid >> 4) & 8);
+    const int ix = (tile % tiles_x) * kTileX + lx, iy = (tile / tiles_x) * kTileY + ly, iz0 = (tl / n_tiles) * TZ;
+    const bool active = ix < nx && iy < ny;
+    const float fz0 = (float)iz0;
+    float acc[TZ];
+#pragma unroll
+    for (int i = 0; i < TZ; ++i) acc[i] = 0.0f;
+
+    struct View {
+        AdjTile w;
+        int k0, rows;
+        bool go;    // staged in LDS
+        bool left;  // gathered from global memory at the end
+    };
+    bool gather = false;
+    auto view_of = [&](int v) {
+        View q;
+        q.go = q.left = false;
+        if (v >= n_views) return q;
+        const int view = view0 + v;
+        q.w = tw[(size_t)view * n_tiles + tile];
+        if (q.w.nc <= 0) {
+            q.left = q.w.nc < 0;
+            return q;
+        }
         const float* A = at + (size_t)view * kAdjViewStride;
-        const int br = (int)A[0];
-        if (br != CTR_BRANCH_X && br != CTR_BRANCH_Y) continue;
-        const bool xs = (br == CTR_BRANCH_X);
-        const int n = xs ? ix : iy;     // slab
-        const int ka = xs ? iy : ix;    // transverse cell
-        const float fn = (float)n, fka = (float)ka;
+        adj_rows(q.w, tabs[(size_t)view * stride + 6 * nu + 2], A[11], A[12], fz0, (float)TZ, q.k0, q.rows);
+        q.k0 = __builtin_amdgcn_readfirstlane(q.k0);
+        q.rows = __builtin_amdgcn_readfirstlane(q.rows);
+        // rows wholly off the detector: every boundary reads the same end value
+        if (q.k0 >= nv || q.k0 + q.rows <= 1) return q;
+        q.go = q.rows <= CAP && adj_pitch(q.rows) * q.w.nc <= CAP;
+        q.left = !q.go;
+        return q;
+    };
+    // the window's cells e = tid + 256 p in registers: column c, row r (c from a reciprocal: the
+    // quotient is at least 0.5/rows from an integer, its rounding error below 3e-5/rows)
+    float pre[kPre];
+    float4 pcol;
+    auto fetch = [&](int v, const View& q) {
+        if (!q.go) return;
+        const float* Yv = Y + ((size_t)(view0 + v) * nu + q.w.j0) * nvp;
+        const float inv = __builtin_amdgcn_rcpf((float)q.rows);
+        int c = (int)(((float)tid + 0.5f) * inv);
+        int r = tid - __mul24(c, q.rows);
+        const int dc = (int)(256.5f * inv), dr = 256 - __mul24(dc, q.rows);
+#pragma unroll
+        for (int p = 0; p < kPre; ++p) {
+            if (c < q.w.nc) pre[p] = Yv[c * nvp + min(max(q.k0 + r, 0), nv)];
+            c += dc;
+            r += dr;
+            if (r >= q.rows) {
+                r -= q.rows;
+                ++c;
+            }
+        }
+        if (tid <= q.w.nc) {
+            const float* Tj = tabs + (size_t)(view0 + v) * stride + q.w.j0 + tid;
+            const bool centre = tid < q.w.nc;
+            pcol = make_float4(Tj[0], Tj[nu + 1], centre ? Tj[2 * nu + 2] : 1.0f, centre ? Tj[3 * nu + 2] : 0.0f);
+        }
+    };
+    auto put = [&](int buf, const View& q) {
+        if (!q.go) return;
+        const int pitch = adj_pitch(q.rows);
+        const float inv = __builtin_amdgcn_rcpf((float)q.rows);
+        int c = (int)(((float)tid + 0.5f) * inv);
+        int r = tid - __mul24(c, q.rows);
+        const int dc = (int)(256.5f * inv), dr = 256 - __mul24(dc, q.rows);
+#pragma unroll
+        for (int p = 0; p < kPre; ++p) {
+            if (c < q.w.nc) win[buf][__mul24(c, pitch) + r] = pre[p];
+            c += dc;
+            r += dr;
+            if (r >= q.rows) {
+                r -= q.rows;
+                ++c;
+            }
+        }
+        if (tid <= q.w.nc) cols[buf][tid] = pcol;
+    };
+    // candidate columns of this work-item's voxel column: the inverse projection is accurate to
+    // ~1e-5 edge; a 0.01 margin covers its rounding
+    auto candidates = [&](const float* A, bool xs, int& j0, int& j1) {
+        const float fn = (float)(xs ? ix : iy), fka = (float)(xs ? iy : ix);
         const float e1 = adj_edge_coord(A, fka, fn, curved);
         const float e2 = adj_edge_coord(A, fka + 1.0f, fn, curved);
-        // the inverse projection is accurate to ~1e-5 edge; a 0.01 margin covers its rounding
-        const int j0 = max((int)floorf(fminf(e1, e2) - 0.01f), 0);
-        const int j1 = min((int)floorf(fmaxf(e1, e2) + 0.01f), nu - 1);
-        const float* T = tabs + (size_t)view * stride;
-        const float gam = T[6 * nu + 2];
-        const float nuA = A[11], inuB = A[12];
-        const float* Yv = Y + (size_t)view * nu * nvp;
-        for (int j = j0; j <= j1; ++j) {
-            const float a1 = fmaf(T[nu + 1 + j], fn, T[j]);
-            const float a2 = fmaf(T[nu + 2 + j], fn, T[j + 1]);
-            const float alo = fminf(a1, a2), ahi = fmaxf(a1, a2);
-            const float wa = ahi - alo;
-            const float oa = fminf(ahi, fka + 1.0f) - fmaxf(alo, fka);
-            if (!(oa > 0.0f) || oa < tol * wa) continue;
-            const float t = fmaf(T[3 * nu + 2 + j], fn, T[2 * nu + 2 + j]);
-            const float rt = __builtin_amdgcn_rcpf(t);
-            // edge coordinate of the chunk's voxel boundaries: e_i = e_0 + i de
-            const float de = rt * inuB;
-            const float eb = fmaf(fz0 - gam, de, -nuA * inuB);
-            const float kap = (de > 0.0f ? oa : -oa) * __builtin_amdgcn_rcpf(wa);  // sgn(nuB tt) o_a / w_a
-            const char* col = reinterpret_cast<const char*>(Yv + (size_t)j * nvp);
-            auto lookup = [&](float e) {
-                const float ec = __builtin_amdgcn_fmed3f(e, 0.0f, fnv);
-                const int k = (int)ec;
-                const PTaps p = *reinterpret_cast<const PTaps*>(col + 4 * k);
-                return fmaf(__builtin_amdgcn_fractf(ec), p.b - p.a, p.a);
-            };
-            float prev = lookup(eb);
-#pragma unroll
-            for (int i = 0; i < kAdjZChunk; ++i) {
-                const float cur = lookup(fmaf((float)(i + 1), de, eb));
-                acc[i] = fmaf(kap, cur - prev, acc[i]);
-                prev = cur;
+        j0 = max((int)floorf(fminf(e1, e2) - 0.01f), 0);
+        j1 = min((int)floorf(fmaxf(e1, e2) + 0.01f), nu - 1);
+    };
+
+    View cur = view_of(0), nxt = view_of(1);
+    gather = cur.left || nxt.left;
+    fetch(0, cur);
+    put(0, cur);
+    fetch(1, nxt);
+    __syncthreads();
+    for (int v = 0; v < n_views; ++v) {
+        if (cur.go && active) {
+            const int view = view0 + v;
+            const float* A = at + (size_t)view * kAdjViewStride;
+            const bool xs = (int)A[0] == CTR_BRANCH_X;
+            const float fn = (float)(xs ? ix : iy), fka = (float)(xs ? iy : ix);
+            int j0, j1;
+            candidates(A, xs, j0, j1);
+            j0 = max(j0, cur.w.j0) - cur.w.j0;
+            j1 = min(j1, cur.w.j0 + cur.w.nc - 1) - cur.w.j0;
+            const float gam = tabs[(size_t)view * stride + 6 * nu + 2], inuB = A[12];
+            const float off = -A[11] * inuB;
+            const int pitch = adj_pitch(cur.rows);
+            const float4* cw = cols[v & 1];
+            float4 col = cw[min(j0, cur.w.nc)];
+            float a1 = fmaf(col.y, fn, col.x);
+            for (int j = j0; j <= j1; ++j) {
+                const float4 next = cw[j + 1];
+                const float a2 = fmaf(next.y, fn, next.x);
+                const float alo = fminf(a1, a2), ahi = fmaxf(a1, a2);
+                const float wa = ahi - alo;
+                const float oa = fminf(ahi, fka + 1.0f) - fmaxf(alo, fka);
+                if (oa > 0.0f && oa >= tol * wa) {
+                    const float de = __builtin_amdgcn_rcpf(fmaf(col.w, fn, col.z)) * inuB;
+                    const float kap = (de > 0.0f ? oa : -oa) * __builtin_amdgcn_rcpf(wa);  // sgn(nuB tt) o_a / w_a
+                    const float* line = &win[v & 1][__mul24(j, pitch) - cur.k0];
+                    auto lookup = [&](float e) {
+                        const int k = (int)floorf(e);
+                        const float pa = line[k], pb = line[k + 1];
+                        return fmaf(__builtin_amdgcn_fractf(e), pb - pa, pa);
+                    };
+                    adj_chunk<TZ>(iz0, gam, off, de, kap, lookup, acc);
+                }
+                col = next;
+                a1 = a2;
+            }
+        }
+        put((v + 1) & 1, nxt);
+        cur = nxt;
+        nxt = view_of(v + 2);
+        gather |= nxt.left;
+        fetch(v + 2, nxt);
+        __syncthreads();
+    }
+    if (gather && active) {
+        const float fnv = (float)nv;
+#pragma unroll 1
+        for (int v = 0; v < n_views; ++v) {
+            const int view = view0 + v;
+            if (!view_of(v).left) continue;
+            const float* A = at + (size_t)view * kAdjViewStride;
+            const float* Tv = tabs + (size_t)view * stride;
+            const bool xs = (int)A[0] == CTR_BRANCH_X;
+            const float fn = (float)(xs ? ix : iy), fka = (float)(xs ? iy : ix);
+            const float gam = Tv[6 * nu + 2], inuB = A[12];
+            int j0, j1;
+            candidates(A, xs, j0, j1);
+            for (int j = j0; j <= j1; ++j) {
+                const float a1 = fmaf(Tv[nu + 1 + j], fn, Tv[j]), a2 = fmaf(Tv[nu + 2 + j], fn, Tv[j + 1]);
+                const float alo = fminf(a1, a2), ahi = fmaxf(a1, a2);
+                const float wa = ahi - alo;
+                const float oa = fminf(ahi, fka + 1.0f) - fmaxf(alo, fka);
+                if (!(oa > 0.0f) || oa < tol * wa) continue;
+                const float de = __builtin_amdgcn_rcpf(fmaf(Tv[3 * nu + 2 + j], fn, Tv[2 * nu + 2 + j])) * inuB;
+                const float kap = (de > 0.0f ? oa : -oa) * __builtin_amdgcn_rcpf(wa);
+                const float* line = Y + ((size_t)view * nu + j) * nvp;
+                auto lookup = [&](float e) {
+                    const float ec = __builtin_amdgcn_fmed3f(e, 0.0f, fnv);
+                    const int k = (int)ec;
+                    const float pa = line[k], pb = line[k + 1];
+                    return fmaf(__builtin_amdgcn_fractf(ec), pb - pa, pa);
+                };
+                adj_chunk<TZ>(iz0, gam, -A[11] * inuB, de, kap, lookup, acc);
             }
         }
     }
-    for (int i = 0; i < nzc; ++i) {
+    if (!active) return;
+#pragma unroll
+    for (int i = 0; i < TZ; ++i) {
+        if (iz0 + i >= nz) break;
         const size_t idx = ((size_t)(iz0 + i) * ny + iy) * nx + ix;
-        const float v = acc[i] * scale;
-        vol[idx] = accumulate ? vol[idx] + v : v;
+        const float r = acc[i] * scale;
+        vol[idx] = accumulate ? vol[idx] + r : r;
     }
 }
 
@@ -2190,26 +2442,6 @@ int static_scratch(void** out) {
     return CTR_OK;
 }
 
-// Adjoint workspace: the forward projector's tables and row table (no volume tables), the
-// per-view adjoint constants, then the row-prefix table Y[view][column][nvp].
-struct AdjLayout {
-    size_t tabs_off, rows_off, at_off, yl_off, total;
-};
-
-// entries per column of the adjoint's row-prefix table: breakpoints e = 0 .. nv and a copy
-// of the total, so that the pair (k, k+1) around any point of [0, nv] is inside the column
-int adj_prefix_stride(int nv) { return nv + 2; }
-
-AdjLayout adj_layout(const ctr_geometry* g) {
-    AdjLayout L;
-    L.tabs_off = 0;
-    L.rows_off = align_up((size_t)fp_view_stride(g->nu) * g->n_views * 4, 256);
-    L.at_off = align_up(L.rows_off + (size_t)(2 * g->nv + 1) * 4, 256);
-    L.yl_off = align_up(L.at_off + (size_t)g->n_views * kAdjViewStride * 4, 256);
-    L.total = align_up(L.yl_off + (size_t)g->n_views * g->nu * adj_prefix_stride(g->nv) * 4, 256);
-    return L;
-}
-
 // Work shape of the FDK backprojection (BpCoarse, BpFine, BpFinest) and whether its fast pass holds
 // the general voxel loop, from what one voxel, one sub-chunk and one tile project to.
 //
@@ -2320,6 +2552,131 @@ BpPlan bp_plan(const ctr_geometry* g, size_t budget) {
     return p;
 }
 
+// entries per column of the adjoint's row-prefix table: breakpoints e = 0 .. nv and a copy
+// of the total, so that the pair (k, k+1) around any point of [0, nv] is inside the column
+int adj_prefix_stride(int nv) { return nv + 2; }
+
+using AdjDeep = AdjShape<32, 2048>;
+using AdjMid = AdjShape<16, 2048>;
+using AdjFlat = AdjShape<8, 4096>;
+enum AdjKind { kAdjDeep, kAdjMid, kAdjFlat };
+
+template <typename F>
+auto adj_with_shape(AdjKind k, F&& f) {
+    switch (k) {
+        case kAdjDeep: return f(AdjDeep{});
+        case kAdjMid: return f(AdjMid{});
+        default: return f(AdjFlat{});
+    }
+}
+
+template <typename S>
+bool adj_shape_fits(const ctr_geometry* g, double cells_u, double cells_v, double spread) {
+    const double cols = kTileX * sqrt(g->dx * g->dx + g->dy * g->dy) * cells_u + 4.0;
+    const double rows = S::TZ * g->dz * cells_v + kTileX * spread + 6.0;
+    return cols * rows <= S::CAP && cols <= kAdjCols;
+}
+
+AdjKind adj_choose(const ctr_geometry* g) {
+    const double rx = 0.5 * g->nx * g->dx + fabs(g->recon_center[0]), ry = 0.5 * g->ny * g->dy + fabs(g->recon_center[1]);
+    const double near = g->sad - 0.7 * sqrt(rx * rx + ry * ry);
+    if (!(near > 0.0)) return kAdjMid;
+    const double cells_u = g->sdd / g->du / near, cells_v = g->sdd / g->dv / near;
+    const double z_reach = 0.5 * g->nz * g->dz + fabs(g->recon_center[2] - g->source_init[2]);
+    const double spread = z_reach * sqrt(g->dx * g->dx + g->dy * g->dy) / near * cells_v;
+    if (g->nz > AdjMid::TZ && adj_shape_fits<AdjDeep>(g, cells_u, cells_v, spread)) return kAdjDeep;
+    if (g->nz > AdjFlat::TZ && adj_shape_fits<AdjMid>(g, cells_u, cells_v, spread)) return kAdjMid;
+    return kAdjFlat;
+}
+
+// Adjoint workspace: the forward projector's tables and row table (no volume tables), the
+// per-view adjoint constants, the windows of every (view, column tile), the row-prefix table
+// Y[view][column][nvp], then the view splits' partial volumes.
+struct AdjLayout {
+    AdjKind shape;
+    int tiles_x, tiles_y, tiles_z, tz, cap, splits, views_per;
+    size_t tabs_off, rows_off, at_off, tw_off, yl_off, parts_off, total;
+};
+
+AdjLayout adj_layout(const ctr_geometry* g) {
+    AdjLayout L;
+    L.shape = adj_choose(g);
+    L.tz = adj_with_shape(L.shape, [](auto sh) { return (int)decltype(sh)::TZ; });
+    L.cap = adj_with_shape(L.shape, [](auto sh) { return (int)decltype(sh)::CAP; });
+    L.tiles_x = (g->nx + kTileX - 1) / kTileX;
+    L.tiles_y = (g->ny + kTileY - 1) / kTileY;
+    L.tiles_z = (g->nz + L.tz - 1) / L.tz;
+    const long long n_tiles = (long long)L.tiles_x * L.tiles_y;
+    // view splits as in the FDK backprojection (2560 and 10240 groups: 1 and 5 % slower on 128^3 x 180)
+    long long want = std::min<long long>((kBpTargetGroups + n_tiles * L.tiles_z - 1) / (n_tiles * L.tiles_z),
+                                         g->n_views / kBpMinViews);
+    want = std::max<long long>(want, 1);
+    L.views_per = (int)((g->n_views + want - 1) / want);
+    L.splits = (g->n_views + L.views_per - 1) / L.views_per;
+    L.tabs_off = 0;
+    L.rows_off = align_up((size_t)fp_view_stride(g->nu) * g->n_views * 4, 256);
+    L.at_off = align_up(L.rows_off + (size_t)(2 * g->nv + 1) * 4, 256);
+    L.tw_off = align_up(L.at_off + (size_t)g->n_views * kAdjViewStride * 4, 256);
+    L.yl_off = align_up(L.tw_off + (size_t)g->n_views * n_tiles * sizeof(AdjTile), 256);
+    L.parts_off = align_up(L.yl_off + (size_t)g->n_views * g->nu * adj_prefix_stride(g->nv) * 4, 256);
+    L.total = L.parts_off + (L.splits > 1 ? align_up((size_t)L.splits * g->nx * g->ny * g->nz * 4, 256) : 0);
+    return L;
+}
+
+// vol = (accumulate ? vol : 0) + the splits' partial volumes
+int bp_reduce(const ctr_geometry* g, const float* parts, float* vol, int splits, int accumulate, hipStream_t s) {
+    const size_t n = (size_t)g->nx * g->ny * g->nz;
+    if (n % 4 == 0 && (reinterpret_cast<uintptr_t>(vol) & 15) == 0)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(bp_reduce_kernel<4>), dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s,
+                           parts, vol, n, splits, accumulate);
+    else
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(bp_reduce_kernel<1>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
+                           parts, vol, n, splits, accumulate);
+    return status_from_hip(hipGetLastError());
+}
+
+// The matched adjoint's launches: the forward projector's tables, the per-view constants and
+// windows, the row-prefix table, the gather over all voxels and views, the sum of the splits.
+int adj_run(const ctr_geometry* g, const double* angles, const int32_t* branch, const float* proj, float* vol,
+            float scale, int accumulate, void* workspace, hipStream_t s) {
+    const AdjLayout L = adj_layout(g);
+    char* ws = (char*)workspace;
+    float* tabs = (float*)(ws + L.tabs_off);
+    float* rows = (float*)(ws + L.rows_off);
+    float* at = (float*)(ws + L.at_off);
+    AdjTile* tw = (AdjTile*)(ws + L.tw_off);
+    float* yp = (float*)(ws + L.yl_off);  // row-prefix table
+    float* parts = (float*)(ws + L.parts_off);
+    const int stride = fp_view_stride(g->nu), n_tiles = L.tiles_x * L.tiles_y;
+    if ((double)n_tiles * g->n_views >= 2147483647.0 || (double)n_tiles * L.tiles_z >= 2147483647.0)
+        return CTR_ERR_INVALID;
+    const int curved = g->detector_shape == CTR_DETECTOR_CURVED ? 1 : 0;
+    int st = CTR_OK;
+    const int gx = (std::max(g->nu + 1, g->nv + 1) + 255) / 256;
+    hipLaunchKernelGGL(fp_geometry_kernel, dim3(gx, g->n_views), dim3(256), 0, s, *g, angles, branch, tabs, rows, stride);
+    if ((st = status_from_hip(hipGetLastError()))) return st;
+    hipLaunchKernelGGL(adj_geometry_kernel, dim3((g->n_views + 255) / 256), dim3(256), 0, s, *g, angles, branch, at);
+    if ((st = status_from_hip(hipGetLastError()))) return st;
+    hipLaunchKernelGGL(adj_tile_kernel, dim3((unsigned)(((size_t)g->n_views * n_tiles + 255) / 256)), dim3(256), 0, s, tw,
+                       tabs, at, g->nx, g->ny, g->nz, g->nu, g->n_views, stride, curved, L.tiles_x, n_tiles, L.tz,
+                       L.tiles_z, L.cap);
+    if ((st = status_from_hip(hipGetLastError()))) return st;
+    const int nvp = adj_prefix_stride(g->nv);
+    hipLaunchKernelGGL(adj_rowprefix_kernel, dim3((g->nu + 31) / 32, g->n_views), dim3(256), 0, s, proj, yp, tabs, rows,
+                       g->nu, g->nv, nvp, stride);
+    if ((st = status_from_hip(hipGetLastError()))) return st;
+    const hipError_t e = adj_with_shape(L.shape, [&](auto sh) {
+        // transverse overlaps under 1e-6 of the footprint are dropped, as in ctr_dd_forward
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(dd_adjoint_kernel<decltype(sh)>), dim3((unsigned)(n_tiles * L.tiles_z), L.splits),
+                           dim3(256), 0, s, yp, vol, parts, tabs, at, tw, g->nx, g->ny, g->nz, g->nu, g->nv, nvp,
+                           g->n_views, L.views_per, stride, curved, scale, 1e-6f, L.splits > 1 ? 0 : accumulate, L.tiles_x,
+                           L.tiles_y, L.tiles_z);
+        return hipGetLastError();
+    });
+    if ((st = status_from_hip(e))) return st;
+    return L.splits > 1 ? bp_reduce(g, parts, vol, L.splits, accumulate, s) : CTR_OK;
+}
+
 // The launches of one shape: the single pass over all cases, or the fast pass over the common
 // case and then the (tile, view) pairs it left.
 template <typename S>
@@ -2376,14 +2733,7 @@ int bp_fdk(const ctr_geometry* g, const double* angles, const float* proj, float
     });
     if (e != hipSuccess) return CTR_ERR_HIP;
     if (p.splits == 1) return CTR_OK;
-    const size_t n = (size_t)g->nx * g->ny * g->nz;
-    if (n % 4 == 0 && (reinterpret_cast<uintptr_t>(vol) & 15) == 0)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(bp_reduce_kernel<4>), dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s,
-                           parts, vol, n, p.splits, accumulate);
-    else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(bp_reduce_kernel<1>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                           parts, vol, n, p.splits, accumulate);
-    return status_from_hip(hipGetLastError());
+    return bp_reduce(g, parts, vol, p.splits, accumulate, s);
 }
 
 }  // namespace
@@ -2605,30 +2955,7 @@ int ctr_dd_backproject(const ctr_geometry* g, const double* angles, const int32_
     if (mode == CTR_BP_ADJOINT) {
         // transpose of ctr_dd_forward: its weights (and its 1e-6 transverse weight zeroing) by construction
         if (!branch) return CTR_ERR_INVALID;
-        const AdjLayout L = adj_layout(g);
-        char* ws = (char*)workspace;
-        float* tabs = (float*)(ws + L.tabs_off);
-        float* rows = (float*)(ws + L.rows_off);
-        float* at = (float*)(ws + L.at_off);
-        float* yp = (float*)(ws + L.yl_off);  // row-prefix table
-        const int stride = fp_view_stride(g->nu);
-        const int gx = (std::max(g->nu + 1, g->nv + 1) + 255) / 256;
-        hipLaunchKernelGGL(fp_geometry_kernel, dim3(gx, g->n_views), dim3(256), 0, s, *g, angles,
-                           branch, tabs, rows, stride);
-        if ((st = status_from_hip(hipGetLastError()))) return st;
-        hipLaunchKernelGGL(adj_geometry_kernel, dim3((g->n_views + 255) / 256), dim3(256), 0, s, *g,
-                           angles, branch, at);
-        if ((st = status_from_hip(hipGetLastError()))) return st;
-        const int nvp = adj_prefix_stride(g->nv);
-        hipLaunchKernelGGL(adj_rowprefix_kernel, dim3((g->nu + 31) / 32, g->n_views), dim3(256), 0, s, proj,
-                           yp, tabs, rows, g->nu, g->nv, nvp, stride);
-        if ((st = status_from_hip(hipGetLastError()))) return st;
-        const dim3 block(64, 4);
-        const dim3 grid((g->nx + 63) / 64, (g->ny + 3) / 4, (g->nz + kAdjZChunk - 1) / kAdjZChunk);
-        hipLaunchKernelGGL(dd_adjoint_kernel, grid, block, 0, s, yp, vol, tabs, at, g->nx, g->ny, g->nz,
-                           g->nu, g->nv, nvp, g->n_views, stride,
-                           g->detector_shape == CTR_DETECTOR_CURVED ? 1 : 0, scale, 1e-6f, accumulate);
-        return status_from_hip(hipGetLastError());
+        return adj_run(g, angles, branch, proj, vol, scale, accumulate, workspace, s);
     }
     return bp_fdk(g, angles, proj, vol, mode, scale, zero_tol, accumulate, workspace, bp_plan(g, SIZE_MAX), s);
 }
