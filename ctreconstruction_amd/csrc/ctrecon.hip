@@ -750,6 +750,132 @@ __global__ void __launch_bounds__(64 * kFpWaves, CTR_FP_MIN_WAVES) dd_forward_ke
     }
 }
 
+// Detectors of at most kThinRows rows (2-D fans and scanners of a few rows), where lanes that own row
+// edges would idle: lane = detector column, all its row edges in registers.  One workgroup per
+// (view, 64 columns); wavefront w takes the slabs w, w + 4, ..., and the four sums of every edge
+// meet in LDS.  The arithmetic of an edge is dd_forward_kernel's: the transverse overlaps of the
+// column's footprint over its width times the slab's magnification, the z integral of a line up to
+// the edge interpolated in the prefix table, FP64 sums over the slabs.  Neighbouring columns cross
+// neighbouring lines, so a wavefront's table reads are one short run while the lines are short.
+// Bound by VALU issue (290 cycles per wavefront and slab for a single row).  Measured: 256^2, 360 views
+// of 512 columns: 1404 us by dd_forward_kernel (2 of 64 lanes at work), 88 us here; 256^2 x 64 and 256^3,
+// 360 views of 512 x 4 and x 3 cells: 1330 and 1362 us by that kernel, 610 and 560 us here, where each
+// lane's table reads touch a line of their own: more rows are left to that kernel.  Four slabs' reads
+// issued before their use, unconditionally (weight 0 off the volume): 105 us, and 3 times slower where
+// half of the columns miss the volume.
+constexpr int kThinRows = 4;
+
+// ONE_Z: a volume of one slice, whose integral up to c is c times the voxel: one read per line serves
+// every edge.
+template <int NE, bool ONE_Z>
+__global__ void __launch_bounds__(256) dd_forward_thin_kernel(
+    const float* __restrict__ t_ys, const float* __restrict__ t_xs, float* __restrict__ proj,
+    const float* __restrict__ tabs, const float* __restrict__ rows, const int32_t* __restrict__ branch, int nx, int ny,
+    int nz, int nzp, int nu, int nv, int stride, float zero_tol) {
+    __shared__ double part[4][NE][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int view = blockIdx.y, col = blockIdx.x * 64 + lane, j = min(col, nu - 1);
+    const int br = branch[view];
+    float* out = proj + (size_t)view * nv * nu;
+    if (br != CTR_BRANCH_X && br != CTR_BRANCH_Y) {  // z slabs: dd_forward_zslab_kernel
+        if (wave < nv && col < nu) out[(size_t)wave * nu + col] = 0.0f;
+        return;
+    }
+    const bool xs = br == CTR_BRANCH_X;
+    const float* __restrict__ src = xs ? t_xs : t_ys;
+    const int ns = xs ? nx : ny, nt = xs ? ny : nx;
+    const float fnt = (float)nt, fnz = (float)nz;
+    const float* T = tabs + (size_t)view * stride;
+    const float gam = T[6 * nu + 2];
+    const float a_al = T[j], b_al = T[j + 1], a_be = T[nu + 1 + j], b_be = T[nu + 2 + j];
+    const float T0 = T[2 * nu + 2 + j], dT = T[3 * nu + 2 + j];
+    float nue[NE];
+#pragma unroll
+    for (int e = 0; e < NE; ++e) nue[e] = rows[min(e, nv)];
+    double H[NE];
+#pragma unroll
+    for (int e = 0; e < NE; ++e) H[e] = 0.0;
+    for (int n = wave; n < ns; n += 4) {
+        const float fn = (float)n;
+        const float a1 = fmaf(a_be, fn, a_al), a2 = fmaf(b_be, fn, b_al);
+        const float alo = fminf(a1, a2), ahi = fmaxf(a1, a2);
+        const int ks = max((int)floorf(alo), 0), ke = min((int)floorf(ahi), nt - 1);
+        const float tt = fmaf(dT, fn, T0);
+        const float za = fmaf(nue[0], tt, gam), zb = fmaf(nue[NE - 1], tt, gam);
+        if (ks > ke || fmaxf(za, zb) < -0.01f || fminf(za, zb) > fnz + 0.01f) continue;
+        const float wa = ahi - alo, tl = zero_tol * wa;
+        const float* __restrict__ slab = src + (size_t)n * nt * nzp;
+        float cz[NE];
+#pragma unroll
+        for (int e = 0; e < NE; ++e) cz[e] = __builtin_amdgcn_fmed3f(fmaf(nue[e], tt, gam), 0.0f, fnz);
+        // the z integrals of line `ln` up to every edge
+        struct Upto {
+            float v[NE];
+        };
+        auto upto = [&](int ln) {
+            Upto u;
+            if constexpr (ONE_Z) {
+                const float f = slab[(unsigned)(ln * nzp + 1)];
+#pragma unroll
+                for (int e = 0; e < NE; ++e) u.v[e] = cz[e] * f;
+            } else {
+#pragma unroll
+                for (int e = 0; e < NE; ++e) {
+                    const float fl = floorf(cz[e]);
+                    const PTaps p = *reinterpret_cast<const PTaps*>(slab + (unsigned)(ln * nzp + (int)fl));
+                    u.v[e] = fmaf(cz[e] - fl, p.b - p.a, p.a);
+                }
+            }
+            return u;
+        };
+        float sum[NE];
+        if (ke - ks <= 2) {
+            const float lo = fmaxf(alo, 0.0f), hi = fminf(ahi, fnt), s1 = (float)ks + 1.0f;
+            const float r = __builtin_amdgcn_rcpf(wa * tt);
+            const float o[3] = {fminf(hi, s1) - lo, fminf(hi, s1 + 1.0f) - s1, hi - (s1 + 1.0f)};
+            const float w0 = o[0] >= tl ? o[0] * r : 0.0f;
+            const Upto first = upto(ks);
+#pragma unroll
+            for (int e = 0; e < NE; ++e) sum[e] = w0 * first.v[e];
+#pragma unroll
+            for (int a = 1; a < 3; ++a) {
+                if (ks + a > ke || o[a] < tl) continue;
+                const float w = o[a] * r;
+                const Upto u = upto(ks + a);
+#pragma unroll
+                for (int e = 0; e < NE; ++e) sum[e] = fmaf(w, u.v[e], sum[e]);
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < NE; ++e) sum[e] = 0.0f;
+            for (int ka = ks; ka <= ke; ++ka) {
+                const float ov = fminf(ahi, (float)(ka + 1)) - fmaxf(alo, (float)ka);
+                if (ov < tl) continue;
+                const Upto u = upto(ka);
+#pragma unroll
+                for (int e = 0; e < NE; ++e) sum[e] = fmaf(ov, u.v[e], sum[e]);
+            }
+            const float r = __builtin_amdgcn_rcpf(wa * tt);
+#pragma unroll
+            for (int e = 0; e < NE; ++e) sum[e] *= r;
+        }
+#pragma unroll
+        for (int e = 0; e < NE; ++e) H[e] += (double)sum[e];
+    }
+#pragma unroll
+    for (int e = 0; e < NE; ++e) part[wave][e][lane] = H[e];
+    __syncthreads();
+    // wavefront k: row k
+    if (wave >= nv || col >= nu) return;
+    double h[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+        h[e] = (part[0][wave + e][lane] + part[1][wave + e][lane]) + (part[2][wave + e][lane] + part[3][wave + e][lane]);
+    const float s2 = rows[nv + 1 + wave] * T[5 * nu + 2 + j];
+    out[(size_t)wave * nu + col] =
+        (float)(h[1] - h[0]) * (T[4 * nu + 2 + j] * sqrtf(1.0f + s2 * s2) / (rows[wave + 1] - rows[wave]));
+}
+
 // z-slab views (|S_z - D_z| dominates the source-detector offset; no circular or helical orbit
 // reaches it): kernel semantics of distance_project_on_z3 (python/GPUFuncs_pycuda.py:526-587)
 // with the host tables of distance_forward (python/Reconstruction_pycuda.py:828-864, 993-1003).
@@ -2822,16 +2948,31 @@ int ctr_dd_forward(const ctr_geometry* g, const double* angles, const int32_t* b
     hipLaunchKernelGGL(zprefix_kernel, dim3((g->nx + 31) / 32, g->ny), dim3(256), 0, s, vol, t_ys, t_xs,
                        g->nx, g->ny, g->nz, nzp);
     if ((st = status_from_hip(hipGetLastError()))) return st;
-    const int col_groups = (g->nu + kFpCols * kFpWaves - 1) / (kFpCols * kFpWaves);
-    const int row_blocks = (g->nv + kColRows - 1) / kColRows;
-    const int n_pairs = (g->n_views + kFpViews - 1) / kFpViews;
-    const int n_vblocks = (n_pairs + kViewBlock - 1) / kViewBlock;
-    const long long n_blocks =
-        8LL * ((col_groups + 7) / 8) * row_blocks * n_vblocks * kViewBlock;
-    if (n_blocks >= 2147483647LL) return CTR_ERR_INVALID;
-    hipLaunchKernelGGL(dd_forward_kernel, dim3((unsigned)n_blocks), dim3(64 * kFpWaves), 0, s, t_ys, t_xs,
-                       proj, tabs, rows, branch, g->nx, g->ny, g->nz, nzp, g->nu, g->nv, stride, 1e-6f,
-                       g->n_views, col_groups, n_vblocks);
+    if (g->nv <= kThinRows) {
+        static_assert(kThinRows == 4, "one wavefront per row");
+        const dim3 grid((g->nu + 63) / 64, g->n_views);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, t_ys, t_xs, proj, tabs, rows, branch, g->nx, g->ny, g->nz,
+                               nzp, g->nu, g->nv, stride, 1e-6f);
+        };
+        if (g->nz == 1)
+            g->nv == 1 ? launch(dd_forward_thin_kernel<2, true>) : launch(dd_forward_thin_kernel<kThinRows + 1, true>);
+        else if (g->nv <= 2)
+            g->nv == 1 ? launch(dd_forward_thin_kernel<2, false>) : launch(dd_forward_thin_kernel<3, false>);
+        else
+            g->nv == 3 ? launch(dd_forward_thin_kernel<4, false>) : launch(dd_forward_thin_kernel<5, false>);
+    } else {
+        const int col_groups = (g->nu + kFpCols * kFpWaves - 1) / (kFpCols * kFpWaves);
+        const int row_blocks = (g->nv + kColRows - 1) / kColRows;
+        const int n_pairs = (g->n_views + kFpViews - 1) / kFpViews;
+        const int n_vblocks = (n_pairs + kViewBlock - 1) / kViewBlock;
+        const long long n_blocks =
+            8LL * ((col_groups + 7) / 8) * row_blocks * n_vblocks * kViewBlock;
+        if (n_blocks >= 2147483647LL) return CTR_ERR_INVALID;
+        hipLaunchKernelGGL(dd_forward_kernel, dim3((unsigned)n_blocks), dim3(64 * kFpWaves), 0, s, t_ys, t_xs,
+                           proj, tabs, rows, branch, g->nx, g->ny, g->nz, nzp, g->nu, g->nv, stride, 1e-6f,
+                           g->n_views, col_groups, n_vblocks);
+    }
     if ((st = status_from_hip(hipGetLastError()))) return st;
     // z-slab views (left at zero above): their own kernel, which returns at once for the others
     hipLaunchKernelGGL(dd_forward_zslab_kernel, dim3(kZslabGroups, g->n_views), dim3(256), 0, s, *g, angles,
