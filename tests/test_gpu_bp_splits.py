@@ -101,3 +101,21 @@ def test_ragged_and_straddling_sub_chunks_match_the_oracle(dev, nz, kind):
     base = dict(NumberOfImage=[19, 18, nz], NumberOfViews=5, NumberOfDetectorPixels=[26, 44], StartAngle=0.2,
                 EndAngle=0.2 + 2 * np.pi)
     _check(dev, make_params(**{**base, **kw}), "edge" if kind == "cut" else "ref")
+
+
+# a single slice has a kernel of its own: one and several detector rows, cells from a fifth of a
+# pixel to three pixels wide, slices off the source height, both grids, weight zeroing
+@pytest.mark.parametrize("nv,cell", [(1, 0.15), (1, 0.7), (3, 0.5), (7, 0.1), (2, 2.0)])
+@pytest.mark.parametrize("shape", ["Flat", "Curved"])
+@pytest.mark.parametrize("zc", [0.0, 0.3])
+def test_single_slice_matches_the_oracle(dev, nv, cell, shape, zc):
+    p = make_params(NumberOfImage=[21, 34, 1], ReconCenter=[0.2, -0.1, zc], NumberOfViews=23, StartAngle=0.1,
+                    EndAngle=0.1 + 2 * np.pi, NumberOfDetectorPixels=[int(24 / cell), nv],
+                    DetectorPixelSize=[cell, 0.6], DetectorShape=shape)
+    for mode in ("ref", "edge"):
+        _check(dev, p, mode)
+    g = O.Geometry(p)
+    q = np.random.default_rng(8).random((g.nview, g.nv, g.nu)).astype(np.float32)
+    ref = O.backproject(g, q, "ref", zero_tol=1e-5)
+    out = ctr.dd_backproject(torch.from_numpy(q).to(dev), ctr.ScanGeometry(p), zero_tol=1e-5).cpu().numpy()
+    assert np.abs(out - ref).max() <= TOL * np.abs(ref).max()
