@@ -12,11 +12,11 @@
 //                         channels: one workgroup per CU with all weights in LDS, walking pixel
 //                         tiles with the next tile's input halo loaded while the current one is
 //                         computed.
-//   conv3x3_wgrad_kernel  weight and bias gradients on MFMA: per (pixel chunk, tap), 64-pixel
-//                         tiles of the output gradient and of the shifted input staged in LDS
-//                         transposed to [channel][pixel]; grad_w = gout^T x_shift with K =
-//                         pixels, FP32 accumulation; partial sums per chunk
-//   conv3x3_wgrad_reduce  sums the chunk partials in a fixed order (deterministic)
+//   conv3x3_wgrad_kernel  weight and bias gradients on MFMA: 8 x 32 pixel tiles of the output
+//                         gradient and their input halos staged in LDS and read transposed;
+//                         grad_w = gout^T x_shift with K = pixels for all nine taps, FP32
+//                         accumulation; partial sums per workgroup
+//   conv3x3_wgrad_reduce  sums the partials in a fixed order (deterministic)
 
 #include <hip/hip_runtime.h>
 
@@ -482,37 +482,60 @@ __global__ void __launch_bounds__(kPThreads) conv3x3_fwd_persistent_kernel(
     }
 }
 
-constexpr int kWgTile = 64;     // pixels per LDS tile: two MFMA K steps of 32
-constexpr int kWgRow = 72;      // bf16 per LDS row (64 pixels + 8 of padding: conflict-free reads)
+// Weight and bias gradients on MFMA: grad_w[tap][co][ci] = sum_p gout[p][co] x[p + tap][ci], nine
+// 64 x 64 GEMMs with K = pixels that share their operands.  A 512-thread workgroup walks 8 x 32 pixel
+// tiles: the output gradient's tile and the input's (8+2) x (32+2) halo are staged in LDS as they lie
+// in memory ([pixel][channel], 16-byte stores) and the K-major operands come out of LDS transposed
+// (ds_read_b64_tr_b16: the 16 lanes of a group read four pixels x 16 channels and lane i receives
+// channel i of the four), so a tap is a pixel offset of the read and no transposed copy is written.
+// Wave (ci tile w % 4, co half w / 4) holds all nine taps of its 32 x 16 block: per K step (32 pixels
+// of a row) it reads two operands of gout and, since a halo row serves three output rows, three of x
+// for 18 MFMAs.  The next tile is loaded into registers meanwhile.  The bias gradient is one more
+// MFMA against ones.  16-channel blocks are XOR-ed with bits of the pixel's column, so that the eight
+// pixels of a half-wave's read fall in distinct banks for every tap.  Partial sums per workgroup are
+// added in a fixed order by conv3x3_wgrad_reduce.  With at most 16 input channels (SPLIT) there is one
+// ci tile, and the four waves of a co half share out the tile's rows instead; each keeps its sums
+// where the other ci tiles' would be.
+// Bound by the staging: a tile's 75 KB take longer to arrive and be stored than its MFMAs (a
+// workgroup per CU, 2.8 TB/s).  Measured at 16 x 128 x 128, 64 -> 64 channels: 28 us, 690 TFLOP/s
+// (118 us with one workgroup per (pixel chunk, tap) that wrote transposed copies of both operands to
+// LDS); at 103 x 54 x 140, 3 -> 64 channels 77 us (97 us without SPLIT, 450 us before).
+constexpr int kGTileH = 8, kGTileW = 32;
+constexpr int kGHaloW = kGTileW + 2, kGHaloPix = (kGTileH + 2) * kGHaloW;
+constexpr int kGThreads = 512;
+constexpr int kGGroups = 256;  // most workgroups: one per CU, and as many partial sums
+constexpr int kGYPer = kGTileH * kGTileW * 8 / kGThreads;              // 16-byte chunks of gout per thread
+constexpr int kGXPer = (kGHaloPix * 8 + kGThreads - 1) / kGThreads;    // and of the halo
 
-// Weight and bias gradients of one tap on MFMA: grad_w[co][ci] = sum_p gout[p][co] x[p + tap][ci],
-// a 64 x 64 GEMM with K = pixels.  The workgroup of (pixel chunk, tap) stages 64-pixel tiles of
-// the output gradient and of the tap-shifted input in LDS transposed to [channel][pixel] (bf16,
-// rows padded to 72 so that the 16 rows a 16-lane group reads fall in distinct banks); wave w
-// accumulates rows 16 w .. 16 w + 15 of grad_w against all 64 columns with
-// v_mfma_f32_16x16x32_bf16 (lane l gives row/column l % 16 with pixels 8 (l / 16) .. +7 of the
-// K step and receives rows 4 (l / 16) .. +3 of column l % 16), FP32 accumulation.  Partial
-// sums per chunk are reduced in a fixed order (deterministic).
-__global__ void __launch_bounds__(256) conv3x3_wgrad_kernel(
+// 16-channel block t of a pixel in tile column r sits in block t ^ gswz(r) of the pixel's row
+__device__ inline int gswz(int r) { return ((r >> 1) & 1) | ((r >> 2) & 2); }
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+// operand of 16 channels x 8 pixels per lane group: two transposed reads, pixels 0-3 and 4-7
+__device__ inline bf16x8 read_tr(const bf16_t* lo, const bf16_t* hi) {
+    typedef __attribute__((address_space(3))) s16x4 lds4;
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)lo);
+    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)hi);
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+template <bool SPLIT>
+__global__ void __launch_bounds__(kGThreads) conv3x3_wgrad_kernel(
     const bf16_t* __restrict__ in, const bf16_t* __restrict__ gout, float* __restrict__ part_w,
-    float* __restrict__ part_b, int N, int H, int W, int Cin, int Cout, int chunk_px) {
-    __shared__ __attribute__((aligned(16))) bf16_t ty[kMaxCout * kWgRow];  // gout^T  [co][p]
-    __shared__ __attribute__((aligned(16))) bf16_t tx[kMaxCout * kWgRow];  // shifted x^T [ci][p]
-    const int tap = blockIdx.y;
-    const int chunk = blockIdx.x;
-    const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-    const int P = N * H * W;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
+    float* __restrict__ part_b, int H, int W, int Cin, int Cout, int tiles_x, int tiles_y, int n_tiles) {
+    __shared__ __attribute__((aligned(16))) bf16_t ly[kGTileH * kGTileW * 64];
+    __shared__ __attribute__((aligned(16))) bf16_t lx[kGHaloPix * 64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int m = lane & 15, g = lane >> 4;
-    f32x4 acc[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float accb = 0.0f;
-    const int p_begin = chunk * chunk_px;
-    const int p_end = min(p_begin + chunk_px, P);
-    // staging: thread tid loads channels c8 .. c8+7 of the pixel pair (2 q, 2 q + 1) of the tile
-    const int q = tid >> 3, c8 = (tid & 7) * 8;
+    constexpr int kRows = SPLIT ? kGTileH / 4 : kGTileH;  // tile rows of a wave, from row0
+    const int slot = wave & 3, co_h = wave >> 2;
+    const int ci_t = SPLIT ? 0 : slot, row0 = SPLIT ? slot * kRows : 0;
+    const int n_ci = (Cin + 15) / 16, n_co = (Cout + 15) / 16;
+    // blocks that hold no channel are neither staged nor multiplied
+    const int co_tiles = ci_t < n_ci ? min(max(n_co - 2 * co_h, 0), 2) : 0;
     const bool vec_y = (Cout & 7) == 0, vec_x = (Cin & 7) == 0;
     auto load8 = [&](const bf16_t* base, int C, int c0, bool vec) {
         bf16x8 v = zero8();
@@ -525,84 +548,168 @@ __global__ void __launch_bounds__(256) conv3x3_wgrad_kernel(
         }
         return v;
     };
-    for (int p0 = p_begin; p0 < p_end; p0 += kWgTile) {
-        bf16x8 vy[2], vx[2];
+    bf16x8 py[kGYPer], px[kGXPer];
+    auto fetch = [&](int tile) {
+        const int tx0 = (tile % tiles_x) * kGTileW, ty0 = ((tile / tiles_x) % tiles_y) * kGTileH;
+        const size_t img = (size_t)(tile / (tiles_x * tiles_y)) * H * W;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int p = p0 + 2 * q + h;
-            vy[h] = zero8();
-            vx[h] = zero8();
-            if (p < p_end) {
-                vy[h] = load8(gout + (size_t)p * Cout, Cout, c8, vec_y);
-                const int x = p % W;
-                const int t = p / W;
-                const int y = t % H, n = t / H;
-                const int yy = y + dy, xx = x + dx;
-                if (yy >= 0 && yy < H && xx >= 0 && xx < W)
-                    vx[h] = load8(in + ((size_t)(n * H + yy) * W + xx) * Cin, Cin, c8, vec_x);
-            }
+        for (int p = 0; p < kGYPer; ++p) {
+            const int e = tid + p * kGThreads, c = e & 7, pix = e >> 3;
+            const int yy = ty0 + pix / kGTileW, xx = tx0 + pix % kGTileW;
+            py[p] = (c < 2 * n_co && yy < H && xx < W) ? load8(gout + (img + (size_t)yy * W + xx) * Cout, Cout, 8 * c, vec_y)
+                                                       : zero8();
         }
-        // transposed store: channel c8 + e, pixels 2 q and 2 q + 1 in one 32-bit word
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int row = (c8 + e) * kWgRow + 2 * q;
-            bf16_t py2[2] = {vy[0][e], vy[1][e]};
-            bf16_t px2[2] = {vx[0][e], vx[1][e]};
-            *reinterpret_cast<uint32_t*>(&ty[row]) = *reinterpret_cast<const uint32_t*>(py2);
-            *reinterpret_cast<uint32_t*>(&tx[row]) = *reinterpret_cast<const uint32_t*>(px2);
+        for (int p = 0; p < kGXPer; ++p) {
+            const int e = tid + p * kGThreads, c = e & 7, pix = e >> 3;
+            const int yy = ty0 + pix / kGHaloW - 1, xx = tx0 + pix % kGHaloW - 1;
+            px[p] = (pix < kGHaloPix && c < 2 * n_ci && (unsigned)yy < (unsigned)H && (unsigned)xx < (unsigned)W)
+                        ? load8(in + (img + (size_t)yy * W + xx) * Cin, Cin, 8 * c, vec_x)
+                        : zero8();
         }
+    };
+    auto store = [&]() {
+#pragma unroll
+        for (int p = 0; p < kGYPer; ++p) {
+            const int e = tid + p * kGThreads, c = e & 7, pix = e >> 3;
+            *reinterpret_cast<bf16x8*>(&ly[pix * 64 + (((c >> 1) ^ gswz(pix % kGTileW)) << 4) + (c & 1) * 8]) = py[p];
+        }
+#pragma unroll
+        for (int p = 0; p < kGXPer; ++p) {
+            const int e = tid + p * kGThreads, c = e & 7, pix = e >> 3;
+            if (pix < kGHaloPix)
+                *reinterpret_cast<bf16x8*>(&lx[pix * 64 + (((c >> 1) ^ gswz(pix % kGHaloW)) << 4) + (c & 1) * 8]) = px[p];
+        }
+    };
+    // this lane's addresses in a tile row: pixel 8 g + m / 4 (+ 4, + dx), channels 4 (m % 4) .. +3
+    int ay[2][2], ax[3][2];  // [co tile | dx][pixel half]
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int r = 8 * g + (m >> 2) + 4 * h;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) ay[t][h] = (row0 * kGTileW + r) * 64 + (((2 * co_h + t) ^ gswz(r)) << 4) + (m & 3) * 4;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) ax[d][h] = (row0 * kGHaloW + r + d) * 64 + ((ci_t ^ gswz(r + d)) << 4) + (m & 3) * 4;
+    }
+    f32x4 acc[9][2], accb[2];
+#pragma unroll
+    for (int k = 0; k < 9; ++k)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[k][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int t = 0; t < 2; ++t) accb[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    bf16x8 ones;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ones[e] = (bf16_t)1.0f;
+
+    int tile = blockIdx.x;
+    fetch(tile);
+    while (tile < n_tiles) {
+        __syncthreads();  // every wave has read the previous tile
+        store();
         __syncthreads();
+        tile += gridDim.x;
+        if (tile < n_tiles) fetch(tile);
+        if (co_tiles) {
+            bf16x8 b[3][3];  // [halo row % 3][dx]
 #pragma unroll
-        for (int ks = 0; ks < kWgTile / 32; ++ks) {
-            const int pk = ks * 32 + 8 * g;
-            const bf16x8 a = *reinterpret_cast<const bf16x8*>(&ty[(16 * wave + m) * kWgRow + pk]);
+            for (int y = 0; y < 2; ++y)
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const bf16x8 bb = *reinterpret_cast<const bf16x8*>(&tx[(16 * t + m) * kWgRow + pk]);
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bb, acc[t], 0, 0, 0);
+                for (int d = 0; d < 3; ++d)
+                    b[y][d] = read_tr(&lx[y * kGHaloW * 64 + ax[d][0]], &lx[y * kGHaloW * 64 + ax[d][1]]);
+#pragma unroll
+            for (int y = 0; y < kRows; ++y) {
+                bf16x8 a[2];
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+                    a[t] = read_tr(&ly[y * kGTileW * 64 + ay[t][0]], &ly[y * kGTileW * 64 + ay[t][1]]);
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+                    b[(y + 2) % 3][d] =
+                        read_tr(&lx[(y + 2) * kGHaloW * 64 + ax[d][0]], &lx[(y + 2) * kGHaloW * 64 + ax[d][1]]);
+#pragma unroll
+                for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+                    for (int d = 0; d < 3; ++d)
+#pragma unroll
+                        for (int t = 0; t < 2; ++t)
+                            acc[3 * dy + d][t] =
+                                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b[(y + dy) % 3][d], acc[3 * dy + d][t], 0, 0, 0);
+                if (ci_t == 0)
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) accb[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], ones, accb[t], 0, 0, 0);
             }
         }
-        if (tap == 0 && tid < kMaxCout) {
+    }
+    // lane (m, g) holds rows (co) 4 g .. 4 g + 3 of column (ci) m of each 16 x 16 block
+    float* pw = part_w + (size_t)blockIdx.x * 9 * kMaxCout * kMaxCout;
+#pragma unroll
+    for (int k = 0; k < 9; ++k)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (t < co_tiles)
+                    pw[(k * kMaxCout + 32 * co_h + 16 * t + 4 * g + r) * kMaxCout + 16 * slot + m] = acc[k][t][r];
+    if (ci_t == 0 && m == 0)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                part_b[((size_t)blockIdx.x * 4 + slot) * kMaxCout + 32 * co_h + 16 * t + 4 * g + r] = accb[t][r];
+}
+
+// grad_w[co][tap][ci] = sum over the workgroups' partial sums (fixed order); grad_b[co] likewise.
+// One workgroup per (co, tap) row and a quarter of the partial sums per wave, so that the reads of a
+// partial sum's row are one 256-byte run; with slots = 4 that row holds the sums of the four row
+// shares, 16 channels each.  7 us for 256 partial sums at 64 -> 64 channels (60 us for 128 with a
+// thread per output and the partial sums one after the other).
+__global__ void __launch_bounds__(256) conv3x3_wgrad_reduce(const float* __restrict__ part_w, const float* __restrict__ part_b,
+                                                            float* __restrict__ grad_w, float* __restrict__ grad_b, int n_parts,
+                                                            int Cin, int Cout, int slots) {
+    __shared__ float sums[4][64];
+    const int ci = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int row = blockIdx.x;  // co * 9 + tap, and Cout * 9 for the bias
+    const bool bias = row == Cout * 9;
+    const int co = row / 9, tap = row - 9 * co;
+    const float* src = bias ? part_b + ci : part_w + ((size_t)tap * kMaxCout + co) * kMaxCout + ci;
+    const size_t step = bias ? 4 * kMaxCout : 9 * kMaxCout * kMaxCout;
+    const int n = bias ? Cout : Cin;
+    const int per = (n_parts + 3) / 4, c1 = min((w + 1) * per, n_parts);
+    float s = 0.0f;
+    if (ci < n || (!bias && slots > 1)) {
 #pragma unroll 8
-            for (int p = 0; p < kWgTile; ++p) accb += (float)ty[tid * kWgRow + p];
-        }
-        __syncthreads();
+        for (int c = w * per; c < c1; ++c) s += src[(size_t)c * step];
+        for (int k = 1; bias && k < slots; ++k)
+            for (int c = w * per; c < c1; ++c) s += src[(size_t)c * step + k * kMaxCout];
     }
-    float* pw = part_w + ((size_t)chunk * 9 + tap) * kMaxCout * kMaxCout;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) pw[(16 * wave + 4 * g + r) * kMaxCout + 16 * t + m] = acc[t][r];
-    if (tap == 0 && tid < kMaxCout) part_b[(size_t)chunk * kMaxCout + tid] = accb;
+    sums[w][ci] = s;
+    __syncthreads();
+    if (w || ci >= n) return;
+    float total = (sums[0][ci] + sums[1][ci]) + (sums[2][ci] + sums[3][ci]);
+    for (int k = 1; !bias && k < slots; ++k)
+        total += (sums[0][16 * k + ci] + sums[1][16 * k + ci]) + (sums[2][16 * k + ci] + sums[3][16 * k + ci]);
+    if (bias)
+        grad_b[ci] = total;
+    else
+        grad_w[(size_t)row * Cin + ci] = total;
 }
 
-// grad_w[co][tap][ci] = sum over chunks (fixed order); grad_b[co] likewise
-__global__ void conv3x3_wgrad_reduce(const float* __restrict__ part_w, const float* __restrict__ part_b,
-                                     float* __restrict__ grad_w, float* __restrict__ grad_b,
-                                     int n_chunks, int Cin, int Cout) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    const int total = Cout * 9 * Cin;
-    if (idx < total) {
-        const int ci = idx % Cin;
-        const int tap = (idx / Cin) % 9;
-        const int co = idx / (9 * Cin);
-        float s = 0.0f;
-        for (int c = 0; c < n_chunks; ++c)
-            s += part_w[(((size_t)c * 9 + tap) * kMaxCout + co) * kMaxCout + ci];
-        grad_w[idx] = s;
-    }
-    if (grad_b && idx < Cout) {
-        float s = 0.0f;
-        for (int c = 0; c < n_chunks; ++c) s += part_b[(size_t)c * kMaxCout + idx];
-        grad_b[idx] = s;
-    }
-}
+// tiles and workgroups of a weight gradient: as many tiles for each workgroup, at most one per CU
+struct WgradGrid {
+    int tiles_x, tiles_y;
+    long long tiles;
+    int groups;
+};
 
-int conv_chunks(long long P) {
-    long long c = (P + 2047) / 2048;
-    if (c > 512) c = 512;
-    if (c < 1) c = 1;
-    return (int)c;
+WgradGrid wgrad_grid(int n, int h, int w) {
+    WgradGrid r;
+    r.tiles_x = (w + kGTileW - 1) / kGTileW;
+    r.tiles_y = (h + kGTileH - 1) / kGTileH;
+    r.tiles = (long long)n * r.tiles_x * r.tiles_y;
+    const long long each = (r.tiles + kGGroups - 1) / kGGroups;
+    r.groups = (int)((r.tiles + each - 1) / each);
+    return r;
 }
 
 }  // namespace
@@ -669,8 +776,7 @@ size_t ctr_conv3x3_bf16_wgrad_workspace_bytes(int n, int h, int w, int cin, int 
     (void)cin;
     (void)cout;
     if (n <= 0 || h <= 0 || w <= 0) return 0;
-    const int chunks = conv_chunks((long long)n * h * w);
-    return (size_t)chunks * (9 * kMaxCout * kMaxCout + kMaxCout) * sizeof(float);
+    return (size_t)wgrad_grid(n, h, w).groups * (9 * kMaxCout * kMaxCout + 4 * kMaxCout) * sizeof(float);
 }
 
 int ctr_conv3x3_bf16_wgrad(const void* in, const void* grad_out, float* grad_weight, float* grad_bias,
@@ -682,17 +788,20 @@ int ctr_conv3x3_bf16_wgrad(const void* in, const void* grad_out, float* grad_wei
     const long long P = (long long)n * h * w;
     if (P * kMaxCout >= 2147483647LL) return CTR_ERR_INVALID;
     if (workspace_bytes < ctr_conv3x3_bf16_wgrad_workspace_bytes(n, h, w, cin, cout)) return CTR_ERR_WORKSPACE;
-    const int chunks = conv_chunks(P);
-    const int chunk_px = (int)(((P + chunks - 1) / chunks + kWgTile - 1) / kWgTile * kWgTile);
+    const WgradGrid wg = wgrad_grid(n, h, w);
+    if (wg.tiles >= 2147483647LL - kGGroups) return CTR_ERR_INVALID;
     float* part_w = (float*)workspace;
-    float* part_b = part_w + (size_t)chunks * 9 * kMaxCout * kMaxCout;
+    float* part_b = part_w + (size_t)wg.groups * 9 * kMaxCout * kMaxCout;
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(conv3x3_wgrad_kernel, dim3(chunks, 9), dim3(256), 0, s, (const bf16_t*)in,
-                       (const bf16_t*)grad_out, part_w, part_b, n, h, w, cin, cout, chunk_px);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(wg.groups), dim3(kGThreads), 0, s, (const bf16_t*)in, (const bf16_t*)grad_out,
+                           part_w, part_b, h, w, cin, cout, wg.tiles_x, wg.tiles_y, (int)wg.tiles);
+    };
+    const bool split = cin <= 16;
+    split ? launch(conv3x3_wgrad_kernel<true>) : launch(conv3x3_wgrad_kernel<false>);
     if (hipGetLastError() != hipSuccess) return CTR_ERR_HIP;
-    const int total = cout * 9 * cin;
-    hipLaunchKernelGGL(conv3x3_wgrad_reduce, dim3((total + 255) / 256), dim3(256), 0, s, part_w, part_b,
-                       grad_weight, grad_bias, chunks, cin, cout);
+    hipLaunchKernelGGL(conv3x3_wgrad_reduce, dim3(cout * 9 + (grad_bias ? 1 : 0)), dim3(256), 0, s, part_w, part_b,
+                       grad_weight, grad_bias, wg.groups, cin, cout, split ? 4 : 1);
     return hipGetLastError() == hipSuccess ? CTR_OK : CTR_ERR_HIP;
 }
 
