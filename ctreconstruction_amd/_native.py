@@ -32,6 +32,7 @@ EXPORTS = (
     "ctr_pixel_filter_spectrum", "ctr_pixel_filter",
     "ctr_pixel_backproject_workspace_bytes", "ctr_pixel_backproject",
     "ctr_conv3x3_bf16_forward", "ctr_conv3x3_bf16_wgrad_workspace_bytes", "ctr_conv3x3_bf16_wgrad",
+    "ctr_conv3x3_bf16_backward_workspace_bytes", "ctr_conv3x3_bf16_backward",
 )
 
 CTR_OK = 0
@@ -132,6 +133,9 @@ def _declare(lib):
         "ctr_conv3x3_bf16_wgrad_workspace_bytes": (c_size, [c_int, c_int, c_int, c_int, c_int]),
         "ctr_conv3x3_bf16_wgrad": (c_int, [c_vp, c_vp, c_vp, c_vp, c_int, c_int, c_int, c_int, c_int,
                                            c_vp, c_size, c_vp]),
+        "ctr_conv3x3_bf16_backward_workspace_bytes": (c_size, [c_int, c_int, c_int, c_int, c_int]),
+        "ctr_conv3x3_bf16_backward": (c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_int, c_int, c_int, c_int,
+                                              c_int, c_vp, c_size, c_vp]),
     }
     for name, (res, args) in sig.items():
         fn = getattr(lib, name)

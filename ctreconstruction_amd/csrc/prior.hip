@@ -17,6 +17,7 @@
 //                         grad_w = gout^T x_shift with K = pixels for all nine taps, FP32
 //                         accumulation; partial sums per workgroup
 //   conv3x3_wgrad_reduce  sums the partials in a fixed order (deterministic)
+//   conv3x3_flip_kernel   weights of the input-gradient convolution
 
 #include <hip/hip_runtime.h>
 
@@ -681,6 +682,7 @@ __global__ void __launch_bounds__(256) conv3x3_wgrad_reduce(const float* __restr
 #pragma unroll 8
         for (int c = w * per; c < c1; ++c) s += src[(size_t)c * step];
         for (int k = 1; bias && k < slots; ++k)
+#pragma unroll 8
             for (int c = w * per; c < c1; ++c) s += src[(size_t)c * step + k * kMaxCout];
     }
     sums[w][ci] = s;
@@ -693,6 +695,15 @@ __global__ void __launch_bounds__(256) conv3x3_wgrad_reduce(const float* __restr
         grad_b[ci] = total;
     else
         grad_w[(size_t)row * Cin + ci] = total;
+}
+
+// Weights of the input-gradient convolution: out[ci][2 - ky][2 - kx][co] = w[co][ky][kx][ci]
+__global__ void __launch_bounds__(256) conv3x3_flip_kernel(const bf16_t* __restrict__ w, bf16_t* __restrict__ out, int Cin,
+                                                           int Cout) {
+    const int i = blockIdx.x * 256 + threadIdx.x;  // index into out
+    if (i >= Cin * 9 * Cout) return;
+    const int co = i % Cout, tap = (i / Cout) % 9, ci = i / (9 * Cout);
+    out[i] = w[(co * 9 + 8 - tap) * Cin + ci];
 }
 
 // tiles and workgroups of a weight gradient: as many tiles for each workgroup, at most one per CU
@@ -803,6 +814,34 @@ int ctr_conv3x3_bf16_wgrad(const void* in, const void* grad_out, float* grad_wei
     hipLaunchKernelGGL(conv3x3_wgrad_reduce, dim3(cout * 9 + (grad_bias ? 1 : 0)), dim3(256), 0, s, part_w, part_b,
                        grad_weight, grad_bias, wg.groups, cin, cout, split ? 4 : 1);
     return hipGetLastError() == hipSuccess ? CTR_OK : CTR_ERR_HIP;
+}
+
+// flipped weights of the input-gradient convolution, then the weight gradient's workspace
+static size_t flipped_bytes(int cin, int cout) { return ((size_t)cin * 9 * cout * sizeof(bf16_t) + 255) / 256 * 256; }
+
+size_t ctr_conv3x3_bf16_backward_workspace_bytes(int n, int h, int w, int cin, int cout) {
+    if (n <= 0 || h <= 0 || w <= 0 || cin <= 0 || cout <= 0 || cin > kMaxCout || cout > kMaxCout) return 0;
+    return flipped_bytes(cin, cout) + ctr_conv3x3_bf16_wgrad_workspace_bytes(n, h, w, cin, cout);
+}
+
+int ctr_conv3x3_bf16_backward(const void* in, const void* weight, const void* grad_out, void* grad_in, float* grad_weight,
+                              float* grad_bias, int n, int h, int w, int cin, int cout, void* workspace,
+                              size_t workspace_bytes, void* stream) {
+    if (!in || !grad_out || !grad_weight || !workspace || (grad_in && !weight)) return CTR_ERR_INVALID;
+    if (n <= 0 || h <= 0 || w <= 0 || cin <= 0 || cout <= 0 || cin > kMaxCout || cout > kMaxCout) return CTR_ERR_INVALID;
+    if ((long long)n * h * w * kMaxCout >= 2147483647LL) return CTR_ERR_INVALID;
+    if (workspace_bytes < ctr_conv3x3_bf16_backward_workspace_bytes(n, h, w, cin, cout)) return CTR_ERR_WORKSPACE;
+    const size_t flipped = flipped_bytes(cin, cout);
+    if (grad_in) {
+        bf16_t* wf = (bf16_t*)workspace;
+        hipLaunchKernelGGL(conv3x3_flip_kernel, dim3((cin * 9 * cout + 255) / 256), dim3(256), 0, (hipStream_t)stream,
+                           (const bf16_t*)weight, wf, cin, cout);
+        if (hipGetLastError() != hipSuccess) return CTR_ERR_HIP;
+        const int st = ctr_conv3x3_bf16_forward(grad_out, wf, nullptr, nullptr, grad_in, n, h, w, cout, cin, 0, stream);
+        if (st != CTR_OK) return st;
+    }
+    return ctr_conv3x3_bf16_wgrad(in, grad_out, grad_weight, grad_bias, n, h, w, cin, cout, (char*)workspace + flipped,
+                                  workspace_bytes - flipped, stream);
 }
 
 }  // extern "C"

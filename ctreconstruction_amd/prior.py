@@ -73,6 +73,22 @@ def flip_transpose(w_bf16: torch.Tensor) -> torch.Tensor:
     return torch.flip(w_bf16, dims=(1, 2)).permute(3, 1, 2, 0).contiguous()
 
 
+def conv3x3_backward(x: torch.Tensor, w_bf16: torch.Tensor, gout: torch.Tensor, input_grad: bool = True):
+    """(grad_x bfloat16 or None, grad_weight, grad_bias): the input gradient (the convolution of the
+    output gradient with :func:`flip_transpose`-d weights) and :func:`conv3x3_wgrad` in one call."""
+    n, h, w, cin = x.shape
+    cout = gout.shape[-1]
+    lib, dev = N.lib(), x.device
+    gx = torch.empty_like(x) if input_grad else None
+    gw = torch.empty((cout, 3, 3, cin), dtype=torch.float32, device=dev)
+    gb = torch.empty(cout, dtype=torch.float32, device=dev)
+    nbytes = lib.ctr_conv3x3_bf16_backward_workspace_bytes(n, h, w, cin, cout)
+    ws = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=dev)
+    N.check(lib.ctr_conv3x3_bf16_backward(_ptr(x), _ptr(w_bf16), _ptr(gout), _ptr(gx), _ptr(gw), _ptr(gb), n, h, w, cin,
+                                          cout, _ptr(ws), nbytes, _stream(dev)), "ctr_conv3x3_bf16_backward")
+    return gx, gw, gb
+
+
 class Conv3x3Function(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias, need_input_grad):
@@ -85,9 +101,7 @@ class Conv3x3Function(torch.autograd.Function):
     def backward(ctx, gout):
         x, wb = ctx.saved_tensors
         gout = gout.to(BF16).contiguous()
-        gx = conv3x3_forward(gout, flip_transpose(wb)) if ctx.need_input_grad else None
-        gw, gb = conv3x3_wgrad(x, gout)
-        return gx, gw, gb, None
+        return (*conv3x3_backward(x, wb, gout, ctx.need_input_grad), None)
 
 
 class ResidualPrior(torch.nn.Module):

@@ -197,7 +197,9 @@ int ctr_pixel_backproject(const ctr_geometry* g, const double* angles, const flo
  * The input gradient is ctr_conv3x3_bf16_forward applied to the output gradient with the
  * weights flipped in space and transposed in channels.
  * ctr_conv3x3_bf16_wgrad: grad_weight[cout][3][3][cin] (float32) and grad_bias[cout] (may be
- * NULL) summed over all pixels, in a fixed order; cin, cout <= 64. */
+ * NULL) summed over all pixels, in a fixed order; cin, cout <= 64.
+ * ctr_conv3x3_bf16_backward: both gradients in one call; grad_in may be NULL (not wanted), and so
+ * may then `weight`. */
 int ctr_conv3x3_bf16_forward(const void* in, const void* weight, const float* bias,
                              const void* residual, void* out, int n, int h, int w, int cin,
                              int cout, int relu, void* stream);
@@ -205,6 +207,11 @@ size_t ctr_conv3x3_bf16_wgrad_workspace_bytes(int n, int h, int w, int cin, int 
 int ctr_conv3x3_bf16_wgrad(const void* in, const void* grad_out, float* grad_weight,
                            float* grad_bias, int n, int h, int w, int cin, int cout,
                            void* workspace, size_t workspace_bytes, void* stream);
+
+size_t ctr_conv3x3_bf16_backward_workspace_bytes(int n, int h, int w, int cin, int cout);
+int ctr_conv3x3_bf16_backward(const void* in, const void* weight, const void* grad_out, void* grad_in,
+                              float* grad_weight, float* grad_bias, int n, int h, int w, int cin, int cout,
+                              void* workspace, size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

@@ -38,3 +38,21 @@ def test_weight_gradient_tiles_match_float64(n, h, w, cin, cout):
     assert (gb.cpu().double() - rb).abs().max() <= 1e-5 * rb.abs().max().clamp_min(1.0)
     gw2, none = PR.conv3x3_wgrad(x.cuda(), g.cuda(), with_bias=False)
     assert none is None and torch.equal(gw2, gw)
+
+
+@pytest.mark.parametrize("cin,cout", [(64, 64), (3, 64), (64, 1), (17, 33)])
+def test_combined_backward_equals_its_parts(cin, cout):
+    """The same kernels on the same operands: bit-identical; the input gradient may be left out."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    N.lib()
+    gen = torch.Generator().manual_seed(cin)
+    x = torch.randn((2, 19, 37, cin), generator=gen).to(torch.bfloat16).cuda()
+    g = torch.randn((2, 19, 37, cout), generator=gen).to(torch.bfloat16).cuda()
+    w = torch.randn((cout, 3, 3, cin), generator=gen).to(torch.bfloat16).cuda()
+    gx, gw, gb = PR.conv3x3_backward(x, w, g)
+    assert torch.equal(gx, PR.conv3x3_forward(g, PR.flip_transpose(w)))
+    rw, rb = PR.conv3x3_wgrad(x, g)
+    assert torch.equal(gw, rw) and torch.equal(gb, rb)
+    none, gw, gb = PR.conv3x3_backward(x, w, g, input_grad=False)
+    assert none is None and torch.equal(gw, rw) and torch.equal(gb, rb)
