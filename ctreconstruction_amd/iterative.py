@@ -17,10 +17,12 @@ All functions accept one volume [nz, ny, nx] (projections [nView, nv, nu]) or a 
 """
 from __future__ import annotations
 
+import ctypes
 import weakref
 
 import torch
 
+from . import _native as N
 from . import projector as P
 from .autograd import DDProjectorFunction, adjoint_batch, forward_batch
 from .geometry import ScanGeometry
@@ -139,9 +141,52 @@ def _normalise_pad(dtv: torch.Tensor, eps: float) -> torch.Tensor:
     return torch.nn.functional.pad(dtv / norm, (1, 1, 1, 1, 1, 1))
 
 
+def _on_tv_kernels(img: torch.Tensor, eps: float) -> bool:
+    """Whether the TV kernels take ``img``: plain contiguous float32 volumes on the GPU that nothing
+    differentiates, maps or traces (the torch expressions serve everything else)."""
+    if type(img) is not torch.Tensor or img.device.type != "cuda" or img.dtype != torch.float32:
+        return False
+    if img.dim() < 3 or min(img.shape[-3:]) < 3 or not img.is_contiguous() or img.numel() == 0 or not eps > 0:
+        return False
+    if img.shape[-3:].numel() >= 2 ** 31 - 1 or img.shape[:-3].numel() > 65535:
+        return False
+    if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or torch.overrides._get_current_function_mode_stack() \
+            or torch.utils._python_dispatch._get_current_dispatch_mode() is not None:
+        return False
+    if torch._C._functorch.is_functorch_wrapped_tensor(img) or torch._C._is_fwd_grad_enabled() and \
+            torch.autograd.forward_ad.unpack_dual(img).tangent is not None:
+        return False
+    return not (torch.is_grad_enabled() and img.requires_grad)
+
+
+def _tv_call(fn, img, out, eps, steps, *args):
+    lib = N.lib()
+    nz, ny, nx = img.shape[-3:]
+    batch = img.shape[:-3].numel()
+    nbytes = lib.ctr_tv_workspace_bytes(batch, nx, ny, nz, steps)
+    ws = P._workspace(nbytes, img.device)
+    ptrs = [P._ptr(t) for t in args]
+    tail = (steps,) if ptrs else ()
+    N.check(getattr(lib, fn)(P._ptr(img), P._ptr(out), *ptrs, batch, nx, ny, nz, float(eps), *tail, P._ptr(ws), nbytes,
+                             P._stream(img.device)), fn)
+    return out
+
+
 def tv_gradient(img: torch.Tensor, eps: float = 1e-7) -> torch.Tensor:
     """Normalised TV gradient with zero border (python/ASD_POCS.py:55-77)."""
+    if _on_tv_kernels(img, eps):
+        return _tv_call("ctr_tv_gradient", img, torch.empty_like(img), eps, 1)
     return _normalise_pad(_tv_terms(img, eps), eps)
+
+
+def _tv_descent(x: torch.Tensor, step: torch.Tensor, n_steps: int, eps: float) -> torch.Tensor:
+    """``n_steps`` of x <- x - step * tv_gradient(x, eps), one ``step`` per volume."""
+    if n_steps > 0 and _on_tv_kernels(x, eps) and step.dtype == torch.float32 and not step.requires_grad:
+        flat = step.reshape(-1).expand(x.shape[:-3].numel()).contiguous()
+        return _tv_call("ctr_tv_descent", x, torch.empty_like(x), eps, n_steps, flat)
+    for _ in range(n_steps):
+        x = x - step * tv_gradient(x, eps)
+    return x
 
 
 def tv_gradient_autograd(img: torch.Tensor, eps: float = 1e-7) -> torch.Tensor:
@@ -169,7 +214,6 @@ def asd_pocs(proj0: torch.Tensor, geom: ScanGeometry, n_outer: int = 20, na: int
     geom.check_supported()
     a1, b1 = normalisers(geom, "matched" if backprojector == "matched" else "ref", proj0.device, eps)
     bp = (lambda r: adjoint_batch(r, geom)) if backprojector == "matched" else (lambda r: _bp_ref(r, geom))
-    tvg = tv_gradient_autograd if tv == "autograd" else tv_gradient
     if x0 is None:
         # the reference starts from the FDK reconstruction (python/ASD_POCS.py:142-143)
         x = (torch.stack([P.fdk(p.contiguous(), geom) for p in proj0]) if proj0.dim() == 4
@@ -191,8 +235,11 @@ def asd_pocs(proj0: torch.Tensor, geom: ScanGeometry, n_outer: int = 20, na: int
         dp = dist(x, f0)
         dtvg = alpha * dp
         f0 = x.clone()
-        for _ in range(ng):
-            x = x - dtvg * tvg(x, eps)
+        if tv == "autograd":
+            for _ in range(ng):
+                x = x - dtvg * tv_gradient_autograd(x, eps)
+        else:
+            x = _tv_descent(x, dtvg, ng, eps)
         dg = dist(x, f0)
         alpha = torch.where(dg > r_max * dp, alpha * alpha_red, alpha)
         beta *= beta_red

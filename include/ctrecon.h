@@ -189,6 +189,18 @@ int ctr_pixel_backproject(const ctr_geometry* g, const double* angles, const flo
                           float* vol, float scale, int accumulate, void* workspace,
                           size_t workspace_bytes, void* stream);
 
+/* ---- Total-variation steps of ASD-POCS ----------------------------------------------------
+ * Replace the TV gradient and descent of python/ASD_POCS.py:55-77 and 188-192 on a batch of
+ * independent volumes float32 [batch][nz][ny][nx], every axis >= 3 voxels, eps > 0.
+ * ctr_tv_gradient: grad = g / ||g||_2 (g itself where the norm is below eps), 0 on the border.
+ * ctr_tv_descent: out = x after `steps` steps x <- x - step[b] * g / ||g||_2; `step` is float32
+ * device memory, `batch` entries.  Outputs must not overlap `x`. */
+size_t ctr_tv_workspace_bytes(int batch, int nx, int ny, int nz, int steps);
+int ctr_tv_gradient(const float* x, float* grad, int batch, int nx, int ny, int nz, float eps,
+                    void* workspace, size_t workspace_bytes, void* stream);
+int ctr_tv_descent(const float* x, float* out, const float* step, int batch, int nx, int ny, int nz,
+                   float eps, int steps, void* workspace, size_t workspace_bytes, void* stream);
+
 /* ---- Learned prior: 3x3 convolutions, bfloat16 on MFMA, FP32 accumulation ---------------
  * No counterpart in the reference (the reference has no learned prior).
  * Activations are NHWC bfloat16 [n][h][w][c]; weights bfloat16 [cout][3][3][cin]; bias float32.
