@@ -7,7 +7,7 @@
 //   dd_forward_zslab_kernel     z-slab views (non-circular geometries), FP64 loops per cell
 //   bp_geometry_kernel          per-view backprojection constants, FP64 -> FP32
 //   dd_backproject_tile_kernel  one workgroup per 16 x 16 x ZC voxel tile and view split, windows in LDS
-//   bp_reduce_kernel            sums the view splits' partial volumes in a fixed order
+//   sum_parts_kernel            sums the view splits' partial volumes in a fixed order (splits.h)
 //   adj_geometry_kernel         per-view constants of the inverse central projection
 //   adj_rowprefix_kernel        row prefix sums of projections times path length
 //   adj_tile_kernel             detector windows of every (view, column tile)
@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "ctrecon.h"
+#include "splits.h"
 
 namespace {
 
@@ -1555,7 +1556,7 @@ __device__ inline void bp_column_view(const BpView& v, const float* __restrict__
 // part or whole) to kBpRest, which adds those contributions; kBpAll does everything.
 // blockIdx.y is the view split: split s takes the views [s * views_per, (s + 1) * views_per) of
 // its tile and, where there is more than one, writes its sums to its own copy of the volume in
-// `parts`, which bp_reduce_kernel adds up in split order (see bp_split).
+// `parts`, which sum_parts_kernel adds up in split order (see bp_split).
 // GENERAL: the fast pass takes every sub-chunk that fits (bp_column_view_fast).
 template <int ZC, int KIND, typename S, bool GENERAL>
 __global__ void __launch_bounds__(256) dd_backproject_tile_kernel(
@@ -1797,20 +1798,6 @@ __global__ void __launch_bounds__(256) bp_slice_kernel(
     }
     const size_t idx = (size_t)iy * nx + ix;
     vol[idx] = accumulate ? vol[idx] + acc : acc;
-}
-
-// vol = (accumulate ? vol : 0) + the splits' partial volumes, in split order (deterministic).
-// One 16-byte load per split and thread where the volume's size and address allow it (W = 4).
-template <int W>
-__global__ void __launch_bounds__(256) bp_reduce_kernel(const float* __restrict__ parts, float* __restrict__ vol,
-                                                        size_t n, int splits, int accumulate) {
-    typedef float vec __attribute__((ext_vector_type(W)));
-    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * W;
-    if (i >= n) return;
-    vec sum = *reinterpret_cast<const vec*>(parts + i);
-    for (int s = 1; s < splits; ++s) sum += *reinterpret_cast<const vec*>(parts + (size_t)s * n + i);
-    vec* out = reinterpret_cast<vec*>(vol + i);
-    *out = accumulate ? *out + sum : sum;
 }
 
 __global__ void __launch_bounds__(256) fill_zero_kernel(uint32_t* __restrict__ p, size_t n) {
@@ -2065,7 +2052,7 @@ __device__ inline void adj_chunk(int iz0, float gam, float off, float de, float 
 }
 
 // vol = (accumulate ? vol : 0) + scale * A^T y of the split's views (blockIdx.y), or that into the
-// split's volume in `parts` (added up by bp_reduce_kernel).
+// split's volume in `parts` (added up by sum_parts_kernel).
 template <typename S>
 __global__ void __launch_bounds__(256) dd_adjoint_kernel(
     const float* __restrict__ Y, float* __restrict__ vol, float* __restrict__ parts, const float* __restrict__ tabs,
@@ -2284,22 +2271,38 @@ int log2_exact(int n) {
 // The cosine table lives in LDS; arguments are reduced exactly as (f*n mod N).
 // ConeBeam.Filter (python/ConeBeamGPU.py:355-384) is the same series times gain = 2 with the
 // mask |w| > mask_w = pi*cutoff; Reconstruction.Filter has gain 1, mask_w = pi*cutoff/(2 tau).
+// 64 frequencies per workgroup, a quarter of the series per wavefront; the taps, which cost an FP64
+// division each, are worked out once per workgroup, 256 at a time.  Bound by the cosine table
+// (N cosines per workgroup): 16 us at N = 2048, 83 us with 256 frequencies per workgroup, each thread
+// dividing for every tap and reducing its argument with a 64-bit remainder.
+constexpr int kSpecFreqs = 64;
+
 __global__ void __launch_bounds__(256) spectrum_kernel(double* __restrict__ out, int N,
                                                        double tau, int ftype, double cutoff,
                                                        double gain, double mask_w) {
     extern __shared__ double costab[];
+    __shared__ double taps[256], sums[4][kSpecFreqs];
     for (int m = threadIdx.x; m < N; m += blockDim.x) costab[m] = cos(2.0 * kPi * m / N);
-    __syncthreads();
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= N) return;
+    const int f = blockIdx.x * kSpecFreqs + (threadIdx.x & (kSpecFreqs - 1)), part = threadIdx.x / kSpecFreqs;
     const int fs = (f < N / 2) ? f : f - N;  // signed frequency; f = N/2 is -N/2 as fftshift has it
     const double h0 = 1.0 / (8.0 * tau * tau);
     double acc = 0.0;
-    const int fm = ((fs % N) + N) % N;
-    for (int n = 1; n < N / 2; n += 2) {
-        const double hn = -0.5 / ((kPi * tau * n) * (kPi * tau * n));
-        acc += hn * costab[(int)(((long long)fm * n) % N)];
+    const unsigned fm = (unsigned)fs & (unsigned)(N - 1);  // N is a power of two
+    for (int n0 = 1; n0 < N / 2; n0 += 512) {  // the odd taps n0, n0 + 2, ..., n0 + 510
+        __syncthreads();
+        const int nt = n0 + 2 * (int)threadIdx.x;
+        taps[threadIdx.x] = nt < N / 2 ? -0.5 / ((kPi * tau * nt) * (kPi * tau * nt)) : 0.0;
+        __syncthreads();
+        for (int k = 64 * part; k < 64 * part + 64; ++k) {
+            const unsigned n = (unsigned)(n0 + 2 * k);
+            if (n >= (unsigned)N / 2) break;
+            acc += taps[k] * costab[(fm * n) & (unsigned)(N - 1)];
+        }
     }
+    sums[part][threadIdx.x & (kSpecFreqs - 1)] = acc;
+    __syncthreads();
+    if (part || f >= N) return;
+    acc = (sums[0][threadIdx.x] + sums[1][threadIdx.x]) + (sums[2][threadIdx.x] + sums[3][threadIdx.x]);
     double H = fabs(h0 + 2.0 * acc) * gain;
     const double w = 2.0 * kPi * fs / N;
     switch (ftype) {
@@ -2692,7 +2695,7 @@ size_t bp_base_bytes(const ctr_geometry* g, BpKind shape) {
 // tiles leaves most of the 256 CUs (five groups each) idle: 32 tiles at 64^3 took 617 us, one per
 // CU at 256^2 x 1 took 1012 us.  Below kBpTargetGroups tiles the views are therefore shared out to
 // so many groups per tile that about kBpTargetGroups run, each summing into its own copy of the
-// volume, added up by bp_reduce_kernel: 98 and 592 us there, 1.91 -> 1.38 ms at 151 x 163 x 107 x
+// volume, added up by sum_parts_kernel: 98 and 592 us there, 1.91 -> 1.38 ms at 151 x 163 x 107 x
 // 241 views, 4.16 -> 3.89 ms at 256^3 x 360 views (2048 tiles: a nearly empty last wave).  2560 and
 // 10240 groups are up to 10 % slower on those than 5120 (too few in flight; more copies to add).
 // A split keeps at least kBpMinViews views (64^3 x 90: 98 us with 4, 116 with 8, 160 with 16).  The
@@ -2797,18 +2800,6 @@ AdjLayout adj_layout(const ctr_geometry* g) {
     return L;
 }
 
-// vol = (accumulate ? vol : 0) + the splits' partial volumes
-int bp_reduce(const ctr_geometry* g, const float* parts, float* vol, int splits, int accumulate, hipStream_t s) {
-    const size_t n = (size_t)g->nx * g->ny * g->nz;
-    if (n % 4 == 0 && (reinterpret_cast<uintptr_t>(vol) & 15) == 0)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(bp_reduce_kernel<4>), dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s,
-                           parts, vol, n, splits, accumulate);
-    else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(bp_reduce_kernel<1>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                           parts, vol, n, splits, accumulate);
-    return status_from_hip(hipGetLastError());
-}
-
 // The matched adjoint's launches: the forward projector's tables, the per-view constants and
 // windows, the row-prefix table, the gather over all voxels and views, the sum of the splits.
 int adj_run(const ctr_geometry* g, const double* angles, const int32_t* branch, const float* proj, float* vol,
@@ -2848,7 +2839,7 @@ int adj_run(const ctr_geometry* g, const double* angles, const int32_t* branch, 
         return hipGetLastError();
     });
     if ((st = status_from_hip(e))) return st;
-    return L.splits > 1 ? bp_reduce(g, parts, vol, L.splits, accumulate, s) : CTR_OK;
+    return L.splits > 1 ? sum_parts(g, parts, vol, L.splits, accumulate, s) : CTR_OK;
 }
 
 // The launches of one shape: the single pass over all cases, or the fast pass over the common
@@ -2902,7 +2893,7 @@ int bp_fdk(const ctr_geometry* g, const double* angles, const float* proj, float
                            g->detector_shape == CTR_DETECTOR_CURVED ? 1 : 0, scale, zero_tol,
                            p.splits > 1 ? 0 : accumulate, tiles_x);
         if ((st = status_from_hip(hipGetLastError()))) return st;
-        return p.splits > 1 ? bp_reduce(g, parts, vol, p.splits, accumulate, s) : CTR_OK;
+        return p.splits > 1 ? sum_parts(g, parts, vol, p.splits, accumulate, s) : CTR_OK;
     }
     // weight zeroing, or a caller's request for one pass (zero_tol < 0): the general kernel does
     // every view
@@ -2919,7 +2910,7 @@ int bp_fdk(const ctr_geometry* g, const double* angles, const float* proj, float
     });
     if (e != hipSuccess) return CTR_ERR_HIP;
     if (p.splits == 1) return CTR_OK;
-    return bp_reduce(g, parts, vol, p.splits, accumulate, s);
+    return sum_parts(g, parts, vol, p.splits, accumulate, s);
 }
 
 }  // namespace
@@ -3059,7 +3050,7 @@ int ctr_filter_spectrum(const ctr_geometry* g, int filter_type, double cutoff, d
     if (N > (1 << kMaxLog2N)) return CTR_ERR_UNSUPPORTED;
     const double tau = g->du * g->sad / g->sdd;
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(spectrum_kernel, dim3((N + 255) / 256), dim3(256), N * sizeof(double), s,
+    hipLaunchKernelGGL(spectrum_kernel, dim3((N + kSpecFreqs - 1) / kSpecFreqs), dim3(256), N * sizeof(double), s,
                        spectrum, N, tau, filter_type, cutoff, 1.0, kPi * cutoff / (2.0 * tau));
     return status_from_hip(hipGetLastError());
 }
@@ -3102,7 +3093,7 @@ int ctr_pixel_filter_spectrum(int n_fft, double tau, int filter_type, double cut
     if (l2 < 1) return CTR_ERR_INVALID;
     if (l2 > kMaxLog2N) return CTR_ERR_UNSUPPORTED;
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(spectrum_kernel, dim3((n_fft + 255) / 256), dim3(256),
+    hipLaunchKernelGGL(spectrum_kernel, dim3((n_fft + kSpecFreqs - 1) / kSpecFreqs), dim3(256),
                        n_fft * sizeof(double), s, spectrum, n_fft, tau, filter_type, cutoff, 2.0,
                        kPi * cutoff);
     return status_from_hip(hipGetLastError());
