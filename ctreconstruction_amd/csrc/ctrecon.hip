@@ -331,7 +331,7 @@ __global__ void __launch_bounds__(64 * kFpWaves, CTR_FP_MIN_WAVES) dd_forward_ke
     const float* __restrict__ t_ys, const float* __restrict__ t_xs, float* __restrict__ proj,
     const float* __restrict__ tabs, const float* __restrict__ rows,
     const int32_t* __restrict__ branch, int nx, int ny, int nz, int nzp, int nu, int nv, int stride,
-    float zero_tol, int n_views, int col_groups, int n_vblocks) {
+    float zero_tol, int n_views, int col_groups, int n_vblocks, int row_shift) {
     // workgroup b runs on XCD b % 8, which takes the column groups cg = 8 c + xcd: every XCD
     // gets an equal share of every band of detector rows (the rows outside the volume's shadow
     // are cheap).  On one XCD the local index runs over (row block, view-pair block, c, pair in
@@ -354,10 +354,10 @@ __global__ void __launch_bounds__(64 * kFpWaves, CTR_FP_MIN_WAVES) dd_forward_ke
     // a wavefront whose columns are all past the detector has no work but stays for the
     // workgroup's final barrier
     const bool live = j0 < nu;
-    const int e0 = rb * kColRows;
+    const int e0 = rb * kColRows - row_shift;  // < 0 in a first block that row_shift moved up
     const int k = e0 + lane;  // this lane's row (lanes 0 .. kColRows-1) and edge
-    const bool active = live && lane < kColRows && k < nv;
-    const int kk = min(k, nv - 1);
+    const bool active = live && lane < kColRows && k >= 0 && k < nv;
+    const int kk = min(max(k, 0), nv - 1);
     // the pair's views: present, slab orientation (x or y slabs; z slabs write zeros)
     int br[kFpViews];
     bool use[kFpViews];
@@ -376,8 +376,8 @@ __global__ void __launch_bounds__(64 * kFpWaves, CTR_FP_MIN_WAVES) dd_forward_ke
     if (!use[0] && !use[1]) return;
     const float fnz = (float)nz;
     // z extent of the wavefront's edges
-    const float nue = rows[min(k, nv)];  // this lane's edge slope
-    const float nu_first = rows[e0], nu_last = rows[min(e0 + kColRows, nv)];
+    const float nue = rows[min(max(k, 0), nv)];  // this lane's edge slope
+    const float nu_first = rows[max(e0, 0)], nu_last = rows[min(e0 + kColRows, nv)];
     // as (slab, column) worker: column j0 + cl of slab n0 + (lane >> 2)
     const int cl = lane & (kFpCols - 1);
     const int jc = min(j0 + cl, nu - 1);
@@ -737,7 +737,7 @@ __global__ void __launch_bounds__(64 * kFpWaves, CTR_FP_MIN_WAVES) dd_forward_ke
         const int r = (it / kFpWaves) % kColRows;
         const int v = it / (kFpWaves * kColRows);
         const int row = e0 + r, jq = jw + q * kFpCols;
-        if (!use[v] || row >= nv || jq >= nu) continue;
+        if (!use[v] || row < 0 || row >= nv || jq >= nu) continue;
         const float4 val = reinterpret_cast<const float4*>(&segs[q][0][0])[v * 64 + r];
         float* __restrict__ o = proj + ((size_t)(view0 + v) * nv + row) * nu + jq;
         if (vec_ok && jq + kFpCols <= nu) {
@@ -2592,6 +2592,43 @@ hipError_t launch_filter(int l2, dim3 grid, hipStream_t st, const float* in, flo
     return hipErrorInvalidValue;
 }
 
+// Rows by which dd_forward_kernel's first row block starts above the detector.  A wavefront skips the
+// slabs that all of its rows miss, so what counts is how many row blocks the volume's shadow touches
+// per slab; the shift with the smallest mean over the distances from the source that the volume spans
+// is taken where it saves at least 3 %.  For circular scans only: a helix moves the shadow.
+// Measured, with the blocks touched per slab: 96^3 x 180 views of 160 rows 3.00 -> 2.00, 309 ->
+// 240 us; 256 x 256 x 200 x 120 views of 420 rows 4.69 -> 4.00, 1847 -> 1688 us; 128^3 x 180 views of
+// 256 rows 3.25 -> 3.00, 505 -> 472 us.  512^3 x 720 views of 768 rows (8.31, at best 8.25) is left
+// alone: shifted so that its largest shadow starts a block it has 8.50 and ran 1.8 % slower.
+int fp_row_shift(const ctr_geometry* g) {
+    constexpr int kDistances = 16;
+    const double reach = 0.5 * std::max(g->nx * g->dx + 2.0 * fabs(g->recon_center[0]),
+                                        g->ny * g->dy + 2.0 * fabs(g->recon_center[1]));
+    if (g->helical != 0.0 || !(g->sad > reach)) return 0;
+    const double z_mid = g->recon_center[2] - g->source_init[2], z_half = 0.5 * g->nz * g->dz;
+    const double half = (g->detector_shape == CTR_DETECTOR_FLAT) ? 0.5 * g->dv : -0.5 * g->dv;
+    const double centre = (g->nv - 1) / 2.0 + (half + g->det_offset[1]) / g->dv;  // edge index at height 0
+    int first[kDistances], last[kDistances];  // rows of the shadow
+    for (int k = 0; k < kDistances; ++k) {
+        const double rows = g->sdd / (g->sad + ((2 * k + 1.0) / kDistances - 1.0) * reach) / g->dv;
+        auto row = [&](double e) { return (int)std::min(std::max(e, 0.0), (double)g->nv); };
+        first[k] = row(floor(centre - (z_mid + z_half) * rows));
+        last[k] = row(ceil(centre - (z_mid - z_half) * rows)) - 1;
+    }
+    int best = 0, fewest = 0, unshifted = 0;
+    for (int shift = 0; shift < kColRows; ++shift) {
+        int touched = 0;
+        for (int k = 0; k < kDistances; ++k)
+            if (first[k] <= last[k]) touched += (last[k] + shift) / kColRows - (first[k] + shift) / kColRows + 1;
+        if (shift == 0) fewest = unshifted = touched;
+        if (touched < fewest) {
+            best = shift;
+            fewest = touched;
+        }
+    }
+    return fewest <= 0.97 * unshifted ? best : 0;
+}
+
 // Scratch memory of ctr_dd_backproject_static, for callers that cannot allocate: the FDK
 // backprojection's per-view table and its (tile, view) flags.  The HIP runtime gives each GPU
 // its own copy when it loads the code object there, and keeps it until the process ends.  In
@@ -3014,7 +3051,8 @@ int ctr_dd_forward(const ctr_geometry* g, const double* angles, const int32_t* b
             g->nv == 3 ? launch(dd_forward_thin_kernel<4, false>) : launch(dd_forward_thin_kernel<5, false>);
     } else {
         const int col_groups = (g->nu + kFpCols * kFpWaves - 1) / (kFpCols * kFpWaves);
-        const int row_blocks = (g->nv + kColRows - 1) / kColRows;
+        const int row_shift = fp_row_shift(g);
+        const int row_blocks = (g->nv + row_shift + kColRows - 1) / kColRows;
         const int n_pairs = (g->n_views + kFpViews - 1) / kFpViews;
         const int n_vblocks = (n_pairs + kViewBlock - 1) / kViewBlock;
         const long long n_blocks =
@@ -3022,7 +3060,7 @@ int ctr_dd_forward(const ctr_geometry* g, const double* angles, const int32_t* b
         if (n_blocks >= 2147483647LL) return CTR_ERR_INVALID;
         hipLaunchKernelGGL(dd_forward_kernel, dim3((unsigned)n_blocks), dim3(64 * kFpWaves), 0, s, t_ys, t_xs,
                            proj, tabs, rows, branch, g->nx, g->ny, g->nz, nzp, g->nu, g->nv, stride, 1e-6f,
-                           g->n_views, col_groups, n_vblocks);
+                           g->n_views, col_groups, n_vblocks, row_shift);
     }
     if ((st = status_from_hip(hipGetLastError()))) return st;
     // z-slab views (left at zero above): their own kernel, which returns at once for the others

@@ -1,0 +1,46 @@
+"""The forward projector's row blocks start above the detector where that makes the volume's shadow
+touch fewer of them: every row is still written once, at the ends of the detector, with the shadow
+anywhere on it, with views of either orientation and of none (z slabs).
+
+Tolerance 1e-4 of the peak against the oracle, as for every operator."""
+import numpy as np
+import pytest
+import torch
+
+import ctreconstruction_amd as ctr
+from ctreconstruction_amd import _native as N
+from oracle import dd_oracle as O
+from tests.conftest import make_params
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-4
+
+
+@pytest.mark.parametrize("nv", [62, 63, 64, 90, 126, 127, 140, 200])
+@pytest.mark.parametrize("nz,zc", [(20, 0.0), (20, 17.0), (20, -25.0), (64, 3.0), (8, 200.0)])
+def test_every_row_is_projected(nv, nz, zc):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    N.lib()
+    p = make_params(NumberOfImage=[9, 10, nz], ReconCenter=[0.0, 0.0, zc], NumberOfDetectorPixels=[14, nv],
+                    DetectorPixelSize=[0.8, 0.6], NumberOfViews=5, StartAngle=0.1, EndAngle=0.1 + 2 * np.pi)
+    g = O.Geometry(p)
+    geom = ctr.ScanGeometry(p)
+    vol = np.random.default_rng(nv).random((g.nz, g.ny, g.nx)).astype(np.float32)
+    ref = O.forward_project(g, vol)
+    out = torch.full(geom.proj_shape, 7.0, device="cuda")
+    out = ctr.dd_forward(torch.from_numpy(vol).cuda(), geom, out=out).cpu().numpy()
+    assert np.abs(out - ref).max() <= TOL * max(np.abs(ref).max(), 1e-30)
+
+
+def test_rows_of_steep_views():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    p = make_params(SourceInit=[0, 300.0, 320.0], DetectorInit=[0, -300.0, -320.0], NumberOfImage=[12, 12, 6],
+                    NumberOfDetectorPixels=[20, 100], NumberOfViews=4)
+    g = O.Geometry(p)
+    vol = np.random.default_rng(1).random((g.nz, g.ny, g.nx)).astype(np.float32)
+    ref = O.forward_project(g, vol)
+    out = ctr.dd_forward(torch.from_numpy(vol).cuda(), ctr.ScanGeometry(p)).cpu().numpy()
+    assert np.abs(out - ref).max() <= TOL * np.abs(ref).max()
