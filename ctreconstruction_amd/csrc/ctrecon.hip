@@ -1,16 +1,16 @@
 // ctrecon.hip -- gfx950 kernels and C ABI for the distance-driven CT projector pair and FDK.
 //
 // Kernels (all FP32 arithmetic; FP64 only in the per-view geometry kernels):
-//   fp_geometry_kernel          per-view DD footprint tables, FP64 -> FP32 (index space)
-//   zprefix_kernel              vol[z][y][x] -> z-prefix tables [y][x][k] and [x][y][k]
+//   fp_prepare_kernel           per-view DD footprint tables, FP64 -> FP32 (index space), and
+//                               vol[z][y][x] -> z-prefix tables [y][x][k] and [x][y][k]
 //   dd_forward_kernel           one wavefront per (2 views, 4 detector columns, 63 rows)
 //   dd_forward_zslab_kernel     z-slab views (non-circular geometries), FP64 loops per cell
-//   bp_geometry_kernel          per-view backprojection constants, FP64 -> FP32
+//   bp_geometry_kernel          per-view backprojection constants, FP64 -> FP32; clears the flags
 //   dd_backproject_tile_kernel  one workgroup per 16 x 16 x ZC voxel tile and view split, windows in LDS
 //   sum_parts_kernel            sums the view splits' partial volumes in a fixed order (splits.h)
-//   adj_geometry_kernel         per-view constants of the inverse central projection
-//   adj_rowprefix_kernel        row prefix sums of projections times path length
-//   adj_tile_kernel             detector windows of every (view, column tile)
+//   adj_geometry_kernel         footprint tables and constants of the inverse central projection
+//   adj_prepare_kernel          row prefix sums of projections times path length; detector windows of
+//                               every (view, column tile)
 //   dd_adjoint_kernel           exact transpose of the forward projector, gathered per voxel, windows in LDS
 //   spectrum_kernel             filter magnitude from the Ram-Lak cosine series, FP64
 //   twiddle_kernel              Stockham twiddles, stage-major, FP64 -> FP32
@@ -122,11 +122,9 @@ __device__ inline void lattice_xy(const ctr_geometry& g, double c, double s, dou
 // One thread per (edge e in [0, nu], view).  FP64 throughout; rounded to FP32 at the store.
 // Follows the host geometry of distance_forward (python/Reconstruction_pycuda.py:828-864,
 // 924-935): lines through the source and the cell-edge lattice, intersection length L.
-__global__ void fp_geometry_kernel(ctr_geometry g, const double* __restrict__ angles,
+__device__ inline void fp_geometry(const ctr_geometry& g, const double* __restrict__ angles,
                                    const int32_t* __restrict__ branch, float* __restrict__ tabs,
-                                   float* __restrict__ rows, int stride) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    const int view = blockIdx.y;
+                                   float* __restrict__ rows, int stride, int e, int view) {
     const int nu = g.nu, nv = g.nv;
     if (view == 0 && e <= nv) {
         // row edges / centres: flat lattice  v2 = -(k - (nv-1)/2) dv + dv/2 (:160),
@@ -205,13 +203,10 @@ __device__ inline float dd_weight(int k, int k0, int k1, float lo, float hi, flo
 // interpolation of P at c.  One workgroup per (y, 32 x-lines): 32 (z) x 32 (x) tiles through
 // LDS, coalesced along x on read and along k on write; lanes 0..31 carry the running sums of
 // the 32 lines.
-__global__ void __launch_bounds__(256) zprefix_kernel(const float* __restrict__ in,
-                                                      float* __restrict__ t_ys,
-                                                      float* __restrict__ t_xs, int nx, int ny,
-                                                      int nz, int nzp) {
+__device__ inline void zprefix(const float* __restrict__ in, float* __restrict__ t_ys, float* __restrict__ t_xs, int nx,
+                               int ny, int nz, int nzp, int x0, int y) {
     __shared__ float tile[32][33];  // [z][x]
     __shared__ float line[32][33];  // [x][z]
-    const int x0 = blockIdx.x * 32, y = blockIdx.y;
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     double run = 0.0;  // running sum of line x0 + threadIdx.x (threads 0..31)
     for (int z0 = 0; z0 < nzp; z0 += 32) {
@@ -238,6 +233,23 @@ __global__ void __launch_bounds__(256) zprefix_kernel(const float* __restrict__ 
             }
         }
         __syncthreads();
+    }
+}
+
+// The forward projector's preparation in one launch: the first workgroups build the z-prefix tables,
+// the others the footprint tables.  Neither needs the other, and for a small scan each would be a
+// launch of a few microseconds.
+__global__ void __launch_bounds__(256) fp_prepare_kernel(ctr_geometry g, const double* __restrict__ angles,
+                                                         const int32_t* __restrict__ branch, float* __restrict__ tabs,
+                                                         float* __restrict__ rows, int stride, int geo_groups,
+                                                         const float* __restrict__ vol, float* __restrict__ t_ys,
+                                                         float* __restrict__ t_xs, int nzp) {
+    const int zx = (g.nx + 31) / 32, zgroups = zx * g.ny, b = blockIdx.x;
+    if (b < zgroups) {
+        zprefix(vol, t_ys, t_xs, g.nx, g.ny, g.nz, nzp, (b % zx) * 32, b / zx);
+    } else {
+        const int r = b - zgroups;
+        fp_geometry(g, angles, branch, tabs, rows, stride, (r % geo_groups) * 256 + (int)threadIdx.x, r / geo_groups);
     }
 }
 
@@ -976,9 +988,12 @@ constexpr int kBpViewStride = 16;  // floats per view in the backprojection tabl
 //                   u index = Au - Bu * atan(slope_u)    (curved, numba units)
 //   [7] Av [8] Bv : v index = Av - Bv * slope_v
 //   [9] SAD
-__global__ void bp_geometry_kernel(ctr_geometry g, const double* __restrict__ angles,
-                                   float* __restrict__ vt, int mode) {
+// The same launch clears the passes' flags (`words` of them; grid-stride).
+__global__ void __launch_bounds__(256) bp_geometry_kernel(ctr_geometry g, const double* __restrict__ angles,
+                                                          float* __restrict__ vt, int mode, uint32_t* __restrict__ flags,
+                                                          size_t words) {
     const int view = blockIdx.x * blockDim.x + threadIdx.x;
+    for (size_t i = view; i < words; i += (size_t)gridDim.x * blockDim.x) flags[i] = 0u;
     if (view >= g.n_views) return;
     const double th = angles[view];
     double s, c;
@@ -1800,11 +1815,6 @@ __global__ void __launch_bounds__(256) bp_slice_kernel(
     vol[idx] = accumulate ? vol[idx] + acc : acc;
 }
 
-__global__ void __launch_bounds__(256) fill_zero_kernel(uint32_t* __restrict__ p, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        p[i] = 0u;
-}
-
 // ------------------------------------------------------------------------------------------
 // Matched adjoint of the forward projector
 // ------------------------------------------------------------------------------------------
@@ -1824,7 +1834,7 @@ __global__ void __launch_bounds__(256) fill_zero_kernel(uint32_t* __restrict__ p
 // edges are equally spaced in nu (nu_e = nuA + nuB e), so a row's footprint is the unit step
 // [k, k+1] in the edge coordinate e(c) = ((c - gamma) / tt - nuA) / nuB, and voxel kc receives
 // sgn(nuB tt) o_a / w_a (Y(e(kc + 1)) - Y(e(kc))) with Y the linear interpolation of the
-// row prefix Y_e = sum_{k < e} y_k L_k (adj_rowprefix_kernel): one table lookup per voxel
+// row prefix Y_e = sum_{k < e} y_k L_k (adj_rowprefix): one table lookup per voxel
 // boundary instead of a walk over rows.
 //
 // Organisation: a workgroup owns a 16 x 16 x TZ voxel tile and a share of the views (splits, as in
@@ -1833,7 +1843,7 @@ __global__ void __launch_bounds__(256) fill_zero_kernel(uint32_t* __restrict__ p
 // those columns) is fetched two views ahead into registers and written to one of two LDS buffers
 // while the other is read, one barrier per view, together with the footprint lines and slab
 // fractions of the window's columns.  Rows off the detector hold the end values of Y, so a lookup
-// needs no clamp.  adj_tile_kernel works the windows out per (view, column tile); a window too
+// needs no clamp.  adj_tile works the windows out per (view, column tile); a window too
 // large for LDS is gathered from global memory after the other views.
 constexpr int kAdjViewStride = 16;
 constexpr int kAdjCols = 127;  // most window columns
@@ -1853,10 +1863,8 @@ struct AdjShape {
 //   [3] r = d_t / d_s  [4] eu_t [5] eu_s [6] ew_t [7] ew_s  (detector axes, transverse/slab parts)
 //   [8] SDD  [9] u2_0: coordinate of edge 0  [10] 1/step (mm or rad)
 //   [11] nuA, [12] 1/nuB : row edge e has z index slope nu_e = nuA + nuB * e
-__global__ void adj_geometry_kernel(ctr_geometry g, const double* __restrict__ angles,
-                                    const int32_t* __restrict__ branch, float* __restrict__ at) {
-    const int view = blockIdx.x * blockDim.x + threadIdx.x;
-    if (view >= g.n_views) return;
+__device__ inline void adj_geometry(const ctr_geometry& g, const double* __restrict__ angles,
+                                    const int32_t* __restrict__ branch, float* __restrict__ at, int view) {
     const double th = angles[view];
     double s, c;
     sincos(th, &s, &c);
@@ -1894,6 +1902,16 @@ __global__ void adj_geometry_kernel(ctr_geometry g, const double* __restrict__ a
     T[12] = (float)(1.0 / nuB);
 }
 
+// The forward projector's footprint tables and the constants above in one launch: one thread per
+// (edge, view), and the view's first one its constants.
+__global__ void __launch_bounds__(256) adj_geometry_kernel(ctr_geometry g, const double* __restrict__ angles,
+                                                           const int32_t* __restrict__ branch, float* __restrict__ tabs,
+                                                           float* __restrict__ rows, int stride, float* __restrict__ at) {
+    const int e = blockIdx.x * 256 + threadIdx.x, view = blockIdx.y;
+    fp_geometry(g, angles, branch, tabs, rows, stride, e, view);
+    if (e == 0) adj_geometry(g, angles, branch, at, view);
+}
+
 // Edge coordinate (fractional edge index) of the ray from the source through the point at
 // transverse index coordinate tk and slab coordinate n.
 __device__ inline float adj_edge_coord(const float* A, float tk, float n, int curved) {
@@ -1908,14 +1926,11 @@ __device__ inline float adj_edge_coord(const float* A, float tk, float n, int cu
 // sqrt(1 + s2_k^2), evaluated as the forward projector evaluates it), summed in FP64, stored in
 // FP32; entries past nv repeat the total.  One workgroup per (view, 32 columns): 32 x 32 tiles
 // through LDS, coalesced along j on read and along e on write; lanes 0..31 carry the sums.
-__global__ void __launch_bounds__(256) adj_rowprefix_kernel(const float* __restrict__ y,
-                                                            float* __restrict__ Y,
-                                                            const float* __restrict__ tabs,
-                                                            const float* __restrict__ rows, int nu,
-                                                            int nv, int nvp, int stride) {
+__device__ inline void adj_rowprefix(const float* __restrict__ y, float* __restrict__ Y, const float* __restrict__ tabs,
+                                     const float* __restrict__ rows, int nu, int nv, int nvp, int stride, int j0,
+                                     int view) {
     __shared__ float tile[32][33];  // [k][j]
     __shared__ float line[32][33];  // [j][e]
-    const int j0 = blockIdx.x * 32, view = blockIdx.y;
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     const float* T = tabs + (size_t)view * stride;
     const int jj = min(j0 + tx, nu - 1);
@@ -1973,10 +1988,9 @@ __device__ inline int adj_pitch(int rows) { return rows | 1; }
 // corners; t is affine in the slab for each column.  A tile that is not wholly in front of the
 // source (its depth, affine over the tile, changes sign between corners, or its slabs reach the
 // source's) has no such window and takes the gather path.
-__global__ void adj_tile_kernel(AdjTile* __restrict__ tw, const float* __restrict__ tabs, const float* __restrict__ at,
+__device__ inline void adj_tile(AdjTile* __restrict__ tw, const float* __restrict__ tabs, const float* __restrict__ at,
                                 int nx, int ny, int nz, int nu, int n_views, int stride, int curved, int tiles_x,
-                                int n_tiles, int tz, int slabs, int cap) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+                                int n_tiles, int tz, int slabs, int cap, int idx) {
     if (idx >= n_views * n_tiles) return;
     const int view = idx / n_tiles, t = idx - view * n_tiles;
     const int x0 = (t % tiles_x) * kTileX, y0 = (t / tiles_x) * kTileY;
@@ -2027,6 +2041,20 @@ __global__ void adj_tile_kernel(AdjTile* __restrict__ tw, const float* __restric
         }
     }
     tw[idx] = w;
+}
+
+// The row-prefix table (the first workgroups) and the windows (the others) in one launch.
+__global__ void __launch_bounds__(256) adj_prepare_kernel(const float* __restrict__ y, float* __restrict__ Y,
+                                                          const float* __restrict__ tabs, const float* __restrict__ rows,
+                                                          const float* __restrict__ at, AdjTile* __restrict__ tw, int nx,
+                                                          int ny, int nz, int nu, int nv, int nvp, int n_views, int stride,
+                                                          int curved, int tiles_x, int n_tiles, int tz, int slabs, int cap) {
+    const int px = (nu + 31) / 32, pgroups = px * n_views, b = blockIdx.x;
+    if (b < pgroups)
+        adj_rowprefix(y, Y, tabs, rows, nu, nv, nvp, stride, (b % px) * 32, b / px);
+    else
+        adj_tile(tw, tabs, at, nx, ny, nz, nu, n_views, stride, curved, tiles_x, n_tiles, tz, slabs, cap,
+                 (b - pgroups) * 256 + (int)threadIdx.x);
 }
 
 // One column's share of a work-item's voxels: boundary c of the volume has the edge coordinate
@@ -2855,17 +2883,15 @@ int adj_run(const ctr_geometry* g, const double* angles, const int32_t* branch, 
     const int curved = g->detector_shape == CTR_DETECTOR_CURVED ? 1 : 0;
     int st = CTR_OK;
     const int gx = (std::max(g->nu + 1, g->nv + 1) + 255) / 256;
-    hipLaunchKernelGGL(fp_geometry_kernel, dim3(gx, g->n_views), dim3(256), 0, s, *g, angles, branch, tabs, rows, stride);
-    if ((st = status_from_hip(hipGetLastError()))) return st;
-    hipLaunchKernelGGL(adj_geometry_kernel, dim3((g->n_views + 255) / 256), dim3(256), 0, s, *g, angles, branch, at);
-    if ((st = status_from_hip(hipGetLastError()))) return st;
-    hipLaunchKernelGGL(adj_tile_kernel, dim3((unsigned)(((size_t)g->n_views * n_tiles + 255) / 256)), dim3(256), 0, s, tw,
-                       tabs, at, g->nx, g->ny, g->nz, g->nu, g->n_views, stride, curved, L.tiles_x, n_tiles, L.tz,
-                       L.tiles_z, L.cap);
+    hipLaunchKernelGGL(adj_geometry_kernel, dim3(gx, g->n_views), dim3(256), 0, s, *g, angles, branch, tabs, rows, stride,
+                       at);
     if ((st = status_from_hip(hipGetLastError()))) return st;
     const int nvp = adj_prefix_stride(g->nv);
-    hipLaunchKernelGGL(adj_rowprefix_kernel, dim3((g->nu + 31) / 32, g->n_views), dim3(256), 0, s, proj, yp, tabs, rows,
-                       g->nu, g->nv, nvp, stride);
+    const long long groups = (long long)((g->nu + 31) / 32) * g->n_views + ((long long)g->n_views * n_tiles + 255) / 256;
+    if (groups >= 2147483647LL) return CTR_ERR_INVALID;
+    hipLaunchKernelGGL(adj_prepare_kernel, dim3((unsigned)groups), dim3(256), 0, s, proj, yp, tabs, rows, at, tw, g->nx,
+                       g->ny, g->nz, g->nu, g->nv, nvp, g->n_views, stride, curved, L.tiles_x, n_tiles, L.tz, L.tiles_z,
+                       L.cap);
     if ((st = status_from_hip(hipGetLastError()))) return st;
     const hipError_t e = adj_with_shape(L.shape, [&](auto sh) {
         // transverse overlaps under 1e-6 of the footprint are dropped, as in ctr_dd_forward
@@ -2915,11 +2941,16 @@ int bp_fdk(const ctr_geometry* g, const double* angles, const float* proj, float
     const size_t tiles = bp_tiles(g, p.shape);
     if (tiles >= 2147483647u) return CTR_ERR_INVALID;
     float* vt = (float*)workspace;
-    hipLaunchKernelGGL(bp_geometry_kernel, dim3((g->n_views + 255) / 256), dim3(256), 0, s, *g,
-                       angles, vt, mode);
-    if ((st = status_from_hip(hipGetLastError()))) return st;
     uint8_t* flags = (uint8_t*)workspace + align_up((size_t)g->n_views * kBpViewStride * sizeof(float), 256);
     float* parts = (float*)((char*)workspace + p.base);
+    // weight zeroing, or a caller's request for one pass (zero_tol < 0): the general kernel does
+    // every view, as the slice kernel does for a single slice; only the two passes use the flags
+    const bool one_pass = zero_tol != 0.0f;
+    const size_t flag_words = one_pass || g->nz == 1 ? 0 : align_up(tiles * g->n_views, 256) / 4;
+    const size_t geo_groups = std::max<size_t>((g->n_views + 255) / 256, std::min<size_t>((flag_words + 1023) / 1024, 4096));
+    hipLaunchKernelGGL(bp_geometry_kernel, dim3((unsigned)geo_groups), dim3(256), 0, s, *g, angles, vt, mode,
+                       (uint32_t*)flags, flag_words);
+    if ((st = status_from_hip(hipGetLastError()))) return st;
     if (g->nz == 1) {
         const int tiles_x = (g->nx + kTileX - 1) / kTileX;
         hipLaunchKernelGGL(bp_slice_kernel, dim3((unsigned)tiles, p.splits), dim3(256), 0, s, proj, vol, vt, parts, g->nx,
@@ -2931,15 +2962,6 @@ int bp_fdk(const ctr_geometry* g, const double* angles, const float* proj, float
                            p.splits > 1 ? 0 : accumulate, tiles_x);
         if ((st = status_from_hip(hipGetLastError()))) return st;
         return p.splits > 1 ? sum_parts(g, parts, vol, p.splits, accumulate, s) : CTR_OK;
-    }
-    // weight zeroing, or a caller's request for one pass (zero_tol < 0): the general kernel does
-    // every view
-    const bool one_pass = zero_tol != 0.0f;
-    if (!one_pass) {
-        const size_t flag_words = align_up(tiles * g->n_views, 256) / 4;
-        hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)std::min<size_t>((flag_words + 255) / 256, 65536)),
-                           dim3(256), 0, s, (uint32_t*)flags, flag_words);
-        if ((st = status_from_hip(hipGetLastError()))) return st;
     }
     const hipError_t e = bp_with_shape(p.shape, [&](auto sh) {
         return bp_passes<decltype(sh)>(g, p, one_pass, proj, vol, vt, flags, parts, scale, zero_tol,
@@ -3029,12 +3051,11 @@ int ctr_dd_forward(const ctr_geometry* g, const double* angles, const int32_t* b
     float* t_xs = (float*)(ws + L.volt_off + L.copy_bytes);
     const int stride = fp_view_stride(g->nu);
     const int gx = (std::max(g->nu + 1, g->nv + 1) + 255) / 256;
-    hipLaunchKernelGGL(fp_geometry_kernel, dim3(gx, g->n_views), dim3(256), 0, s, *g, angles, branch,
-                       tabs, rows, stride);
-    if ((st = status_from_hip(hipGetLastError()))) return st;
     const int nzp = zprefix_stride(g->nz);
-    hipLaunchKernelGGL(zprefix_kernel, dim3((g->nx + 31) / 32, g->ny), dim3(256), 0, s, vol, t_ys, t_xs,
-                       g->nx, g->ny, g->nz, nzp);
+    const long long prep = (long long)((g->nx + 31) / 32) * g->ny + (long long)gx * g->n_views;
+    if (prep >= 2147483647LL) return CTR_ERR_INVALID;
+    hipLaunchKernelGGL(fp_prepare_kernel, dim3((unsigned)prep), dim3(256), 0, s, *g, angles, branch, tabs, rows, stride, gx,
+                       vol, t_ys, t_xs, nzp);
     if ((st = status_from_hip(hipGetLastError()))) return st;
     if (g->nv <= kThinRows) {
         static_assert(kThinRows == 4, "one wavefront per row");
