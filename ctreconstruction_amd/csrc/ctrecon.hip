@@ -2353,8 +2353,12 @@ __global__ void __launch_bounds__(256) spectrum_kernel(double* __restrict__ out,
 // keeps exp(-2 pi i r m / (ns R)), r = 1 .. R-1, m = 0 .. ns-1, at index r ns + m - 1 (N - 1
 // entries in all).  A butterfly's twiddles for one r are then consecutive across the lanes of a
 // wavefront.  The angle is evaluated as 2 pi k / N with k = r m N / (ns R).
-__global__ void twiddle_kernel(float2* __restrict__ tw, int N, int log2n) {
+// The same launch stores the spectrum times the output scale (rounded once, from FP64) as hs[N], so
+// that the filter reads half the bytes per frequency and has nothing to convert or scale.
+__global__ void twiddle_kernel(float2* __restrict__ tw, float* __restrict__ hs, const double* __restrict__ spec,
+                               double scale, int N, int log2n) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < N) hs[e] = (float)(spec[e] * scale);
     if (e >= N - 1) return;
     const int x = e + 1;        // r ns + m
     const int n16 = log2n / 4;  // radix-16 stages
@@ -2374,9 +2378,11 @@ __device__ inline float2 cmul(float2 a, float2 b) {
 __device__ inline float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __device__ inline float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
 
-// Threads per FFT workgroup: 128 up to N = 2048 (one radix-16 butterfly per thread and stage,
-// and twice the workgroups per CU of 256 threads), 256 above (the butterflies' registers)
-constexpr int fft_threads(int log2n) { return log2n <= 11 ? 128 : 256; }
+// Threads per row pair: one radix-16 butterfly per thread and stage (at most 256: two, N = 8192).  Up
+// to N = 1024 that is a wavefront or less, so a workgroup is one wavefront with 1024 / N row pairs
+// and its barriers cost nothing; with 128 threads per pair most of them had no butterfly.
+constexpr int fft_threads(int log2n) { return log2n <= 4 ? 1 : log2n >= 12 ? 256 : 1 << (log2n - 4); }
+constexpr int fft_pairs(int log2n) { return fft_threads(log2n) >= 64 ? 1 : 64 / fft_threads(log2n); }
 
 // In-register DFTs of 2, 4, 8 and 16 points (forward: exp(-2 pi i n k / R); `inv` conjugates),
 // results in natural order.  8 = 2 x 4 and 16 = 4 x 4 Cooley-Tukey with the internal twiddles.
@@ -2393,8 +2399,19 @@ __device__ inline void dft4(float2& x0, float2& x1, float2& x2, float2& x3, bool
     x3 = csub(a1, a3);
 }
 
-template <int R>
+// dft4 of inputs whose upper half is zero
+__device__ inline void dft4_half(float2& x0, float2& x1, float2& x2, float2& x3, bool inv) {
+    const float2 a = x0, b = x1, c = mul_mi(x1, inv);
+    x0 = cadd(a, b);
+    x1 = cadd(a, c);
+    x2 = csub(a, b);
+    x3 = csub(a, c);
+}
+
+// HALF: elements R/2 .. R-1 are zero (radix 16 only)
+template <int R, bool HALF = false>
 __device__ inline void dft_reg(float2 (&v)[R], bool inv) {
+    static_assert(!HALF || R == 16, "zero upper half");
     if constexpr (R == 2) {
         const float2 a = v[0], b = v[1];
         v[0] = cadd(a, b);
@@ -2423,7 +2440,12 @@ __device__ inline void dft_reg(float2 (&v)[R], bool inv) {
         static_assert(R == 16, "radix");
         // n = 4 n1 + n2, k = k1 + 4 k2: DFT4 over n1, twiddle W16^(n2 k1), DFT4 over n2
 #pragma unroll
-        for (int n2 = 0; n2 < 4; ++n2) dft4(v[n2], v[4 + n2], v[8 + n2], v[12 + n2], inv);
+        for (int n2 = 0; n2 < 4; ++n2) {
+            if constexpr (HALF)
+                dft4_half(v[n2], v[4 + n2], v[8 + n2], v[12 + n2], inv);
+            else
+                dft4(v[n2], v[4 + n2], v[8 + n2], v[12 + n2], inv);
+        }
         const float s = inv ? 1.0f : -1.0f;
         constexpr float c1 = 0.92387953251128674f, s1 = 0.38268343236508978f, h = 0.70710678118654752f;
         // element [4 k1 + n2] now holds A[n2][k1]
@@ -2452,7 +2474,7 @@ __device__ inline void dft_reg(float2 (&v)[R], bool inv) {
 // largest power of two not above r (r >= 1)
 constexpr int top_bit(int r) { return (r & (r - 1)) == 0 ? r : top_bit(r & (r - 1)); }
 
-// One radix-R Stockham stage over sub-transforms of length ns, with T threads per workgroup:
+// One radix-R Stockham stage over sub-transforms of length ns, with T threads (index tid) per transform:
 // butterfly j reads element j + r N/R, applies the twiddles exp(-+2 pi i r (j mod ns) / (ns R))
 // (stage-major table of twiddle_kernel; the power-of-two ones loaded, the others formed as
 // products of two earlier ones, at most three roundings deep), takes an R-point DFT and writes
@@ -2466,19 +2488,29 @@ constexpr int top_bit(int r) { return (r & (r - 1)) == 0 ? r : top_bit(r & (r - 
 constexpr int kFromLds = 0, kFromGlobal = 1;
 constexpr int kToLds = 0, kToLdsTimesSpectrum = 1, kToGlobal = 2;
 
-template <int R, int N, int T, int SRC, int DST, typename Load, typename Store>
-__device__ void stockham_stage_io(float2* buf, const float2* __restrict__ tw, int ns, bool inv,
-                                  const double* __restrict__ spec, Load&& load, Store&& store) {
+//
+// Element n sits at position n ^ ((n >> 4) & 15) of the buffer: the first stage writes runs of 16
+// elements per lane, which in natural order fall in two of the 64 banks.  With element indices of
+// the form base + r * step (step a power of two above base's low part) the position is
+// (base's position ^ a constant of r) + r * step, one exclusive or at most per element.
+// HALF: only the first N/2 samples are read from and written to global memory (the rest is padding):
+// half of the first stage's inputs are zero, and half of the last stage's outputs are not formed.
+template <int R, int N, int T, int ns, int SRC, int DST, bool HALF, typename Load, typename Store>
+__device__ void stockham_stage_io(float2* buf, int tid, const float2* __restrict__ tw, bool inv,
+                                  const float* __restrict__ spec, Load&& load, Store&& store) {
+    constexpr bool kHalfIn = HALF && SRC == kFromGlobal && R == 16;
+    constexpr int kIn = kHalfIn ? R / 2 : R, kOut = HALF && DST == kToGlobal ? R / 2 : R;
     constexpr int NBF = N / R;  // butterflies
     constexpr int NB = (NBF + T - 1) / T;
-    const int tid = threadIdx.x;
     float2 v[NB][R];
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
         const int j = tid + b * T;
         if (j < NBF) {
+            const int jp = j ^ ((j >> 4) & 15);
 #pragma unroll
-            for (int r = 0; r < R; ++r) v[b][r] = SRC == kFromGlobal ? load(j + r * NBF) : buf[j + r * NBF];
+            for (int r = 0; r < kIn; ++r)
+                v[b][r] = SRC == kFromGlobal ? load(b, r, j + r * NBF) : buf[(jp ^ ((r * NBF >> 4) & 15)) + r * NBF];
             const int m = j % ns;
             if (m != 0) {
                 float2 w[R];
@@ -2495,7 +2527,7 @@ __device__ void stockham_stage_io(float2* buf, const float2* __restrict__ tw, in
 #pragma unroll
                 for (int r = 1; r < R; ++r) v[b][r] = cmul(v[b][r], w[r]);
             }
-            dft_reg<R>(v[b], inv);
+            dft_reg<R, kHalfIn>(v[b], inv);
         }
     }
     if constexpr (SRC == kFromLds && DST != kToGlobal) __syncthreads();
@@ -2504,16 +2536,18 @@ __device__ void stockham_stage_io(float2* buf, const float2* __restrict__ tw, in
         const int j = tid + b * T;
         if (j < NBF) {
             const int base = (j / ns) * ns * R + (j % ns);
+            const int bp = base ^ ((base >> 4) & 15);
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
+            for (int r = 0; r < kOut; ++r) {
                 const int n = base + r * ns;
+                const int at = ns == 1 ? bp ^ r : (bp ^ ((r * ns >> 4) & 15)) + r * ns;
                 if constexpr (DST == kToGlobal) {
                     store(n, v[b][r]);
                 } else if constexpr (DST == kToLdsTimesSpectrum) {
-                    const float h = (float)spec[n];
-                    buf[n] = make_float2(v[b][r].x * h, v[b][r].y * h);
+                    const float h = spec[n];
+                    buf[at] = make_float2(v[b][r].x * h, v[b][r].y * h);
                 } else {
-                    buf[n] = v[b][r];
+                    buf[at] = v[b][r];
                 }
             }
         }
@@ -2523,22 +2557,22 @@ __device__ void stockham_stage_io(float2* buf, const float2* __restrict__ tw, in
 
 // Stage st of the length-2^LOG2N transform (radix 16 for st < LOG2N / 4, then the radix of the
 // remaining factor), with its source and sink.
-template <int LOG2N, int ST, int SRC, int DST, typename Load, typename Store>
-__device__ void fft_stage_io(float2* buf, const float2* __restrict__ tw, bool inv, const double* __restrict__ spec,
+template <int LOG2N, int ST, int SRC, int DST, bool HALF, typename Load, typename Store>
+__device__ void fft_stage_io(float2* buf, int tid, const float2* __restrict__ tw, bool inv, const float* __restrict__ spec,
                              Load&& load, Store&& store) {
     constexpr int N = 1 << LOG2N;
     constexpr int T = fft_threads(LOG2N);
     constexpr int n16 = LOG2N / 4;
     constexpr int R = ST < n16 ? 16 : 1 << (LOG2N % 4);
-    const int ns = 1 << (4 * ST);
-    stockham_stage_io<R, N, T, SRC, DST>(buf, tw, ns, inv, spec, load, store);
+    constexpr int ns = 1 << (4 * ST);
+    stockham_stage_io<R, N, T, ns, SRC, DST, HALF>(buf, tid, tw, inv, spec, load, store);
 }
 
 // The filter's convolution: forward FFT from `load`, times the spectrum, inverse FFT to `store`,
 // with the first forward stage reading global memory, the spectrum applied as the last forward
 // stage writes LDS and the last inverse stage writing global memory.
-template <int LOG2N, int ST = 0, typename Load, typename Store>
-__device__ void fft_filter_stages(float2* buf, const float2* __restrict__ tw, const double* __restrict__ spec,
+template <int LOG2N, bool HALF, int ST = 0, typename Load, typename Store>
+__device__ void fft_filter_stages(float2* buf, int tid, const float2* __restrict__ tw, const float* __restrict__ spec,
                                   Load&& load, Store&& store) {
     constexpr int NST = LOG2N / 4 + (LOG2N % 4 ? 1 : 0);  // stages per transform
     if constexpr (ST < 2 * NST) {
@@ -2546,8 +2580,8 @@ __device__ void fft_filter_stages(float2* buf, const float2* __restrict__ tw, co
         constexpr int k = inv ? ST - NST : ST;
         constexpr int SRC = ST == 0 ? kFromGlobal : kFromLds;
         constexpr int DST = ST == NST - 1 ? kToLdsTimesSpectrum : (ST == 2 * NST - 1 ? kToGlobal : kToLds);
-        fft_stage_io<LOG2N, k, SRC, DST>(buf, tw, inv, spec, load, store);
-        fft_filter_stages<LOG2N, ST + 1>(buf, tw, spec, load, store);
+        fft_stage_io<LOG2N, k, SRC, DST, HALF>(buf, tid, tw, inv, spec, load, store);
+        fft_filter_stages<LOG2N, HALF, ST + 1>(buf, tid, tw, spec, load, store);
     }
 }
 
@@ -2559,6 +2593,9 @@ __device__ void fft_filter_stages(float2* buf, const float2* __restrict__ tw, co
 // ConeBeamGPU's filtering (python/ConeBeamGPU.py:296-302) weighs at cell centres (off_u =
 // du R/(2 SDD), off_v = -dv R/(2 SDD)) and filters fliplr(row): the spectrum is real and
 // even, so that equals the mirror image of the filtered row, written with mirror = 1.
+// Bound by VALU issue and the wait for the rows: 2.8 TB/s at 720 x 768 rows of 1024 (2.1 TB/s before the
+// swizzled buffer, the half transforms, the FP32 spectrum and the persistent workgroups); at 180 x 256
+// rows of 256 columns 2.45 TB/s (1.4 TB/s with a row pair per 128 threads).
 // The FFTs are Stockham transforms in LDS, radix-16 stages (two radix-4 levels in registers per
 // LDS round trip) and one radix-2, 4 or 8 stage for the remaining factor.  The first forward
 // stage reads the two rows from global memory and the last inverse stage writes them back, so the
@@ -2566,56 +2603,96 @@ __device__ void fft_filter_stages(float2* buf, const float2* __restrict__ tw, co
 // no separate load, spectrum or store pass.
 // `in` and `out` may be the same buffer (in-place filtering): a block reads its two rows before
 // its first barrier and writes them after its last one, and no other block touches them.
-template <int LOG2N>
-__global__ void __launch_bounds__(fft_threads(LOG2N)) fdk_filter_kernel(
-    const float* in, float* out, const double* __restrict__ spec,
+template <int LOG2N, bool HALF, bool PERSIST>
+__global__ void __launch_bounds__(fft_threads(LOG2N) * fft_pairs(LOG2N)) fdk_filter_kernel(
+    const float* in, float* out, const float* __restrict__ spec,
     const float2* __restrict__ tw, int n_rows, int nu, int nv, float R, float su, float ou,
-    float sv, float ov, float out_scale, int mirror) {
+    float sv, float ov, int mirror) {
     constexpr int N = 1 << LOG2N;
-    constexpr int T = fft_threads(LOG2N);
-    __shared__ float2 buf[N];
-    const int rowA = 2 * blockIdx.x;
-    const int rowB = rowA + 1;
-    const bool hasB = rowB < n_rows;
-    const float pa = ((float)(nv / 2.0f) - (float)(rowA % nv)) * sv + ov;
-    const float pb = ((float)(nv / 2.0f) - (float)(rowB % nv)) * sv + ov;
-    // sample n of the weighted, zero-padded row pair (read by the first forward stage)
-    auto load = [&](int n) {
-        float2 val = make_float2(0.0f, 0.0f);
-        if (n < nu) {
-            const float kk = ((float)n - (float)nu / 2.0f) * su + ou;
-            const float wa = R * rsqrtf(R * R + kk * kk + pa * pa);
-            val.x = in[(size_t)rowA * nu + n] * wa;
-            if (hasB) {
-                const float wb = R * rsqrtf(R * R + kk * kk + pb * pb);
-                val.y = in[(size_t)rowB * nu + n] * wb;
+    constexpr int T = fft_threads(LOG2N), P = fft_pairs(LOG2N);
+    __shared__ float2 bufs[P * N];
+    const int tid = threadIdx.x % T;
+    float2* buf = bufs + (threadIdx.x / T) * N;
+    // the first stage's samples: butterfly b of this thread reads n = j + r N/R0
+    constexpr int R0 = LOG2N / 4 > 0 ? 16 : 1 << LOG2N, NBF = N / R0, NB = (NBF + T - 1) / T;
+    constexpr int kIn = HALF && R0 == 16 ? R0 / 2 : R0;
+    const int step = 2 * P * gridDim.x;
+    float2 raw[NB][kIn];
+    auto fetch = [&](int rowA) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int r = 0; r < kIn; ++r) {
+                const int n = tid + b * T + r * NBF;
+                const bool ok = n < nu && rowA < n_rows;
+                raw[b][r].x = ok ? in[(size_t)rowA * nu + n] : 0.0f;
+                raw[b][r].y = ok && rowA + 1 < n_rows ? in[(size_t)(rowA + 1) * nu + n] : 0.0f;
             }
-        }
-        return val;
     };
-    // sample n of the filtered pair (written by the last inverse stage; the padding is dropped)
-    auto store = [&](int n, float2 val) {
-        if (n < nu) {
-            const int j = mirror ? nu - 1 - n : n;
-            out[(size_t)rowA * nu + j] = val.x * out_scale;
-            if (hasB) out[(size_t)rowB * nu + j] = val.y * out_scale;
-        }
-    };
-    fft_filter_stages<LOG2N>(buf, tw, spec, load, store);
+    int rowA = 2 * (blockIdx.x * P + threadIdx.x / T);
+    fetch(rowA);
+    // uniform: the workgroup's first pair decides how often it goes round
+    for (int first = 2 * P * blockIdx.x; first < n_rows; first += step, rowA += step) {
+        const float pa = ((float)(nv / 2.0f) - (float)(rowA % nv)) * sv + ov;
+        const float pb = ((float)(nv / 2.0f) - (float)((rowA + 1) % nv)) * sv + ov;
+        // sample n of the weighted, zero-padded row pair
+        auto load = [&](int b, int r, int n) {
+            const float kk = ((float)n - (float)nu / 2.0f) * su + ou;
+            const float wa = R * rsqrtf(R * R + kk * kk + pa * pa), wb = R * rsqrtf(R * R + kk * kk + pb * pb);
+            const float2 val = make_float2(raw[b][r].x * wa, raw[b][r].y * wb);
+            // the next pair's rows arrive while this one is transformed
+            if (PERSIST && b == NB - 1 && r == kIn - 1) fetch(rowA + step);
+            return val;
+        };
+        // sample n of the filtered pair (written by the last inverse stage; the padding is dropped)
+        auto store = [&](int n, float2 val) {
+            if (n < nu && rowA < n_rows) {
+                const int j = mirror ? nu - 1 - n : n;
+                out[(size_t)rowA * nu + j] = val.x;
+                if (rowA + 1 < n_rows) out[(size_t)(rowA + 1) * nu + j] = val.y;
+            }
+        };
+        fft_filter_stages<LOG2N, HALF>(buf, tid, tw, spec, load, store);
+        if (!PERSIST) break;
+        // the last stage reads LDS and the next pair's first stage writes it
+        __syncthreads();
+    }
 }
 
+// PERSIST workgroups: two wavefronts per SIMD (their registers, below) on 256 CUs.  Persistent
+// workgroups fetch the next row pair while they transform one and keep the twiddles in registers
+// (205 of them): 2.14 -> 1.62 ms at 720 x 768 rows of 1024 (1.97 without), 1.45 -> 1.11 ms at 360 x 500
+// rows of 1800 (1.23).  Shorter transforms gain nothing from it (300 columns, 300 x 200 rows: 75 us
+// without, 80 with), nor does a launch of fewer than four rounds.  Without PERSIST more wavefronts at 96
+// registers (five per SIMD) are slower: 2.25 ms, 1.61 ms.
+constexpr int kFftResident = 256 * 4 * 2 * 64;  // threads
+
 template <int L>
-hipError_t launch_filter(int l2, dim3 grid, hipStream_t st, const float* in, float* out,
-                         const double* spec, const float2* tw, int n_rows, int nu, int nv, float R,
-                         float su, float ou, float sv, float ov, float scale, int mirror) {
+hipError_t launch_filter(int l2, hipStream_t st, const float* in, float* out,
+                         const float* spec, const float2* tw, int n_rows, int nu, int nv, float R,
+                         float su, float ou, float sv, float ov, int mirror) {
     if (l2 == L) {
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(fdk_filter_kernel<L>), grid, dim3(fft_threads(L)), 0, st,
-                           in, out, spec, tw, n_rows, nu, nv, R, su, ou, sv, ov, scale, mirror);
+        // nu is at most N/2 + 1, and that only where nu - 1 is a power of two
+        constexpr int P = fft_pairs(L);
+        int groups = (n_rows + 2 * P - 1) / (2 * P);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(groups), dim3(fft_threads(L) * P), 0, st, in, out, spec, tw, n_rows, nu, nv, R, su,
+                               ou, sv, ov, mirror);
+        };
+        const bool half = nu <= (1 << L) / 2;
+        if constexpr (L == 11 || L == 12) {
+            if (groups >= 4 * kFftResident / fft_threads(L)) {
+                groups = kFftResident / fft_threads(L);
+                half ? launch(fdk_filter_kernel<L, true, true>) : launch(fdk_filter_kernel<L, false, true>);
+                return hipGetLastError();
+            }
+        }
+        half ? launch(fdk_filter_kernel<L, true, false>) : launch(fdk_filter_kernel<L, false, false>);
         return hipGetLastError();
     }
     if constexpr (L < kMaxLog2N) {
-        return launch_filter<L + 1>(l2, grid, st, in, out, spec, tw, n_rows, nu, nv, R, su, ou, sv,
-                                    ov, scale, mirror);
+        return launch_filter<L + 1>(l2, st, in, out, spec, tw, n_rows, nu, nv, R, su, ou, sv,
+                                    ov, mirror);
     }
     return hipErrorInvalidValue;
 }
@@ -3094,7 +3171,7 @@ size_t ctr_fdk_filter_workspace_bytes(const ctr_geometry* g) {
     if (check_geometry(g)) return 0;
     const int N = ctr_zero_padded_length(g->nu);
     if (N <= 0) return 0;
-    return align_up((size_t)N * sizeof(float2), 256);
+    return align_up((size_t)N * (sizeof(float2) + sizeof(float)), 256);  // twiddles, scaled spectrum
 }
 
 int ctr_filter_spectrum(const ctr_geometry* g, int filter_type, double cutoff, double* spectrum,
@@ -3129,17 +3206,17 @@ int ctr_fdk_filter(const ctr_geometry* g, const double* spectrum, const float* p
     if (workspace_bytes < ctr_fdk_filter_workspace_bytes(g)) return CTR_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     float2* tw = (float2*)workspace;
-    hipLaunchKernelGGL(twiddle_kernel, dim3((N + 255) / 256), dim3(256), 0, s, tw, N, l2);
-    if ((st = status_from_hip(hipGetLastError()))) return st;
-    const int n_rows = n_views * g->nv;
+    float* hs = (float*)(tw + N);
     const double R = g->sad;
     const double mag = g->sad / g->sdd;  // R / (R + D)
     const double tau = g->du * mag;
-    const dim3 grid((n_rows + 1) / 2);
+    hipLaunchKernelGGL(twiddle_kernel, dim3((N + 255) / 256), dim3(256), 0, s, tw, hs, spectrum, tau / N, N, l2);
+    if ((st = status_from_hip(hipGetLastError()))) return st;
+    const int n_rows = n_views * g->nv;
     return status_from_hip(launch_filter<3>(
-        l2, grid, s, proj_in, proj_out, spectrum, tw, n_rows, g->nu, g->nv, (float)R,
+        l2, s, proj_in, proj_out, hs, tw, n_rows, g->nu, g->nv, (float)R,
         (float)(g->du * mag), (float)(g->det_offset[0] * mag), (float)(g->dv * mag),
-        (float)(g->det_offset[1] * mag), (float)(tau / N), 0));
+        (float)(g->det_offset[1] * mag), 0));
 }
 
 int ctr_pixel_filter_spectrum(int n_fft, double tau, int filter_type, double cutoff,
@@ -3175,16 +3252,15 @@ int ctr_pixel_filter(const ctr_geometry* g, const double* spectrum, const float*
     if (workspace_bytes < ctr_fdk_filter_workspace_bytes(g)) return CTR_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     float2* tw = (float2*)workspace;
-    hipLaunchKernelGGL(twiddle_kernel, dim3((N + 255) / 256), dim3(256), 0, s, tw, N, l2);
+    float* hs = (float*)(tw + N);
+    hipLaunchKernelGGL(twiddle_kernel, dim3((N + 255) / 256), dim3(256), 0, s, tw, hs, spectrum, 1.0 / N, N, l2);
     if ((st = status_from_hip(hipGetLastError()))) return st;
     const int n_rows = n_views * g->nv;
     const double mag = g->sad / g->sdd;
     const double su = g->du * mag, sv = g->dv * mag;
-    const dim3 grid((n_rows + 1) / 2);
-    return status_from_hip(launch_filter<3>(l2, grid, s, proj_in, q_out, spectrum, tw, n_rows,
+    return status_from_hip(launch_filter<3>(l2, s, proj_in, q_out, hs, tw, n_rows,
                                             g->nu, g->nv, (float)g->sad, (float)su,
-                                            (float)(0.5 * su), (float)sv, (float)(-0.5 * sv),
-                                            (float)(1.0 / N), 1));
+                                            (float)(0.5 * su), (float)sv, (float)(-0.5 * sv), 1));
 }
 
 size_t ctr_dd_backproject_workspace_bytes(const ctr_geometry* g, int mode) {
