@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <type_traits>
 
 #include "ctrecon.h"
 #include "splits.h"
@@ -281,18 +282,38 @@ __global__ void __launch_bounds__(kPxThreads) pixel_backproject_kernel(
         const float fvb_c = in_win ? fvb : wr0;
         const int cu = min(max(iu - w.c0, 0), w.cols - 2);
         const float* base = buf + cu - w.r0 * kPxPitch;
+        // fv(k) is monotone in k: both ends on the detector put every sample of the column there.  Where
+        // that holds for a wavefront's columns (all but the tiles whose samples leave the detector) the
+        // row test is left out: 11 instead of 13 VALU instructions per voxel.  Measured: 512^3 x 680 views
+        // 34.0 -> 32.9 ms, 160 x 160 x 120 x 200 views 444 -> 339 us.  The two loops stand in two ifs, not
+        // in an if and its else: merging their accumulators cost a copy of each (32 registers, and two of
+        // the six wavefronts per SIMD).
+        const float f_last_c = fmaf((float)(TZ - 1), kz_c, fvb_c);
+        const bool on_det = wc == 0.0f || (px_row_ok(fvb_c, vlast_bits) && px_row_ok(f_last_c, vlast_bits));
+        auto column = [&](auto checked, const float* win_at, float f0, float step) {
 #pragma unroll
-        for (int k = 0; k < TZ; ++k) {
-            const float fv = fmaf((float)k, kz_c, fvb_c);
-            const int iv = (int)floorf(fv);
-            const float fy = __builtin_amdgcn_fractf(fv);
-            const float* p = base + __mul24(iv, kPxPitch);
-            const float q00 = p[0], q01 = p[1], q10 = p[kPxPitch], q11 = p[kPxPitch + 1];
-            const float m0 = fmaf(fx, q01 - q00, q00);
-            const float m1 = fmaf(fx, q11 - q10, q10);
-            const float val = fmaf(fy, m1 - m0, m0);
-            const float wk = px_row_ok(fv, vlast_bits) ? wc : 0.0f;
-            acc[k] = fmaf(val, wk, acc[k]);
+            for (int k = 0; k < TZ; ++k) {
+                const float fv = fmaf((float)k, step, f0);
+                const int iv = (int)floorf(fv);
+                const float fy = __builtin_amdgcn_fractf(fv);
+                const float* p = win_at + __mul24(iv, kPxPitch);
+                const float q00 = p[0], q01 = p[1], q10 = p[kPxPitch], q11 = p[kPxPitch + 1];
+                const float m0 = fmaf(fx, q01 - q00, q00);
+                const float m1 = fmaf(fx, q11 - q10, q10);
+                const float val = fmaf(fy, m1 - m0, m0);
+                const float wk = !decltype(checked)::value || px_row_ok(fv, vlast_bits) ? wc : 0.0f;
+                acc[k] = fmaf(val, wk, acc[k]);
+            }
+        };
+        int whole = __builtin_amdgcn_readfirstlane(__ballot(!on_det) == 0 ? 1 : 0);
+        if (whole) column(std::false_type{}, base, fvb_c, kz_c);
+        whole = __builtin_amdgcn_readfirstlane(whole);
+        asm volatile("" : "+s"(whole));
+        if (!whole) {
+            // opaque copies: keep the two loops' samples from being computed before the branch
+            float f0 = fvb_c, step = kz_c;
+            asm volatile("" : "+v"(f0), "+v"(step));
+            column(std::true_type{}, base, f0, step);
         }
     }
 
