@@ -339,7 +339,11 @@ __device__ inline int quad_max(int v) {
 // per (slab, column, view) record of a batch: packed flags (see below) and the weights
 constexpr int kRecHit = 1 << 10;
 
-__global__ void __launch_bounds__(64 * kFpWaves, CTR_FP_MIN_WAVES) dd_forward_kernel(
+// SPLIT wavefronts share the slabs of a column group: wavefront kFpWaves s + w of a workgroup walks the
+// s-th share of the slabs for column group w, and the first share's wavefront adds up the others' sums
+// (in LDS, in share order) before it forms its rows.
+template <int SPLIT>
+__global__ void __launch_bounds__(64 * kFpWaves * SPLIT, CTR_FP_MIN_WAVES) dd_forward_kernel(
     const float* __restrict__ t_ys, const float* __restrict__ t_xs, float* __restrict__ proj,
     const float* __restrict__ tabs, const float* __restrict__ rows,
     const int32_t* __restrict__ branch, int nx, int ny, int nz, int nzp, int nu, int nv, int stride,
@@ -362,7 +366,8 @@ __global__ void __launch_bounds__(64 * kFpWaves, CTR_FP_MIN_WAVES) dd_forward_ke
     const int lane = threadIdx.x & 63;
     // wave-uniform: lets the compiler keep column data and addresses in scalar registers
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int j0 = (cg * kFpWaves + wave) * kFpCols;  // first column of this wavefront
+    const int share = SPLIT == 1 ? 0 : wave / kFpWaves;  // of the slabs
+    const int j0 = (cg * kFpWaves + wave % kFpWaves) * kFpCols;  // first column of this wavefront
     // a wavefront whose columns are all past the detector has no work but stays for the
     // workgroup's final barrier
     const bool live = j0 < nu;
@@ -378,7 +383,7 @@ __global__ void __launch_bounds__(64 * kFpWaves, CTR_FP_MIN_WAVES) dd_forward_ke
         const bool present = view0 + v < n_views;
         br[v] = present ? branch[view0 + v] : -1;
         use[v] = br[v] == CTR_BRANCH_X || br[v] == CTR_BRANCH_Y;
-        if (present && !use[v] && active) {
+        if (present && !use[v] && active && share == 0) {
             float* o = proj + ((size_t)(view0 + v) * nv + kk) * nu + j0;
 #pragma unroll
             for (int c = 0; c < kFpCols; ++c)
@@ -438,8 +443,8 @@ __global__ void __launch_bounds__(64 * kFpWaves, CTR_FP_MIN_WAVES) dd_forward_ke
         for (int c = 0; c < kFpCols; ++c) H[v][c] = 0.0;
     // two segment buffers per wavefront: a pair of slabs is loaded straight into LDS
     // (buffer_load ... lds: no VGPRs, no ds_write) while nothing of the pair is read yet
-    __shared__ uint4 segs[kFpWaves][2][kFpMaxQuads];
-    __shared__ float4 recs[kFpWaves][kFpViews][64];
+    __shared__ uint4 segs[kFpWaves * SPLIT][2][kFpMaxQuads];
+    __shared__ float4 recs[kFpWaves * SPLIT][kFpViews][64];
     const char* segs_bytes = reinterpret_cast<const char*>(&segs[0][0][0]);
     const int seg_off = wave * 2 * kFpMaxQuads * 16;  // this wavefront's segment buffers in segs
     // lanes g = 64 i + lane of segment load i: (g + 1/2) as a float, for the line index
@@ -476,8 +481,10 @@ __global__ void __launch_bounds__(64 * kFpWaves, CTR_FP_MIN_WAVES) dd_forward_ke
             const float zmin = fminf(fminf(z1, z2), fminf(z3, z4)), zmax = fmaxf(fmaxf(z1, z2), fmaxf(z3, z4));
             may_hit |= col_ok && hi >= -1.0f && lo <= fnt + 1.0f && zmax >= -1.0f && zmin <= fnz + 1.0f;
         }
-        const int n_end = __ballot(may_hit) ? ns : 0;
-        for (int n0 = 0; n0 < n_end; n0 += kFpBatch) {
+        // this share's slabs, in whole batches
+        const int per = SPLIT == 1 ? ns : ((ns + SPLIT - 1) / SPLIT + kFpBatch - 1) / kFpBatch * kFpBatch;
+        const int n_end = __ballot(may_hit) ? min((share + 1) * per, ns) : 0;
+        for (int n0 = share * per; n0 < n_end; n0 += kFpBatch) {
             // the batch's slabs through one buffer resource: a line is addressed by a scalar byte
             // offset, the lane's quad by a vector one
             const char* batch = src_bytes + (size_t)n0 * slab_bytes;
@@ -722,12 +729,32 @@ __global__ void __launch_bounds__(64 * kFpWaves, CTR_FP_MIN_WAVES) dd_forward_ke
     // ([view][row][column]), and after one barrier the workgroup writes each row's 16 columns as
     // one 64-byte run, so that no cache line is written back in pieces by wavefronts that finish
     // at different times.
+    if constexpr (SPLIT > 1) {
+        static_assert(sizeof(double) * kFpViews * kFpCols * 64 <= sizeof(uint4) * 2 * kFpMaxQuads, "sums fit the buffers");
+        if (share) {
+            double* sums = reinterpret_cast<double*>(&segs[wave][0][0]);
+#pragma unroll
+            for (int v = 0; v < kFpViews; ++v)
+#pragma unroll
+                for (int c = 0; c < kFpCols; ++c) sums[(v * kFpCols + c) * 64 + lane] = H[v][c];
+        }
+        __syncthreads();
+        if (share == 0) {
+            for (int q = 1; q < SPLIT; ++q) {
+                const double* sums = reinterpret_cast<const double*>(&segs[kFpWaves * q + wave][0][0]);
+#pragma unroll
+                for (int v = 0; v < kFpViews; ++v)
+#pragma unroll
+                    for (int c = 0; c < kFpCols; ++c) H[v][c] += sums[(v * kFpCols + c) * 64 + lane];
+            }
+        }
+    }
     const float vc = rows[nv + 1 + kk];
     const float dnu = rows[kk + 1] - rows[kk];
     float4* __restrict__ stage = reinterpret_cast<float4*>(&segs[wave][0][0]);
 #pragma unroll
     for (int v = 0; v < kFpViews; ++v) {
-        if (!use[v]) continue;
+        if (!use[v] || share) continue;
         float res[kFpCols];
 #pragma unroll
         for (int c = 0; c < kFpCols; ++c) {
@@ -744,7 +771,7 @@ __global__ void __launch_bounds__(64 * kFpWaves, CTR_FP_MIN_WAVES) dd_forward_ke
     // the wavefronts of one row
     const int jw = cg * kFpWaves * kFpCols;  // the workgroup's first column
     const bool vec_ok = (nu & 3) == 0 && (reinterpret_cast<uintptr_t>(proj) & 15) == 0;
-    for (int it = threadIdx.x; it < kFpViews * kColRows * kFpWaves; it += 64 * kFpWaves) {
+    for (int it = threadIdx.x; it < kFpViews * kColRows * kFpWaves; it += 64 * kFpWaves * SPLIT) {
         const int q = it % kFpWaves;
         const int r = (it / kFpWaves) % kColRows;
         const int v = it / (kFpWaves * kColRows);
@@ -2705,20 +2732,36 @@ hipError_t launch_filter(int l2, hipStream_t st, const float* in, float* out,
 // 240 us; 256 x 256 x 200 x 120 views of 420 rows 4.69 -> 4.00, 1847 -> 1688 us; 128^3 x 180 views of
 // 256 rows 3.25 -> 3.00, 505 -> 472 us.  512^3 x 720 views of 768 rows (8.31, at best 8.25) is left
 // alone: shifted so that its largest shadow starts a block it has 8.50 and ran 1.8 % slower.
-int fp_row_shift(const ctr_geometry* g) {
+//
+// Slabs are shared out (dd_forward_kernel's SPLIT) where the groups that the shadow gives work to are
+// too few for the four that every CU holds: one group's serial walk over the slabs then decides.
+// Measured with 1, 2 and 4 shares, by those groups: 83 groups 68, 44, 39 us; 135 groups 93, 61, 58 us;
+// 209 groups 63, 53, 59 us; 631 groups 91, 84, 107 us; 338 groups of 44 slabs 59, 67, 73 us (shares
+// are whole batches of 16 slabs); 2430 groups 470, 573, 785 us.  At a coarse angular step, where a
+// group walks the slabs once per view, two shares also pay with more groups (256^3 x 60 views, 1810
+// groups: 1030, 970, 1210 us; 2084 groups: 602, 612, 818 us).
+struct FpPlan {
+    int row_shift, split;
+};
+
+FpPlan fp_plan(const ctr_geometry* g) {
     constexpr int kDistances = 16;
     const double reach = 0.5 * std::max(g->nx * g->dx + 2.0 * fabs(g->recon_center[0]),
                                         g->ny * g->dy + 2.0 * fabs(g->recon_center[1]));
-    if (g->helical != 0.0 || !(g->sad > reach)) return 0;
-    const double z_mid = g->recon_center[2] - g->source_init[2], z_half = 0.5 * g->nz * g->dz;
+    if (!(g->sad > reach)) return {0, 1};
+    // a helix passes the volume at every height: at its middle, for the count of groups
+    const double z_mid = g->helical != 0.0 ? 0.0 : g->recon_center[2] - g->source_init[2], z_half = 0.5 * g->nz * g->dz;
     const double half = (g->detector_shape == CTR_DETECTOR_FLAT) ? 0.5 * g->dv : -0.5 * g->dv;
     const double centre = (g->nv - 1) / 2.0 + (half + g->det_offset[1]) / g->dv;  // edge index at height 0
+    const double width = 1.25 * std::max(g->nx * g->dx, g->ny * g->dy);  // of a square seen from any side
     int first[kDistances], last[kDistances];  // rows of the shadow
+    double columns = 0.0;                     // its mean width
     for (int k = 0; k < kDistances; ++k) {
         const double rows = g->sdd / (g->sad + ((2 * k + 1.0) / kDistances - 1.0) * reach) / g->dv;
         auto row = [&](double e) { return (int)std::min(std::max(e, 0.0), (double)g->nv); };
         first[k] = row(floor(centre - (z_mid + z_half) * rows));
         last[k] = row(ceil(centre - (z_mid - z_half) * rows)) - 1;
+        columns += std::min((double)g->nu, width * rows * g->dv / g->du) / kDistances;
     }
     int best = 0, fewest = 0, unshifted = 0;
     for (int shift = 0; shift < kColRows; ++shift) {
@@ -2731,7 +2774,17 @@ int fp_row_shift(const ctr_geometry* g) {
             fewest = touched;
         }
     }
-    return fewest <= 0.97 * unshifted ? best : 0;
+    FpPlan p = {g->helical == 0.0 && fewest <= 0.97 * unshifted ? best : 0, 1};
+    const double touched = (double)(p.row_shift ? fewest : unshifted) / kDistances;
+    const double groups = touched * columns / (kFpCols * kFpWaves) * ((g->n_views + 1) / 2);
+    const int slabs = std::max(g->nx, g->ny);
+    // a full turn moves the outermost lines of adjacent views by this much
+    const bool coarse = kPi * slabs / g->n_views > kFpPairShift;
+    if (groups <= 150 && slabs >= 2 * kFpBatch)
+        p.split = 4;
+    else if (groups <= 256 || (slabs >= 56 && groups <= (coarse ? 1900 : 700)))
+        p.split = 2;
+    return p;
 }
 
 // Scratch memory of ctr_dd_backproject_static, for callers that cannot allocate: the FDK
@@ -3149,16 +3202,21 @@ int ctr_dd_forward(const ctr_geometry* g, const double* angles, const int32_t* b
             g->nv == 3 ? launch(dd_forward_thin_kernel<4, false>) : launch(dd_forward_thin_kernel<5, false>);
     } else {
         const int col_groups = (g->nu + kFpCols * kFpWaves - 1) / (kFpCols * kFpWaves);
-        const int row_shift = fp_row_shift(g);
-        const int row_blocks = (g->nv + row_shift + kColRows - 1) / kColRows;
+        const FpPlan plan = fp_plan(g);
+        const int row_blocks = (g->nv + plan.row_shift + kColRows - 1) / kColRows;
         const int n_pairs = (g->n_views + kFpViews - 1) / kFpViews;
         const int n_vblocks = (n_pairs + kViewBlock - 1) / kViewBlock;
         const long long n_blocks =
             8LL * ((col_groups + 7) / 8) * row_blocks * n_vblocks * kViewBlock;
         if (n_blocks >= 2147483647LL) return CTR_ERR_INVALID;
-        hipLaunchKernelGGL(dd_forward_kernel, dim3((unsigned)n_blocks), dim3(64 * kFpWaves), 0, s, t_ys, t_xs,
-                           proj, tabs, rows, branch, g->nx, g->ny, g->nz, nzp, g->nu, g->nv, stride, 1e-6f,
-                           g->n_views, col_groups, n_vblocks, row_shift);
+        auto launch = [&](auto kernel, int split) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)n_blocks), dim3(64 * kFpWaves * split), 0, s, t_ys, t_xs, proj, tabs,
+                               rows, branch, g->nx, g->ny, g->nz, nzp, g->nu, g->nv, stride, 1e-6f, g->n_views, col_groups,
+                               n_vblocks, plan.row_shift);
+        };
+        plan.split == 1   ? launch(dd_forward_kernel<1>, 1)
+        : plan.split == 2 ? launch(dd_forward_kernel<2>, 2)
+                          : launch(dd_forward_kernel<4>, 4);
     }
     if ((st = status_from_hip(hipGetLastError()))) return st;
     // z-slab views (left at zero above): their own kernel, which returns at once for the others

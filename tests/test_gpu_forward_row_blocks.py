@@ -44,3 +44,20 @@ def test_rows_of_steep_views():
     ref = O.forward_project(g, vol)
     out = ctr.dd_forward(torch.from_numpy(vol).cuda(), ctr.ScanGeometry(p)).cpu().numpy()
     assert np.abs(out - ref).max() <= TOL * np.abs(ref).max()
+
+
+# one, two and four shares of the slabs per column group, with fewer slabs than a share holds, a coarse
+# and a fine angular step, columns off the volume, both slab orientations
+@pytest.mark.parametrize("nx,ny,views,nu", [(20, 33, 5, 20), (34, 31, 40, 40), (70, 64, 61, 100), (60, 66, 220, 70)])
+def test_slab_shares_match_the_oracle(nx, ny, views, nu):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    N.lib()
+    p = make_params(NumberOfImage=[nx, ny, 6], NumberOfDetectorPixels=[nu, 12], NumberOfViews=views, StartAngle=0.02,
+                    EndAngle=0.02 + 2 * np.pi)
+    g = O.Geometry(p)
+    vol = np.random.default_rng(nx).random((g.nz, g.ny, g.nx)).astype(np.float32)
+    keep = list(range(0, views, max(1, views // 12)))
+    ref = O.forward_project(g, vol, views=keep)
+    out = ctr.dd_forward(torch.from_numpy(vol).cuda(), ctr.ScanGeometry(p)).cpu().numpy()[keep]
+    assert np.abs(out - ref).max() <= TOL * np.abs(ref).max()
