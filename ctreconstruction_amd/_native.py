@@ -17,7 +17,8 @@ REPO_DIR = os.path.dirname(PKG_DIR)
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libctrecon.so")
 SOURCES = [os.path.join(PKG_DIR, "csrc", "ctrecon.hip"), os.path.join(PKG_DIR, "csrc", "prior.hip"),
-           os.path.join(PKG_DIR, "csrc", "pixel.hip"), os.path.join(PKG_DIR, "csrc", "tv.hip")]
+           os.path.join(PKG_DIR, "csrc", "pixel.hip"), os.path.join(PKG_DIR, "csrc", "tv.hip"),
+           os.path.join(PKG_DIR, "csrc", "iterate.hip")]
 INCLUDE_DIR = os.path.join(REPO_DIR, "include")
 # instruction-issue microbenchmarks for bench.py --calibrate-valu (not part of the product ABI)
 CALIB_PATH = os.path.join(LIB_DIR, "libctrcalib.so")
@@ -31,7 +32,7 @@ EXPORTS = (
     "ctr_dd_backproject_workspace_bytes", "ctr_dd_backproject", "ctr_dd_backproject_static",
     "ctr_pixel_filter_spectrum", "ctr_pixel_filter",
     "ctr_pixel_backproject_workspace_bytes", "ctr_pixel_backproject",
-    "ctr_tv_workspace_bytes", "ctr_tv_gradient", "ctr_tv_descent",
+    "ctr_tv_workspace_bytes", "ctr_tv_gradient", "ctr_tv_descent", "ctr_residual", "ctr_update",
     "ctr_conv3x3_bf16_forward", "ctr_conv3x3_bf16_wgrad_workspace_bytes", "ctr_conv3x3_bf16_wgrad",
     "ctr_conv3x3_bf16_backward_workspace_bytes", "ctr_conv3x3_bf16_backward",
 )
@@ -129,6 +130,8 @@ def _declare(lib):
         "ctr_pixel_filter": (c_int, [gp, c_vp, c_vp, c_vp, c_int, c_vp, c_size, c_vp]),
         "ctr_pixel_backproject_workspace_bytes": (c_size, [gp]),
         "ctr_pixel_backproject": (c_int, [gp, c_vp, c_vp, c_vp, c_flt, c_int, c_vp, c_size, c_vp]),
+        "ctr_residual": (c_int, [c_vp, c_vp, c_vp, c_vp, c_size, c_int, c_int, c_flt, c_vp]),
+        "ctr_update": (c_int, [c_vp, c_vp, c_vp, c_vp, c_size, c_int, c_flt, c_flt, c_int, c_int, c_vp]),
         "ctr_tv_workspace_bytes": (c_size, [c_int, c_int, c_int, c_int, c_int]),
         "ctr_tv_gradient": (c_int, [c_vp, c_vp, c_int, c_int, c_int, c_int, c_flt, c_vp, c_size, c_vp]),
         "ctr_tv_descent": (c_int, [c_vp, c_vp, c_vp, c_int, c_int, c_int, c_int, c_flt, c_int, c_vp, c_size, c_vp]),

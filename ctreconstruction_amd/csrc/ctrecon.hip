@@ -3121,7 +3121,7 @@ const char* ctr_strerror(int code) {
         case CTR_ERR_HIP: return "HIP runtime error";
         case CTR_ERR_SCRATCH:
             return "problem too large for the static scratch of ctr_dd_backproject_static (32 MiB: "
-                   "64 bytes per view plus one byte per 16x16x16 voxel tile and view)";
+                   "64 bytes per view plus one byte per 16x16x32 voxel tile and view)";
         default: return "unknown error";
     }
 }

@@ -8,8 +8,8 @@ Two backprojectors are available:
   and the reference's placement of eps.
 * ``"matched"`` — the update is the gradient of the weighted least-squares data term
   ``0.5 * sum W (A x - p)^2`` with W = 1/(A 1 + eps), taken by torch autograd through
-  :class:`DDProjectorFunction`, whose backward is the matched backprojector A^T; it is scaled
-  by 1/(A^T 1 + eps) (the SART normalisation).
+  :class:`DDProjectorFunction`, whose backward applies the matched backprojector A^T to
+  W (A x - p); it is scaled by 1/(A^T 1 + eps) (the SART normalisation).
 
 ``tv_gradient`` is the normalised total-variation gradient of python/ASD_POCS.py:55-77;
 ``tv_gradient_autograd`` obtains the same vector by differentiating the TV functional.
@@ -99,16 +99,15 @@ def sart(proj0: torch.Tensor, geom: ScanGeometry, n_iter: int, relaxation: float
                      device=proj0.device) if x0 is None else x0.detach().clone())
     for it in range(n_iter):
         if backprojector == "matched":
+            # the gradient of 0.5 sum w (A x - p)^2: the projector's backward of w (A x - p)
             xv = x.detach().requires_grad_(True)
-            r = DDProjectorFunction.apply(xv, geom) - proj0
-            loss = 0.5 * (w * r * r).sum()
-            (grad,) = torch.autograd.grad(loss, xv)
-            step = -grad
+            ax = DDProjectorFunction.apply(xv, geom)
+            r = _residual(proj0, ax.detach(), w, weighted=True).sum_to_size(ax.shape).to(ax.dtype)
+            (grad,) = torch.autograd.grad(ax, xv, r)
+            x = _update(x.detach(), grad, b1, -relaxation, eps, False, nonneg)
         else:
             step = _bp_ref((proj0 - forward_batch(x, geom)) * w, geom, "edge" if backprojector == "edge" else "ref")
-        x = x.detach() + relaxation * step / (b1 + eps)
-        if nonneg:
-            x = torch.clamp_min(x, 0.0)
+            x = _update(x.detach(), step, b1, relaxation, eps, False, nonneg)
         if callback is not None:
             callback(it, x)
     return x.detach()
@@ -141,14 +140,12 @@ def _normalise_pad(dtv: torch.Tensor, eps: float) -> torch.Tensor:
     return torch.nn.functional.pad(dtv / norm, (1, 1, 1, 1, 1, 1))
 
 
-def _on_tv_kernels(img: torch.Tensor, eps: float) -> bool:
-    """Whether the TV kernels take ``img``: plain contiguous float32 volumes on the GPU that nothing
-    differentiates, maps or traces (the torch expressions serve everything else)."""
+def _plain(img: torch.Tensor) -> bool:
+    """Whether a kernel may take ``img``: a contiguous float32 batch of volumes (or projections) on the
+    GPU that nothing differentiates, maps or traces (the torch expressions serve everything else)."""
     if type(img) is not torch.Tensor or img.device.type != "cuda" or img.dtype != torch.float32:
         return False
-    if img.dim() < 3 or min(img.shape[-3:]) < 3 or not img.is_contiguous() or img.numel() == 0 or not eps > 0:
-        return False
-    if img.shape[-3:].numel() >= 2 ** 31 - 1 or img.shape[:-3].numel() > 65535:
+    if img.dim() < 3 or not img.is_contiguous() or img.numel() == 0 or img.shape[:-3].numel() > 65535:
         return False
     if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or torch.overrides._get_current_function_mode_stack() \
             or torch.utils._python_dispatch._get_current_dispatch_mode() is not None:
@@ -157,6 +154,44 @@ def _on_tv_kernels(img: torch.Tensor, eps: float) -> bool:
             torch.autograd.forward_ad.unpack_dual(img).tangent is not None:
         return False
     return not (torch.is_grad_enabled() and img.requires_grad)
+
+
+def _on_tv_kernels(img: torch.Tensor, eps: float) -> bool:
+    """Whether the TV kernels take ``img``."""
+    return (_plain(img) and min(img.shape[-3:]) >= 3 and img.shape[-3:].numel() < 2 ** 31 - 1 and eps > 0)
+
+
+def _elementwise(x: torch.Tensor, y: torch.Tensor, per_geom: torch.Tensor, *scalars) -> bool:
+    """Whether the residual and update kernels take (x, y) with ``per_geom`` for every item: no
+    broadcasting but that, and plain numbers as scalars."""
+    return (all(isinstance(s, (int, float)) for s in scalars) and per_geom.numel() <= 0xffffff00 and _plain(x) and _plain(y) and _plain(per_geom) and x.shape == y.shape and x.shape[-3:] == per_geom.shape
+            and x.device == y.device == per_geom.device)
+
+
+def _residual(p, ax, a, weighted: bool, eps: float = 0.0):
+    """weighted: a (ax - p); else (p - ax) / (a + eps), 0 where a is 0."""
+    if _elementwise(p, ax, a, eps):
+        out = torch.empty_like(ax)
+        N.check(N.lib().ctr_residual(P._ptr(p), P._ptr(ax), P._ptr(a), P._ptr(out), a.numel(), p.numel() // a.numel(),
+                                     int(weighted), float(eps), P._stream(p.device)), "ctr_residual")
+        return out
+    if weighted:
+        return a * (ax - p)
+    r = (p - ax) / (a + eps)
+    return torch.where(a == 0, torch.zeros_like(r), r)
+
+
+def _update(x, u, b, relax: float, eps: float, masked: bool, nonneg: bool):
+    """x + relax u / (b + eps); masked: u counts as 0 where b is 0; nonneg: clamped at 0."""
+    if _elementwise(x, u, b, relax, eps):
+        out = torch.empty_like(x)
+        N.check(N.lib().ctr_update(P._ptr(x), P._ptr(u), P._ptr(b), P._ptr(out), b.numel(), x.numel() // b.numel(),
+                                   float(relax), float(eps), int(masked), int(nonneg), P._stream(x.device)), "ctr_update")
+        return out
+    if masked:
+        u = torch.where(b == 0, torch.zeros_like(u), u)
+    x = x + relax * u / (b + eps)
+    return torch.clamp_min(x, 0.0) if nonneg else x
 
 
 def _tv_call(fn, img, out, eps, steps, *args):
@@ -227,11 +262,8 @@ def asd_pocs(proj0: torch.Tensor, geom: ScanGeometry, n_outer: int = 20, na: int
     for it in range(n_outer):
         f0 = x.clone()
         for _ in range(na):
-            r = (proj0 - forward_batch(x, geom)) / (a1 + eps)
-            r = torch.where(a1 == 0, torch.zeros_like(r), r)
-            upd = bp(r)
-            upd = torch.where(b1 == 0, torch.zeros_like(upd), upd)
-            x = torch.clamp_min(x + beta * upd / (b1 + eps), 0.0)
+            upd = bp(_residual(proj0, forward_batch(x, geom), a1, weighted=False, eps=eps))
+            x = _update(x, upd, b1, beta, eps, True, True)
         dp = dist(x, f0)
         dtvg = alpha * dp
         f0 = x.clone()

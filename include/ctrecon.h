@@ -201,6 +201,17 @@ int ctr_tv_gradient(const float* x, float* grad, int batch, int nx, int ny, int 
 int ctr_tv_descent(const float* x, float* out, const float* step, int batch, int nx, int ny, int nz,
                    float eps, int steps, void* workspace, size_t workspace_bytes, void* stream);
 
+/* ---- Elementwise parts of SART and ASD-POCS iterations -----------------------------------
+ * (python/SART.py:44-59, python/ASD_POCS.py:170-186), one pass each over a batch; `a` and `b` hold
+ * n values that serve every item of the batch, the other arrays batch * n.
+ * ctr_residual: out = weighted ? a (ax - p) : (a == 0 ? 0 : (p - ax) / (a + eps)).
+ * ctr_update: out = x + relax u / (b + eps); masked: u counts as 0 where b == 0; nonneg: negative
+ * results become 0. */
+int ctr_residual(const float* p, const float* ax, const float* a, float* out, size_t n, int batch,
+                 int weighted, float eps, void* stream);
+int ctr_update(const float* x, const float* u, const float* b, float* out, size_t n, int batch,
+               float relax, float eps, int masked, int nonneg, void* stream);
+
 /* ---- Learned prior: 3x3 convolutions, bfloat16 on MFMA, FP32 accumulation ---------------
  * No counterpart in the reference (the reference has no learned prior).
  * Activations are NHWC bfloat16 [n][h][w][c]; weights bfloat16 [cout][3][3][cin]; bias float32.
