@@ -4,8 +4,8 @@
 hand-written matched backprojector A^T (``ctr_dd_backproject`` in adjoint mode), so gradients
 of any loss of A x flow through the project's own kernels.  ``DDBackprojectorFunction`` is the
 transpose pair (y -> A^T y, backward A).  Both accept one volume [nz, ny, nx] or a batch
-[B, nz, ny, nx] (projections [nView, nv, nu] or [B, nView, nv, nu]); a batch is processed one
-item at a time on the current stream.
+[B, nz, ny, nx] (projections [nView, nv, nu] or [B, nView, nv, nu]); on the current stream, the
+volumes of a batch are projected together and its projections backprojected one item at a time.
 """
 from __future__ import annotations
 
@@ -28,6 +28,8 @@ def _batched(fn, x: torch.Tensor, item_shape, out_shape, geom):
 
 
 def forward_batch(vol: torch.Tensor, geom: ScanGeometry) -> torch.Tensor:
+    if vol.dim() == 4 and tuple(vol.shape[1:]) == tuple(geom.vol_shape):
+        return P.dd_forward_batch(vol.contiguous(), geom)
     return _batched(P.dd_forward, vol, geom.vol_shape, geom.proj_shape, geom)
 
 

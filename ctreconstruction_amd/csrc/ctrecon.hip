@@ -90,7 +90,8 @@ int zprefix_stride(int nz) { return (nz + 2 + 3) & ~3; }
 
 // workspace: tables, row table, then the z-prefix tables of the volume (k fastest) twice:
 // [y][x][k] (gathered by y-slab views) and [x][y][k] (x-slab views)
-FpLayout fp_layout(const ctr_geometry* g) {
+// (one pair of tables per volume of a batch)
+FpLayout fp_layout(const ctr_geometry* g, int batch) {
     FpLayout L;
     // + 1024: a staged segment (up to 168 breakpoints) may read past the end of the last line
     const size_t vbytes = align_up((size_t)g->nx * g->ny * zprefix_stride(g->nz) * sizeof(float) + 1024, 256);
@@ -98,7 +99,7 @@ FpLayout fp_layout(const ctr_geometry* g) {
     L.rows_off = align_up(L.tabs_off + (size_t)fp_view_stride(g->nu) * g->n_views * 4, 256);
     L.volt_off = align_up(L.rows_off + (size_t)(2 * g->nv + 1) * 4, 256);
     L.copy_bytes = vbytes;
-    L.total = L.volt_off + 2 * vbytes;
+    L.total = L.volt_off + 2 * vbytes * batch;
     return L;
 }
 
@@ -238,16 +239,18 @@ __device__ inline void zprefix(const float* __restrict__ in, float* __restrict__
 
 // The forward projector's preparation in one launch: the first workgroups build the z-prefix tables,
 // the others the footprint tables.  Neither needs the other, and for a small scan each would be a
-// launch of a few microseconds.
+// launch of a few microseconds.  blockIdx.y is the volume of a batch (item_stride: floats between the
+// tables of consecutive volumes); the footprint tables serve all of them.
 __global__ void __launch_bounds__(256) fp_prepare_kernel(ctr_geometry g, const double* __restrict__ angles,
                                                          const int32_t* __restrict__ branch, float* __restrict__ tabs,
                                                          float* __restrict__ rows, int stride, int geo_groups,
                                                          const float* __restrict__ vol, float* __restrict__ t_ys,
-                                                         float* __restrict__ t_xs, int nzp) {
+                                                         float* __restrict__ t_xs, int nzp, size_t item_stride) {
     const int zx = (g.nx + 31) / 32, zgroups = zx * g.ny, b = blockIdx.x;
     if (b < zgroups) {
-        zprefix(vol, t_ys, t_xs, g.nx, g.ny, g.nz, nzp, (b % zx) * 32, b / zx);
-    } else {
+        const size_t t = blockIdx.y * item_stride;
+        zprefix(vol + blockIdx.y * ((size_t)g.nx * g.ny * g.nz), t_ys + t, t_xs + t, g.nx, g.ny, g.nz, nzp, (b % zx) * 32, b / zx);
+    } else if (blockIdx.y == 0) {
         const int r = b - zgroups;
         fp_geometry(g, angles, branch, tabs, rows, stride, (r % geo_groups) * 256 + (int)threadIdx.x, r / geo_groups);
     }
@@ -347,7 +350,11 @@ __global__ void __launch_bounds__(64 * kFpWaves * SPLIT, CTR_FP_MIN_WAVES) dd_fo
     const float* __restrict__ t_ys, const float* __restrict__ t_xs, float* __restrict__ proj,
     const float* __restrict__ tabs, const float* __restrict__ rows,
     const int32_t* __restrict__ branch, int nx, int ny, int nz, int nzp, int nu, int nv, int stride,
-    float zero_tol, int n_views, int col_groups, int n_vblocks, int row_shift) {
+    float zero_tol, int n_views, int col_groups, int n_vblocks, int row_shift, size_t item_stride) {
+    // the volume of a batch
+    t_ys += blockIdx.y * item_stride;
+    t_xs += blockIdx.y * item_stride;
+    proj += blockIdx.y * ((size_t)n_views * nv * nu);
     // workgroup b runs on XCD b % 8, which takes the column groups cg = 8 c + xcd: every XCD
     // gets an equal share of every band of detector rows (the rows outside the volume's shadow
     // are cheap).  On one XCD the local index runs over (row block, view-pair block, c, pair in
@@ -811,8 +818,11 @@ template <int NE, bool ONE_Z>
 __global__ void __launch_bounds__(256) dd_forward_thin_kernel(
     const float* __restrict__ t_ys, const float* __restrict__ t_xs, float* __restrict__ proj,
     const float* __restrict__ tabs, const float* __restrict__ rows, const int32_t* __restrict__ branch, int nx, int ny,
-    int nz, int nzp, int nu, int nv, int stride, float zero_tol) {
+    int nz, int nzp, int nu, int nv, int stride, float zero_tol, size_t item_stride) {
     __shared__ double part[4][NE][64];
+    t_ys += blockIdx.z * item_stride;
+    t_xs += blockIdx.z * item_stride;
+    proj += blockIdx.z * ((size_t)gridDim.y * nv * nu);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int view = blockIdx.y, col = blockIdx.x * 64 + lane, j = min(col, nu - 1);
     const int br = branch[view];
@@ -932,6 +942,8 @@ __global__ void __launch_bounds__(256) dd_forward_zslab_kernel(ctr_geometry g, c
                                                                float* __restrict__ proj, double zero_tol) {
     const int view = blockIdx.y;
     if (branch[view] != CTR_BRANCH_Z) return;
+    vol += blockIdx.z * ((size_t)g.nx * g.ny * g.nz);
+    proj += blockIdx.z * ((size_t)g.n_views * g.nv * g.nu);
     const int nu = g.nu, nv = g.nv, nx = g.nx, ny = g.ny, nz = g.nz;
     const double th = angles[view];
     double s, c;
@@ -2740,11 +2752,16 @@ hipError_t launch_filter(int l2, hipStream_t st, const float* in, float* out,
 // are whole batches of 16 slabs); 2430 groups 470, 573, 785 us.  At a coarse angular step, where a
 // group walks the slabs once per view, two shares also pay with more groups (256^3 x 60 views, 1810
 // groups: 1030, 970, 1210 us; 2084 groups: 602, 612, 818 us).
+//
+// The volumes of a batch are projected by one launch: a 128^3 volume's 2430 groups leave the last wave
+// of the 1024 that run at once partly empty (eight of them at 180 views: 470 -> 392 us each), and small
+// volumes pay every launch once.
 struct FpPlan {
     int row_shift, split;
 };
+constexpr int kFpMaxBatch = 4096;
 
-FpPlan fp_plan(const ctr_geometry* g) {
+FpPlan fp_plan(const ctr_geometry* g, int batch) {
     constexpr int kDistances = 16;
     const double reach = 0.5 * std::max(g->nx * g->dx + 2.0 * fabs(g->recon_center[0]),
                                         g->ny * g->dy + 2.0 * fabs(g->recon_center[1]));
@@ -2776,7 +2793,7 @@ FpPlan fp_plan(const ctr_geometry* g) {
     }
     FpPlan p = {g->helical == 0.0 && fewest <= 0.97 * unshifted ? best : 0, 1};
     const double touched = (double)(p.row_shift ? fewest : unshifted) / kDistances;
-    const double groups = touched * columns / (kFpCols * kFpWaves) * ((g->n_views + 1) / 2);
+    const double groups = touched * columns / (kFpCols * kFpWaves) * ((g->n_views + 1) / 2) * batch;
     const int slabs = std::max(g->nx, g->ny);
     // a full turn moves the outermost lines of adjacent views by this much
     const bool coarse = kPi * slabs / g->n_views > kFpPairShift;
@@ -3158,17 +3175,28 @@ int ctr_zero_padded_length(int nu) {
 }
 
 size_t ctr_dd_forward_workspace_bytes(const ctr_geometry* g) {
-    if (check_geometry(g)) return 0;
-    return fp_layout(g).total;
+    return ctr_dd_forward_batch_workspace_bytes(g, 1);
+}
+
+size_t ctr_dd_forward_batch_workspace_bytes(const ctr_geometry* g, int batch) {
+    if (check_geometry(g) || batch < 1 || batch > kFpMaxBatch) return 0;
+    return fp_layout(g, batch).total;
 }
 
 int ctr_dd_forward(const ctr_geometry* g, const double* angles, const int32_t* branch,
                    const float* vol, float* proj, void* workspace, size_t workspace_bytes,
                    void* stream) {
+    return ctr_dd_forward_batch(g, angles, branch, vol, proj, 1, workspace, workspace_bytes, stream);
+}
+
+int ctr_dd_forward_batch(const ctr_geometry* g, const double* angles, const int32_t* branch,
+                         const float* vol, float* proj, int batch, void* workspace, size_t workspace_bytes,
+                         void* stream) {
     int st = check_geometry(g);
     if (st) return st;
-    if (!angles || !branch || !vol || !proj || !workspace) return CTR_ERR_INVALID;
-    const FpLayout L = fp_layout(g);
+    if (!angles || !branch || !vol || !proj || !workspace || batch < 1 || batch > kFpMaxBatch) return CTR_ERR_INVALID;
+    const FpLayout L = fp_layout(g, batch);
+    const size_t item_stride = 2 * L.copy_bytes / sizeof(float);
     if (workspace_bytes < L.total) return CTR_ERR_WORKSPACE;
     // the projector addresses a batch of 64 slabs of the z-prefix tables with 31-bit offsets
     if (64.0 * 4.0 * zprefix_stride(g->nz) * std::max(g->nx, g->ny) >= 2147483647.0)
@@ -3184,15 +3212,15 @@ int ctr_dd_forward(const ctr_geometry* g, const double* angles, const int32_t* b
     const int nzp = zprefix_stride(g->nz);
     const long long prep = (long long)((g->nx + 31) / 32) * g->ny + (long long)gx * g->n_views;
     if (prep >= 2147483647LL) return CTR_ERR_INVALID;
-    hipLaunchKernelGGL(fp_prepare_kernel, dim3((unsigned)prep), dim3(256), 0, s, *g, angles, branch, tabs, rows, stride, gx,
-                       vol, t_ys, t_xs, nzp);
+    hipLaunchKernelGGL(fp_prepare_kernel, dim3((unsigned)prep, batch), dim3(256), 0, s, *g, angles, branch, tabs, rows,
+                       stride, gx, vol, t_ys, t_xs, nzp, item_stride);
     if ((st = status_from_hip(hipGetLastError()))) return st;
     if (g->nv <= kThinRows) {
         static_assert(kThinRows == 4, "one wavefront per row");
-        const dim3 grid((g->nu + 63) / 64, g->n_views);
+        const dim3 grid((g->nu + 63) / 64, g->n_views, batch);
         auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, t_ys, t_xs, proj, tabs, rows, branch, g->nx, g->ny, g->nz,
-                               nzp, g->nu, g->nv, stride, 1e-6f);
+                               nzp, g->nu, g->nv, stride, 1e-6f, item_stride);
         };
         if (g->nz == 1)
             g->nv == 1 ? launch(dd_forward_thin_kernel<2, true>) : launch(dd_forward_thin_kernel<kThinRows + 1, true>);
@@ -3202,7 +3230,7 @@ int ctr_dd_forward(const ctr_geometry* g, const double* angles, const int32_t* b
             g->nv == 3 ? launch(dd_forward_thin_kernel<4, false>) : launch(dd_forward_thin_kernel<5, false>);
     } else {
         const int col_groups = (g->nu + kFpCols * kFpWaves - 1) / (kFpCols * kFpWaves);
-        const FpPlan plan = fp_plan(g);
+        const FpPlan plan = fp_plan(g, batch);
         const int row_blocks = (g->nv + plan.row_shift + kColRows - 1) / kColRows;
         const int n_pairs = (g->n_views + kFpViews - 1) / kFpViews;
         const int n_vblocks = (n_pairs + kViewBlock - 1) / kViewBlock;
@@ -3210,9 +3238,9 @@ int ctr_dd_forward(const ctr_geometry* g, const double* angles, const int32_t* b
             8LL * ((col_groups + 7) / 8) * row_blocks * n_vblocks * kViewBlock;
         if (n_blocks >= 2147483647LL) return CTR_ERR_INVALID;
         auto launch = [&](auto kernel, int split) {
-            hipLaunchKernelGGL(kernel, dim3((unsigned)n_blocks), dim3(64 * kFpWaves * split), 0, s, t_ys, t_xs, proj, tabs,
-                               rows, branch, g->nx, g->ny, g->nz, nzp, g->nu, g->nv, stride, 1e-6f, g->n_views, col_groups,
-                               n_vblocks, plan.row_shift);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)n_blocks, batch), dim3(64 * kFpWaves * split), 0, s, t_ys, t_xs, proj,
+                               tabs, rows, branch, g->nx, g->ny, g->nz, nzp, g->nu, g->nv, stride, 1e-6f, g->n_views, col_groups,
+                               n_vblocks, plan.row_shift, item_stride);
         };
         plan.split == 1   ? launch(dd_forward_kernel<1>, 1)
         : plan.split == 2 ? launch(dd_forward_kernel<2>, 2)
@@ -3220,7 +3248,7 @@ int ctr_dd_forward(const ctr_geometry* g, const double* angles, const int32_t* b
     }
     if ((st = status_from_hip(hipGetLastError()))) return st;
     // z-slab views (left at zero above): their own kernel, which returns at once for the others
-    hipLaunchKernelGGL(dd_forward_zslab_kernel, dim3(kZslabGroups, g->n_views), dim3(256), 0, s, *g, angles,
+    hipLaunchKernelGGL(dd_forward_zslab_kernel, dim3(kZslabGroups, g->n_views, batch), dim3(256), 0, s, *g, angles,
                        branch, vol, proj, 1e-6);
     return status_from_hip(hipGetLastError());
 }

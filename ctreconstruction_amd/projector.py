@@ -60,6 +60,35 @@ def dd_forward(vol: torch.Tensor, geom: ScanGeometry, out: torch.Tensor | None =
     return out
 
 
+# bytes of z-prefix tables that the volumes projected by one launch may take together: up to fifteen
+# 128^3 volumes share one (a forward and adjoint pass over 8 of them at 180 views 6.22 -> 5.59 ms),
+# and a volume from about 256^3 on has work enough alone
+_FORWARD_TABLES = 256 << 20
+
+
+def dd_forward_batch(vol: torch.Tensor, geom: ScanGeometry) -> torch.Tensor:
+    """:func:`dd_forward` of every volume of a batch [B, nz, ny, nx], several to a launch."""
+    batch, dev = vol.shape[0], vol.device
+    out = torch.empty((batch,) + tuple(geom.proj_shape), dtype=torch.float32, device=dev)
+    if batch == 0:
+        return out
+    _require(vol, (batch,) + tuple(geom.vol_shape), "vol")
+    lib = N.lib()
+    g = geom.ctypes_struct()
+    ang, br = geom.device_views(dev)
+    size = lambda n: lib.ctr_dd_forward_batch_workspace_bytes(ctypes.byref(g), n)  # noqa: E731
+    most = max(1, min(batch, 4096, _FORWARD_TABLES // max(size(2) - size(1), 1)))
+    launches = -(-batch // most)
+    per = -(-batch // launches)
+    nbytes = size(per)
+    ws = _workspace(nbytes, dev)
+    for b in range(0, batch, per):
+        n = min(per, batch - b)
+        N.check(lib.ctr_dd_forward_batch(ctypes.byref(g), _ptr(ang), _ptr(br), _ptr(vol[b]), _ptr(out[b]), n, _ptr(ws),
+                                         nbytes, _stream(dev)), "ctr_dd_forward_batch")
+    return out
+
+
 def filter_spectrum(geom: ScanGeometry, filter_type: str | None = None, cutoff: float | None = None,
                     device="cuda") -> torch.Tensor:
     """Filter magnitude in FFT order, float64[N] with N = zero-padded length, computed on the GPU.

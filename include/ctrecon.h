@@ -99,6 +99,12 @@ size_t ctr_dd_forward_workspace_bytes(const ctr_geometry* g);
 int ctr_dd_forward(const ctr_geometry* g, const double* angles, const int32_t* branch,
                    const float* vol, float* proj, void* workspace, size_t workspace_bytes,
                    void* stream);
+/* The same for `batch` volumes (1 .. 4096, one after the other in `vol`, their projections likewise in
+ * `proj`) in the launches of one; the workspace holds the tables of all of them. */
+size_t ctr_dd_forward_batch_workspace_bytes(const ctr_geometry* g, int batch);
+int ctr_dd_forward_batch(const ctr_geometry* g, const double* angles, const int32_t* branch,
+                         const float* vol, float* proj, int batch, void* workspace,
+                         size_t workspace_bytes, void* stream);
 
 /* ---- FDK filter -------------------------------------------------------------------------
  * ctr_filter_spectrum replaces Reconstruction.Filter (python/Reconstruction_pycuda.py:186-221):
