@@ -29,6 +29,7 @@ EXPORTS = (
     "ctr_version", "ctr_strerror", "ctr_select_branches", "ctr_zero_padded_length",
     "ctr_dd_forward_workspace_bytes", "ctr_dd_forward",
     "ctr_dd_forward_batch_workspace_bytes", "ctr_dd_forward_batch",
+    "ctr_dd_adjoint_batch_workspace_bytes", "ctr_dd_adjoint_batch",
     "ctr_fdk_filter_workspace_bytes", "ctr_filter_spectrum", "ctr_fdk_filter",
     "ctr_dd_backproject_workspace_bytes", "ctr_dd_backproject", "ctr_dd_backproject_static",
     "ctr_pixel_filter_spectrum", "ctr_pixel_filter",
@@ -120,6 +121,8 @@ def _declare(lib):
         "ctr_zero_padded_length": (c_int, [c_int]),
         "ctr_dd_forward_workspace_bytes": (c_size, [gp]),
         "ctr_dd_forward": (c_int, [gp, c_vp, c_vp, c_vp, c_vp, c_vp, c_size, c_vp]),
+        "ctr_dd_adjoint_batch_workspace_bytes": (c_size, [gp, c_int]),
+        "ctr_dd_adjoint_batch": (c_int, [gp, c_vp, c_vp, c_vp, c_vp, c_int, c_flt, c_vp, c_size, c_vp]),
         "ctr_dd_forward_batch_workspace_bytes": (c_size, [gp, c_int]),
         "ctr_dd_forward_batch": (c_int, [gp, c_vp, c_vp, c_vp, c_vp, c_int, c_vp, c_size, c_vp]),
         "ctr_fdk_filter_workspace_bytes": (c_size, [gp]),

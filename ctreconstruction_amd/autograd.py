@@ -4,8 +4,8 @@
 hand-written matched backprojector A^T (``ctr_dd_backproject`` in adjoint mode), so gradients
 of any loss of A x flow through the project's own kernels.  ``DDBackprojectorFunction`` is the
 transpose pair (y -> A^T y, backward A).  Both accept one volume [nz, ny, nx] or a batch
-[B, nz, ny, nx] (projections [nView, nv, nu] or [B, nView, nv, nu]); on the current stream, the
-volumes of a batch are projected together and its projections backprojected one item at a time.
+[B, nz, ny, nx] (projections [nView, nv, nu] or [B, nView, nv, nu]); the items of a batch share
+launches on the current stream.
 """
 from __future__ import annotations
 
@@ -34,6 +34,8 @@ def forward_batch(vol: torch.Tensor, geom: ScanGeometry) -> torch.Tensor:
 
 
 def adjoint_batch(proj: torch.Tensor, geom: ScanGeometry) -> torch.Tensor:
+    if proj.dim() == 4 and tuple(proj.shape[1:]) == tuple(geom.proj_shape):
+        return P.dd_adjoint_batch(proj.contiguous(), geom)
     return _batched(P.dd_adjoint, proj, geom.proj_shape, geom.vol_shape, geom)
 
 

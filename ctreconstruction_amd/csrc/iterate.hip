@@ -5,7 +5,7 @@
 // torch expressions they were about ten passes over the projections and five over the volume; each is
 // one pass here, bound by HBM.  The operations and their order are the expressions', so the results are
 // theirs bit for bit.  Three SART iterations at 256^3 x 60 views of 384 x 384: 5.58 -> 5.03 ms; an outer
-// ASD-POCS iteration over a batch of 128^3 volumes: 9.40 -> 8.81 ms.
+// ASD-POCS iteration over eight 128^3 volumes: 9.40 -> 8.81 ms.
 
 #include <hip/hip_runtime.h>
 

@@ -143,6 +143,13 @@ int ctr_dd_backproject(const ctr_geometry* g, const double* angles, const int32_
                        const float* proj, float* vol, int mode, float scale, float zero_tol,
                        int accumulate, void* workspace, size_t workspace_bytes, void* stream);
 
+/* CTR_BP_ADJOINT for `batch` scans of one geometry (1 .. 4096, one after the other in `proj`, their volumes
+ * likewise in `vol`, overwritten) in the launches of one. */
+size_t ctr_dd_adjoint_batch_workspace_bytes(const ctr_geometry* g, int batch);
+int ctr_dd_adjoint_batch(const ctr_geometry* g, const double* angles, const int32_t* branch,
+                         const float* proj, float* vol, int batch, float scale, void* workspace,
+                         size_t workspace_bytes, void* stream);
+
 /* No counterpart in the reference: ctr_dd_backproject (modes CTR_BP_FDK_REF and
  * CTR_BP_FDK_EDGE) without a workspace argument, for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).

@@ -9,7 +9,7 @@ import torch
 import ctreconstruction_amd as ctr
 from ctreconstruction_amd import _native as N
 from ctreconstruction_amd import projector as P
-from ctreconstruction_amd.autograd import forward_batch
+from ctreconstruction_amd.autograd import adjoint_batch, forward_batch
 from tests.conftest import make_params
 
 pytestmark = pytest.mark.gpu
@@ -50,3 +50,18 @@ def test_several_launches(monkeypatch):
     monkeypatch.setattr(P, "_FORWARD_TABLES", 0)
     assert (forward_batch(vols, geom) - whole).abs().max() <= 1e-6 * whole.abs().max()
     assert forward_batch(vols[:0], geom).shape == (0,) + tuple(geom.proj_shape)
+
+
+@pytest.mark.parametrize("n,det,views,batch", [([9, 10, 1], [15, 3], 4, 2), ([20, 17, 33], [37, 70], 9, 5),
+                                               ([64, 64, 20], [80, 130], 24, 4)])
+def test_adjoint_batch_equals_single_scans(n, det, views, batch, monkeypatch):
+    """The view splits differ with the batch: FP32 sums of at most `views` terms in another order."""
+    geom, _ = _case(n, det, views, 1)
+    proj = torch.rand((batch,) + tuple(geom.proj_shape), generator=torch.Generator().manual_seed(4)).cuda()
+    got = adjoint_batch(proj, geom)
+    for b in range(batch):
+        ref = P.dd_adjoint(proj[b], geom)
+        assert (got[b] - ref).abs().max() <= 2e-6 * ref.abs().max()
+    monkeypatch.setattr(P, "_ADJOINT_TABLES", 4 * 2 * proj[0].numel())      # two scans to a launch
+    assert (adjoint_batch(proj, geom) - got).abs().max() <= 2e-6 * got.abs().max()
+    assert adjoint_batch(proj[:0], geom).shape == (0,) + tuple(geom.vol_shape)
