@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstdint>
 
@@ -29,7 +30,7 @@ constexpr int kTvZ = 16;            // planes a work-item walks
 
 enum { kTvNorm, kTvGradient, kTvStep };
 
-// 1 / sqrt(s): the hardware's estimate and one Newton step (0 where s has overflowed)
+// 1 / sqrt(s) of a normal s: the hardware's estimate and one Newton step (0 where s has overflowed)
 __device__ inline float tv_rsqrt(float s) {
     const float r = __builtin_amdgcn_rsqf(s);
     return s <= 3.4028235e38f ? fmaf(0.5f * r, fmaf(-s * r, r, 1.0f), r) : r;
@@ -182,7 +183,7 @@ size_t ctr_tv_workspace_bytes(int batch, int nx, int ny, int nz, int steps) {
 
 int ctr_tv_gradient(const float* x, float* grad, int batch, int nx, int ny, int nz, float eps, void* workspace,
                     size_t workspace_bytes, void* stream) {
-    if (!x || !grad || !workspace || x == grad || !tv_sizes_ok(batch, nx, ny, nz) || !(eps > 0)) return CTR_ERR_INVALID;
+    if (!x || !grad || !workspace || x == grad || !tv_sizes_ok(batch, nx, ny, nz) || !(eps >= FLT_MIN)) return CTR_ERR_INVALID;
     const TvLayout l = tv_layout(batch, nx, ny, nz, 1);
     if (workspace_bytes < l.total) return CTR_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
@@ -197,7 +198,7 @@ int ctr_tv_gradient(const float* x, float* grad, int batch, int nx, int ny, int 
 
 int ctr_tv_descent(const float* x, float* out, const float* step, int batch, int nx, int ny, int nz, float eps, int steps,
                    void* workspace, size_t workspace_bytes, void* stream) {
-    if (!x || !out || !step || !workspace || x == out || steps < 1 || !tv_sizes_ok(batch, nx, ny, nz) || !(eps > 0))
+    if (!x || !out || !step || !workspace || x == out || steps < 1 || !tv_sizes_ok(batch, nx, ny, nz) || !(eps >= FLT_MIN))
         return CTR_ERR_INVALID;
     const TvLayout l = tv_layout(batch, nx, ny, nz, steps);
     if (workspace_bytes < l.total) return CTR_ERR_WORKSPACE;

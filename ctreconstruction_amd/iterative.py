@@ -157,8 +157,10 @@ def _plain(img: torch.Tensor) -> bool:
 
 
 def _on_tv_kernels(img: torch.Tensor, eps: float) -> bool:
-    """Whether the TV kernels take ``img``."""
-    return (_plain(img) and min(img.shape[-3:]) >= 3 and img.shape[-3:].numel() < 2 ** 31 - 1 and eps > 0)
+    """Whether the TV kernels take ``img`` and ``eps``: a plain number that is a normal float32 (the
+    kernels' reciprocal root flushes smaller ones, which torch computes with)."""
+    return (_plain(img) and min(img.shape[-3:]) >= 3 and img.shape[-3:].numel() < 2 ** 31 - 1
+            and isinstance(eps, (int, float)) and ctypes.c_float(eps).value >= 2.0 ** -126)
 
 
 def _elementwise(x: torch.Tensor, y: torch.Tensor, per_geom: torch.Tensor, *scalars) -> bool:

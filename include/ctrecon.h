@@ -204,7 +204,8 @@ int ctr_pixel_backproject(const ctr_geometry* g, const double* angles, const flo
 
 /* ---- Total-variation steps of ASD-POCS ----------------------------------------------------
  * Replace the TV gradient and descent of python/ASD_POCS.py:55-77 and 188-192 on a batch of
- * independent volumes float32 [batch][nz][ny][nx], every axis >= 3 voxels, eps > 0.
+ * independent volumes float32 [batch][nz][ny][nx], every axis >= 3 voxels, eps a normal float
+ * (at least FLT_MIN, 1.2e-38).
  * ctr_tv_gradient: grad = g / ||g||_2 (g itself where the norm is below eps), 0 on the border.
  * ctr_tv_descent: out = x after `steps` steps x <- x - step[b] * g / ||g||_2; `step` is float32
  * device memory, `batch` entries.  Outputs must not overlap `x`. */
