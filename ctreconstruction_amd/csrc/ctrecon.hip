@@ -64,6 +64,16 @@ int check_geometry(const ctr_geometry* g) {
 
 int status_from_hip(hipError_t e) { return e == hipSuccess ? CTR_OK : CTR_ERR_HIP; }
 
+// A launch's x extent is at most 2^32 - 1 threads.  The preparation kernels, whose workgroups may be more
+// (slices over about 23 000^2, scans over about 5e8 detector columns), go on in z.
+constexpr long long kMaxThreadsX = 0xffffffffLL;
+
+dim3 groups_of_256(long long groups, unsigned y) {
+    const long long most = kMaxThreadsX / 256, z = (groups + most - 1) / most;
+    return dim3((unsigned)((groups + z - 1) / z), y, (unsigned)z);
+}
+__device__ inline int group_of_256() { return blockIdx.z * gridDim.x + blockIdx.x; }
+
 // ------------------------------------------------------------------------------------------
 // Forward projection
 // ------------------------------------------------------------------------------------------
@@ -246,11 +256,11 @@ __global__ void __launch_bounds__(256) fp_prepare_kernel(ctr_geometry g, const d
                                                          float* __restrict__ rows, int stride, int geo_groups,
                                                          const float* __restrict__ vol, float* __restrict__ t_ys,
                                                          float* __restrict__ t_xs, int nzp, size_t item_stride) {
-    const int zx = (g.nx + 31) / 32, zgroups = zx * g.ny, b = blockIdx.x;
+    const int zx = (g.nx + 31) / 32, zgroups = zx * g.ny, b = group_of_256();
     if (b < zgroups) {
         const size_t t = blockIdx.y * item_stride;
         zprefix(vol + blockIdx.y * ((size_t)g.nx * g.ny * g.nz), t_ys + t, t_xs + t, g.nx, g.ny, g.nz, nzp, (b % zx) * 32, b / zx);
-    } else if (blockIdx.y == 0) {
+    } else if (blockIdx.y == 0 && b - zgroups < geo_groups * g.n_views) {
         const int r = b - zgroups;
         fp_geometry(g, angles, branch, tabs, rows, stride, (r % geo_groups) * 256 + (int)threadIdx.x, r / geo_groups);
     }
@@ -2029,8 +2039,8 @@ __device__ inline int adj_pitch(int rows) { return rows | 1; }
 // source's) has no such window and takes the gather path.
 __device__ inline void adj_tile(AdjTile* __restrict__ tw, const float* __restrict__ tabs, const float* __restrict__ at,
                                 int nx, int ny, int nz, int nu, int n_views, int stride, int curved, int tiles_x,
-                                int n_tiles, int tz, int slabs, int cap, int idx) {
-    if (idx >= n_views * n_tiles) return;
+                                int n_tiles, int tz, int slabs, int cap, unsigned idx) {
+    if (idx >= (unsigned)n_views * n_tiles) return;
     const int view = idx / n_tiles, t = idx - view * n_tiles;
     const int x0 = (t % tiles_x) * kTileX, y0 = (t / tiles_x) * kTileY;
     const int x1 = min(x0 + kTileX, nx) - 1, y1 = min(y0 + kTileY, ny) - 1;
@@ -2089,12 +2099,12 @@ __global__ void __launch_bounds__(256) adj_prepare_kernel(const float* __restric
                                                           const float* __restrict__ at, AdjTile* __restrict__ tw, int nx,
                                                           int ny, int nz, int nu, int nv, int nvp, int n_views, int stride,
                                                           int curved, int tiles_x, int n_tiles, int tz, int slabs, int cap) {
-    const int px = (nu + 31) / 32, pgroups = px * n_views, b = blockIdx.x;
+    const int px = (nu + 31) / 32, pgroups = px * n_views, b = group_of_256();
     if (b < pgroups)
         adj_rowprefix(y + blockIdx.y * ((size_t)n_views * nv * nu), Y + blockIdx.y * ((size_t)n_views * nu * nvp), tabs, rows, nu, nv, nvp, stride, (b % px) * 32, b / px);
     else if (blockIdx.y == 0)
         adj_tile(tw, tabs, at, nx, ny, nz, nu, n_views, stride, curved, tiles_x, n_tiles, tz, slabs, cap,
-                 (b - pgroups) * 256 + (int)threadIdx.x);
+                 (unsigned)(b - pgroups) * 256 + threadIdx.x);
 }
 
 // One column's share of a work-item's voxels: boundary c of the volume has the edge coordinate
@@ -2930,8 +2940,8 @@ struct BpPlan {
 BpPlan bp_plan(const ctr_geometry* g, size_t budget) {
     BpPlan p;
     p.shape = bp_choose(g);
-    // no shape has fewer flags than this
-    if (bp_base_bytes(g, p.shape) > budget) p.shape = kShapeWhole;
+    // no shape has fewer flags, or workgroups, than this
+    if (bp_base_bytes(g, p.shape) > budget || (double)bp_tiles(g, p.shape) * 256 > kMaxThreadsX) p.shape = kShapeWhole;
     const long long tiles = (long long)bp_tiles(g, p.shape);
     const size_t part = (size_t)g->nx * g->ny * g->nz * sizeof(float);
     p.base = bp_base_bytes(g, p.shape);
@@ -2996,12 +3006,16 @@ struct AdjLayout {
 
 AdjLayout adj_layout(const ctr_geometry* g, int batch) {
     AdjLayout L;
-    L.shape = adj_choose(g);
-    L.tz = adj_with_shape(L.shape, [](auto sh) { return (int)decltype(sh)::TZ; });
-    L.cap = adj_with_shape(L.shape, [](auto sh) { return (int)decltype(sh)::CAP; });
     L.tiles_x = (g->nx + kTileX - 1) / kTileX;
     L.tiles_y = (g->ny + kTileY - 1) / kTileY;
-    L.tiles_z = (g->nz + L.tz - 1) / L.tz;
+    L.shape = adj_choose(g);
+    for (int pass = 0; pass < 2; ++pass) {
+        L.tz = adj_with_shape(L.shape, [](auto sh) { return (int)decltype(sh)::TZ; });
+        L.tiles_z = (g->nz + L.tz - 1) / L.tz;
+        if ((double)L.tiles_x * L.tiles_y * L.tiles_z * 256 <= kMaxThreadsX) break;
+        L.shape = kAdjDeep;  // fewer workgroups than one launch takes
+    }
+    L.cap = adj_with_shape(L.shape, [](auto sh) { return (int)decltype(sh)::CAP; });
     const long long n_tiles = (long long)L.tiles_x * L.tiles_y, all_tiles = n_tiles * L.tiles_z * batch;
     // view splits as in the FDK backprojection (2560 and 10240 groups: 1 and 5 % slower on 128^3 x 180)
     long long want = std::min<long long>((kBpTargetGroups + all_tiles - 1) / all_tiles, g->n_views / kBpMinViews);
@@ -3031,7 +3045,7 @@ int adj_run(const ctr_geometry* g, const double* angles, const int32_t* branch, 
     float* yp = (float*)(ws + L.yl_off);  // row-prefix table
     float* parts = (float*)(ws + L.parts_off);
     const int stride = fp_view_stride(g->nu), n_tiles = L.tiles_x * L.tiles_y;
-    if ((double)n_tiles * g->n_views >= 2147483647.0 || (double)n_tiles * L.tiles_z >= 2147483647.0)
+    if ((double)n_tiles * g->n_views >= 2147483647.0 || (double)n_tiles * L.tiles_z * 256 > kMaxThreadsX)
         return CTR_ERR_INVALID;
     const int curved = g->detector_shape == CTR_DETECTOR_CURVED ? 1 : 0;
     int st = CTR_OK;
@@ -3041,8 +3055,7 @@ int adj_run(const ctr_geometry* g, const double* angles, const int32_t* branch, 
     if ((st = status_from_hip(hipGetLastError()))) return st;
     const int nvp = adj_prefix_stride(g->nv);
     const long long groups = (long long)((g->nu + 31) / 32) * g->n_views + ((long long)g->n_views * n_tiles + 255) / 256;
-    if (groups >= 2147483647LL) return CTR_ERR_INVALID;
-    hipLaunchKernelGGL(adj_prepare_kernel, dim3((unsigned)groups, batch), dim3(256), 0, s, proj, yp, tabs, rows, at, tw, g->nx,
+    hipLaunchKernelGGL(adj_prepare_kernel, groups_of_256(groups, batch), dim3(256), 0, s, proj, yp, tabs, rows, at, tw, g->nx,
                        g->ny, g->nz, g->nu, g->nv, nvp, g->n_views, stride, curved, L.tiles_x, n_tiles, L.tz, L.tiles_z,
                        L.cap);
     if ((st = status_from_hip(hipGetLastError()))) return st;
@@ -3092,7 +3105,7 @@ int bp_fdk(const ctr_geometry* g, const double* angles, const float* proj, float
                   float zero_tol, int accumulate, void* workspace, const BpPlan& p, hipStream_t s) {
     int st = CTR_OK;
     const size_t tiles = bp_tiles(g, p.shape);
-    if (tiles >= 2147483647u) return CTR_ERR_INVALID;
+    if ((long long)tiles > kMaxThreadsX / 256) return CTR_ERR_INVALID;
     float* vt = (float*)workspace;
     uint8_t* flags = (uint8_t*)workspace + align_up((size_t)g->n_views * kBpViewStride * sizeof(float), 256);
     float* parts = (float*)((char*)workspace + p.base);
@@ -3217,8 +3230,7 @@ int ctr_dd_forward_batch(const ctr_geometry* g, const double* angles, const int3
     const int gx = (std::max(g->nu + 1, g->nv + 1) + 255) / 256;
     const int nzp = zprefix_stride(g->nz);
     const long long prep = (long long)((g->nx + 31) / 32) * g->ny + (long long)gx * g->n_views;
-    if (prep >= 2147483647LL) return CTR_ERR_INVALID;
-    hipLaunchKernelGGL(fp_prepare_kernel, dim3((unsigned)prep, batch), dim3(256), 0, s, *g, angles, branch, tabs, rows,
+    hipLaunchKernelGGL(fp_prepare_kernel, groups_of_256(prep, batch), dim3(256), 0, s, *g, angles, branch, tabs, rows,
                        stride, gx, vol, t_ys, t_xs, nzp, item_stride);
     if ((st = status_from_hip(hipGetLastError()))) return st;
     if (g->nv <= kThinRows) {
@@ -3243,14 +3255,15 @@ int ctr_dd_forward_batch(const ctr_geometry* g, const double* angles, const int3
         const long long n_blocks =
             8LL * ((col_groups + 7) / 8) * row_blocks * n_vblocks * kViewBlock;
         if (n_blocks >= 2147483647LL) return CTR_ERR_INVALID;
-        auto launch = [&](auto kernel, int split) {
-            hipLaunchKernelGGL(kernel, dim3((unsigned)n_blocks, batch), dim3(64 * kFpWaves * split), 0, s, t_ys, t_xs, proj,
+        const int split = n_blocks * 64 * kFpWaves * plan.split <= kMaxThreadsX ? plan.split : 1;
+        auto launch = [&](auto kernel, int shares) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)n_blocks, batch), dim3(64 * kFpWaves * shares), 0, s, t_ys, t_xs, proj,
                                tabs, rows, branch, g->nx, g->ny, g->nz, nzp, g->nu, g->nv, stride, 1e-6f, g->n_views, col_groups,
                                n_vblocks, plan.row_shift, item_stride);
         };
-        plan.split == 1   ? launch(dd_forward_kernel<1>, 1)
-        : plan.split == 2 ? launch(dd_forward_kernel<2>, 2)
-                          : launch(dd_forward_kernel<4>, 4);
+        split == 1   ? launch(dd_forward_kernel<1>, 1)
+        : split == 2 ? launch(dd_forward_kernel<2>, 2)
+                     : launch(dd_forward_kernel<4>, 4);
     }
     if ((st = status_from_hip(hipGetLastError()))) return st;
     // z-slab views (left at zero above): their own kernel, which returns at once for the others
