@@ -2092,18 +2092,19 @@ __device__ inline void adj_tile(AdjTile* __restrict__ tw, const float* __restric
     tw[idx] = w;
 }
 
-// The row-prefix tables (the first workgroups; blockIdx.y is the item of a batch) and the windows (the
-// others; they serve every item) in one launch.
+// The row-prefix tables (the first `pgroups` workgroups; blockIdx.y is the item of a batch) and the windows
+// of a run of views (the others; they serve every item) in one launch.
 __global__ void __launch_bounds__(256) adj_prepare_kernel(const float* __restrict__ y, float* __restrict__ Y,
                                                           const float* __restrict__ tabs, const float* __restrict__ rows,
-                                                          const float* __restrict__ at, AdjTile* __restrict__ tw, int nx,
-                                                          int ny, int nz, int nu, int nv, int nvp, int n_views, int stride,
+                                                          const float* __restrict__ run_tabs, const float* __restrict__ run_at,
+                                                          AdjTile* __restrict__ tw, int nx, int ny, int nz, int nu, int nv,
+                                                          int nvp, int n_views, int pgroups, int run_views, int stride,
                                                           int curved, int tiles_x, int n_tiles, int tz, int slabs, int cap) {
-    const int px = (nu + 31) / 32, pgroups = px * n_views, b = group_of_256();
+    const int px = (nu + 31) / 32, b = group_of_256();
     if (b < pgroups)
         adj_rowprefix(y + blockIdx.y * ((size_t)n_views * nv * nu), Y + blockIdx.y * ((size_t)n_views * nu * nvp), tabs, rows, nu, nv, nvp, stride, (b % px) * 32, b / px);
     else if (blockIdx.y == 0)
-        adj_tile(tw, tabs, at, nx, ny, nz, nu, n_views, stride, curved, tiles_x, n_tiles, tz, slabs, cap,
+        adj_tile(tw, run_tabs, run_at, nx, ny, nz, nu, run_views, stride, curved, tiles_x, n_tiles, tz, slabs, cap,
                  (unsigned)(b - pgroups) * 256 + threadIdx.x);
 }
 
@@ -2130,18 +2131,19 @@ __device__ inline void adj_chunk(int iz0, float gam, float off, float de, float 
 }
 
 // vol = (accumulate ? vol : 0) + scale * A^T y of the split's views (blockIdx.y), or that into the
-// split's volume in `parts` (added up by sum_parts_kernel); blockIdx.z is the item of a batch.
+// split's volume in `parts` (added up by sum_parts_kernel); blockIdx.z is the item of a batch, whose
+// row-prefix tables lie `item` floats apart.  `all_views` views, of which Y, tabs, at and tw are the first's.
 template <typename S>
 __global__ void __launch_bounds__(256) dd_adjoint_kernel(
-    const float* __restrict__ Y, float* __restrict__ vol, float* __restrict__ parts, const float* __restrict__ tabs,
-    const float* __restrict__ at, const AdjTile* __restrict__ tw, int nx, int ny, int nz, int nu, int nv, int nvp,
-    int all_views, int views_per, int stride, int curved, float scale, float tol, int accumulate, int tiles_x,
+    const float* __restrict__ Y, size_t item, float* __restrict__ vol, float* __restrict__ parts,
+    const float* __restrict__ tabs, const float* __restrict__ at, const AdjTile* __restrict__ tw, int nx, int ny, int nz,
+    int nu, int nv, int nvp, int all_views, int views_per, int stride, int curved, float scale, float tol, int accumulate, int tiles_x,
     int tiles_y, int tiles_z) {
     constexpr int TZ = S::TZ, CAP = S::CAP, kPre = (CAP + 255) / 256;
     __shared__ float win[2][CAP];
     __shared__ float4 cols[2][kAdjCols + 1];  // per column edge: footprint line (at, per slab), slab fraction (at, per slab)
     const int view0 = blockIdx.y * views_per, n_views = min(views_per, all_views - view0);
-    Y += blockIdx.z * ((size_t)all_views * nu * nvp);
+    Y += blockIdx.z * item;
     if (gridDim.y > 1)
         vol = parts + ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * nx * ny * nz;
     else
@@ -2994,13 +2996,17 @@ AdjKind adj_choose(const ctr_geometry* g) {
 }
 
 // Adjoint workspace: the forward projector's tables and row table (no volume tables), the
-// per-view adjoint constants, the windows of every (view, column tile), the row-prefix tables
-// Y[item][view][column][nvp], then the view splits' partial volumes.  The items of a batch share the
+// per-view adjoint constants, the windows of every (view, column tile) of a run of views, the row-prefix
+// tables Y[item][view][column][nvp], then the view splits' partial volumes.  A run holds all views unless
+// its windows would take more than kAdjMaxWindows entries (1 GiB: 65535 views of 512^2, 256 of 8192^2): the
+// adjoint then goes through the views run by run, each added to the volume.  The items of a batch share the
 // launches: with eight 128^3 volumes a volume's views are split into 3 parts instead of 20, each a volume
 // to write and to sum (234 -> 185 us per volume at 180 views).
+constexpr int kAdjMaxWindows = 1 << 26;
+
 struct AdjLayout {
     AdjKind shape;
-    int tiles_x, tiles_y, tiles_z, tz, cap, splits, views_per;
+    int tiles_x, tiles_y, tiles_z, tz, cap, run, splits, views_per;
     size_t tabs_off, rows_off, at_off, tw_off, yl_off, parts_off, total;
 };
 
@@ -3018,15 +3024,16 @@ AdjLayout adj_layout(const ctr_geometry* g, int batch) {
     L.cap = adj_with_shape(L.shape, [](auto sh) { return (int)decltype(sh)::CAP; });
     const long long n_tiles = (long long)L.tiles_x * L.tiles_y, all_tiles = n_tiles * L.tiles_z * batch;
     // view splits as in the FDK backprojection (2560 and 10240 groups: 1 and 5 % slower on 128^3 x 180)
-    long long want = std::min<long long>((kBpTargetGroups + all_tiles - 1) / all_tiles, g->n_views / kBpMinViews);
+    L.run = (int)std::min<long long>(g->n_views, std::max<long long>(kAdjMaxWindows / n_tiles, 1));
+    long long want = std::min<long long>((kBpTargetGroups + all_tiles - 1) / all_tiles, L.run / kBpMinViews);
     want = std::max<long long>(want, 1);
-    L.views_per = (int)((g->n_views + want - 1) / want);
-    L.splits = (g->n_views + L.views_per - 1) / L.views_per;
+    L.views_per = (int)((L.run + want - 1) / want);
+    L.splits = (L.run + L.views_per - 1) / L.views_per;
     L.tabs_off = 0;
     L.rows_off = align_up((size_t)fp_view_stride(g->nu) * g->n_views * 4, 256);
     L.at_off = align_up(L.rows_off + (size_t)(2 * g->nv + 1) * 4, 256);
     L.tw_off = align_up(L.at_off + (size_t)g->n_views * kAdjViewStride * 4, 256);
-    L.yl_off = align_up(L.tw_off + (size_t)g->n_views * n_tiles * sizeof(AdjTile), 256);
+    L.yl_off = align_up(L.tw_off + (size_t)L.run * n_tiles * sizeof(AdjTile), 256);
     L.parts_off = align_up(L.yl_off + (size_t)batch * g->n_views * g->nu * adj_prefix_stride(g->nv) * 4, 256);
     L.total = L.parts_off + (L.splits > 1 ? align_up((size_t)batch * L.splits * g->nx * g->ny * g->nz * 4, 256) : 0);
     return L;
@@ -3045,8 +3052,7 @@ int adj_run(const ctr_geometry* g, const double* angles, const int32_t* branch, 
     float* yp = (float*)(ws + L.yl_off);  // row-prefix table
     float* parts = (float*)(ws + L.parts_off);
     const int stride = fp_view_stride(g->nu), n_tiles = L.tiles_x * L.tiles_y;
-    if ((double)n_tiles * g->n_views >= 2147483647.0 || (double)n_tiles * L.tiles_z * 256 > kMaxThreadsX)
-        return CTR_ERR_INVALID;
+    if ((double)n_tiles * L.tiles_z * 256 > kMaxThreadsX) return CTR_ERR_INVALID;
     const int curved = g->detector_shape == CTR_DETECTOR_CURVED ? 1 : 0;
     int st = CTR_OK;
     const int gx = (std::max(g->nu + 1, g->nv + 1) + 255) / 256;
@@ -3054,21 +3060,32 @@ int adj_run(const ctr_geometry* g, const double* angles, const int32_t* branch, 
                        at);
     if ((st = status_from_hip(hipGetLastError()))) return st;
     const int nvp = adj_prefix_stride(g->nv);
-    const long long groups = (long long)((g->nu + 31) / 32) * g->n_views + ((long long)g->n_views * n_tiles + 255) / 256;
-    hipLaunchKernelGGL(adj_prepare_kernel, groups_of_256(groups, batch), dim3(256), 0, s, proj, yp, tabs, rows, at, tw, g->nx,
-                       g->ny, g->nz, g->nu, g->nv, nvp, g->n_views, stride, curved, L.tiles_x, n_tiles, L.tz, L.tiles_z,
-                       L.cap);
-    if ((st = status_from_hip(hipGetLastError()))) return st;
-    const hipError_t e = adj_with_shape(L.shape, [&](auto sh) {
-        // transverse overlaps under 1e-6 of the footprint are dropped, as in ctr_dd_forward
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(dd_adjoint_kernel<decltype(sh)>), dim3((unsigned)(n_tiles * L.tiles_z), L.splits, batch),
-                           dim3(256), 0, s, yp, vol, parts, tabs, at, tw, g->nx, g->ny, g->nz, g->nu, g->nv, nvp,
-                           g->n_views, L.views_per, stride, curved, scale, 1e-6f, L.splits > 1 ? 0 : accumulate, L.tiles_x,
-                           L.tiles_y, L.tiles_z);
-        return hipGetLastError();
-    });
-    if ((st = status_from_hip(e))) return st;
-    return L.splits > 1 ? sum_parts(g, parts, vol, L.splits, accumulate, s, batch) : CTR_OK;
+    const size_t item = (size_t)g->n_views * g->nu * nvp;
+    for (int view0 = 0; view0 < g->n_views; view0 += L.run) {
+        const int views = std::min(L.run, g->n_views - view0), splits = (views + L.views_per - 1) / L.views_per;
+        const int add = view0 ? 1 : accumulate;
+        // the first run's preparation builds every view's row-prefix table
+        const int prefix_groups = view0 ? 0 : (g->nu + 31) / 32 * g->n_views;
+        const float* run_tabs = tabs + (size_t)view0 * stride;
+        const float* run_at = at + (size_t)view0 * kAdjViewStride;
+        const long long groups = prefix_groups + ((long long)views * n_tiles + 255) / 256;
+        hipLaunchKernelGGL(adj_prepare_kernel, groups_of_256(groups, view0 ? 1 : batch), dim3(256), 0, s, proj, yp, tabs,
+                           rows, run_tabs, run_at, tw, g->nx, g->ny, g->nz, g->nu, g->nv, nvp, g->n_views, prefix_groups,
+                           views, stride, curved, L.tiles_x, n_tiles, L.tz, L.tiles_z, L.cap);
+        if ((st = status_from_hip(hipGetLastError()))) return st;
+        const hipError_t e = adj_with_shape(L.shape, [&](auto sh) {
+            // transverse overlaps under 1e-6 of the footprint are dropped, as in ctr_dd_forward
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(dd_adjoint_kernel<decltype(sh)>),
+                               dim3((unsigned)(n_tiles * L.tiles_z), splits, batch), dim3(256), 0, s,
+                               yp + (size_t)view0 * g->nu * nvp, item, vol, parts, run_tabs, run_at, tw, g->nx, g->ny, g->nz,
+                               g->nu, g->nv, nvp, views, L.views_per, stride, curved, scale, 1e-6f, splits > 1 ? 0 : add,
+                               L.tiles_x, L.tiles_y, L.tiles_z);
+            return hipGetLastError();
+        });
+        if ((st = status_from_hip(e))) return st;
+        if (splits > 1 && (st = sum_parts(g, parts, vol, splits, add, s, batch))) return st;
+    }
+    return CTR_OK;
 }
 
 // The launches of one shape: the single pass over all cases, or the fast pass over the common
