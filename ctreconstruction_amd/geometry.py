@@ -122,6 +122,12 @@ class ScanGeometry:
         g.det_offset[:] = [float(v) for v in self.det_offset]
         return g
 
+    def contents(self) -> bytes:
+        """Everything the operators read, as bytes: equal for two states of a geometry that describe
+        the same scan."""
+        return b"".join((bytes(self.ctypes_struct()), np.float64(self.dtheta).tobytes(),
+                         np.ascontiguousarray(self.angles).tobytes(), np.ascontiguousarray(self.branch).tobytes()))
+
     def device_views(self, device):
         """(angles float64, branch int32) device tensors, uploaded once per device."""
         import torch

@@ -40,18 +40,25 @@ def _bp_ref(proj: torch.Tensor, geom: ScanGeometry, mode: str = "ref") -> torch.
     return out
 
 
-# per geometry object: {(backprojector, device): (A 1, B 1)}, freed with the geometry
+# per geometry object: {(backprojector, device): (contents, A 1, B 1)}, freed with the geometry
 _NORM_CACHE: "weakref.WeakKeyDictionary[ScanGeometry, dict]" = weakref.WeakKeyDictionary()
 
 
 def normalisers(geom: ScanGeometry, backprojector: str, device, eps: float):
     """(row sums A 1, column sums B 1) for the chosen backprojector B; cached per geometry object
-    (held weakly: the cache goes when the geometry does)."""
+    (held weakly: the cache goes when the geometry does) for the scan it describes at the time.
+
+    The sums are finished when they enter the cache (one wait per scan), so that any stream, thread or
+    graph capture may read them; each stream that does is noted, so that their memory outlives its
+    reads.  Sums worked out inside a graph capture exist only when the graph runs and are not kept."""
     per_geom = _NORM_CACHE.setdefault(geom, {})
-    key = (backprojector, str(device))
+    key, contents = (backprojector, str(device)), geom.contents()
     hit = per_geom.get(key)
-    if hit is not None:
-        return hit
+    if hit is not None and hit[0] == contents:
+        stream = torch.cuda.current_stream(device)
+        for t in hit[1:]:
+            t.record_stream(stream)
+        return hit[1:]
     ones_v = torch.ones(geom.vol_shape, device=device)
     ones_p = torch.ones(geom.proj_shape, device=device)
     a1 = P.dd_forward(ones_v, geom)
@@ -61,7 +68,9 @@ def normalisers(geom: ScanGeometry, backprojector: str, device, eps: float):
         b1 = P.dd_backproject(ones_p, geom, mode="edge")
     else:
         b1 = _bp_ref(ones_p, geom)
-    per_geom[key] = (a1, b1)
+    if not torch.cuda.is_current_stream_capturing():
+        torch.cuda.current_stream(device).synchronize()
+        per_geom[key] = (contents, a1, b1)
     return a1, b1
 
 
