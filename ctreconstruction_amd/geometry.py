@@ -129,14 +129,25 @@ class ScanGeometry:
                          np.ascontiguousarray(self.angles).tobytes(), np.ascontiguousarray(self.branch).tobytes()))
 
     def device_views(self, device):
-        """(angles float64, branch int32) device tensors, uploaded once per device."""
+        """(angles float64, branch int32) device tensors, uploaded once per device and again when the
+        arrays have changed.  Their memory outlives the work of every stream that asked for them."""
         import torch
-        key = str(device)
-        if key not in self._device_cache:
-            ang = torch.from_numpy(np.ascontiguousarray(self.angles, dtype=np.float64)).to(device)
-            br = torch.from_numpy(np.ascontiguousarray(self.branch, dtype=np.int32)).to(device)
-            self._device_cache[key] = (ang, br)
-        return self._device_cache[key]
+        key, contents = str(device), (self.angles.tobytes(), self.branch.tobytes())
+        stream = torch.cuda.current_stream(device)
+        hit = self._device_cache.get(key)
+        if hit is None or hit[0] != contents:
+            # copies from pageable memory: finished when they return
+            ang = torch.from_numpy(np.array(self.angles, dtype=np.float64)).to(device)
+            br = torch.from_numpy(np.array(self.branch, dtype=np.int32)).to(device)
+            hit = self._device_cache[key] = (contents, stream, ang, br)
+        elif hit[1] != stream:
+            for t in hit[2:]:
+                t.record_stream(stream)
+        return hit[2:]
+
+    def __getstate__(self):
+        """Copies and pickles upload their own views."""
+        return {**self.__dict__, "_device_cache": {}}
 
     def with_views(self, views) -> "ScanGeometry":
         """The same scan restricted to ``views`` (their angles and branches; dtheta of the full scan)."""
