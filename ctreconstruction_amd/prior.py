@@ -54,10 +54,24 @@ def conv3x3_forward(x: torch.Tensor, w_bf16: torch.Tensor, bias: torch.Tensor | 
     return out
 
 
+def _gradient_operands(x: torch.Tensor, gout: torch.Tensor):
+    """(n, h, w, cin, cout), after checking what the kernels read as raw memory.  On a training step's host
+    path, which is longer than its kernels take: attributes that cost little."""
+    if x.dtype is not BF16 or gout.dtype is not BF16 or x.dim() != 4 or not x.is_contiguous():
+        raise TypeError("x must be contiguous NHWC bfloat16 and the output gradient bfloat16")
+    n, h, w, cin = x.shape
+    shape = gout.shape
+    cout = shape[-1] if len(shape) else 0
+    if shape != (n, h, w, cout):
+        raise ValueError(f"output gradient {tuple(shape)} does not match the input {tuple(x.shape)}")
+    if not x.is_cuda or gout.get_device() != x.get_device():
+        raise ValueError(f"x and the output gradient must be on one GPU (got {x.device}, {gout.device})")
+    return n, h, w, cin, cout
+
+
 def conv3x3_wgrad(x: torch.Tensor, gout: torch.Tensor, with_bias: bool = True):
     """(grad_weight [Cout,3,3,Cin] float32, grad_bias [Cout] float32) summed over all pixels."""
-    n, h, w, cin = x.shape
-    cout = gout.shape[-1]
+    n, h, w, cin, cout = _gradient_operands(x, gout)
     lib = N.lib()
     gw = torch.empty((cout, 3, 3, cin), dtype=torch.float32, device=x.device)
     gb = torch.empty(cout, dtype=torch.float32, device=x.device) if with_bias else None
@@ -76,8 +90,12 @@ def flip_transpose(w_bf16: torch.Tensor) -> torch.Tensor:
 def conv3x3_backward(x: torch.Tensor, w_bf16: torch.Tensor, gout: torch.Tensor, input_grad: bool = True):
     """(grad_x bfloat16 or None, grad_weight, grad_bias): the input gradient (the convolution of the
     output gradient with :func:`flip_transpose`-d weights) and :func:`conv3x3_wgrad` in one call."""
-    n, h, w, cin = x.shape
-    cout = gout.shape[-1]
+    n, h, w, cin, cout = _gradient_operands(x, gout)
+    if w_bf16.dtype is not BF16:
+        raise TypeError("weights must be bfloat16")
+    if w_bf16.shape != (cout, 3, 3, cin) or w_bf16.get_device() != x.get_device():
+        raise ValueError(f"weights {tuple(w_bf16.shape)} on {w_bf16.device}: expected ({cout}, 3, 3, {cin}) on {x.device}")
+    gout, w_bf16 = gout.contiguous(), w_bf16.contiguous()
     lib, dev = N.lib(), x.device
     gx = torch.empty_like(x) if input_grad else None
     gw = torch.empty((cout, 3, 3, cin), dtype=torch.float32, device=dev)
@@ -100,8 +118,7 @@ class Conv3x3Function(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gout):
         x, wb = ctx.saved_tensors
-        gout = gout.to(BF16).contiguous()
-        return (*conv3x3_backward(x, wb, gout, ctx.need_input_grad), None)
+        return (*conv3x3_backward(x, wb, gout.to(BF16), ctx.need_input_grad), None)
 
 
 class ResidualPrior(torch.nn.Module):
