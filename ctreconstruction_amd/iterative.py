@@ -149,20 +149,32 @@ def _normalise_pad(dtv: torch.Tensor, eps: float) -> torch.Tensor:
     return torch.nn.functional.pad(dtv / norm, (1, 1, 1, 1, 1, 1))
 
 
+def _observed(img: torch.Tensor) -> bool:
+    """Whether something maps, differentiates forward, traces or intercepts torch's work on ``img``, which a
+    kernel called by address would pass by.  torch has no public form for some of these questions: where it
+    cannot answer one, the answer is yes."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return True
+    try:
+        if torch.overrides._get_current_function_mode_stack():
+            return True
+        if torch.utils._python_dispatch._get_current_dispatch_mode() is not None:
+            return True
+        if torch._C._functorch.is_functorch_wrapped_tensor(img):
+            return True
+        return torch.autograd.forward_ad.unpack_dual(img).tangent is not None
+    except (AttributeError, ImportError):
+        return True
+
+
 def _plain(img: torch.Tensor) -> bool:
     """Whether a kernel may take ``img``: a contiguous float32 batch of volumes (or projections) on the
-    GPU that nothing differentiates, maps or traces (the torch expressions serve everything else)."""
+    GPU that nothing differentiates or observes (the torch expressions serve everything else)."""
     if type(img) is not torch.Tensor or img.device.type != "cuda" or img.dtype != torch.float32:
         return False
     if img.dim() < 3 or not img.is_contiguous() or img.numel() == 0 or img.shape[:-3].numel() > 65535:
         return False
-    if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or torch.overrides._get_current_function_mode_stack() \
-            or torch.utils._python_dispatch._get_current_dispatch_mode() is not None:
-        return False
-    if torch._C._functorch.is_functorch_wrapped_tensor(img) or torch._C._is_fwd_grad_enabled() and \
-            torch.autograd.forward_ad.unpack_dual(img).tangent is not None:
-        return False
-    return not (torch.is_grad_enabled() and img.requires_grad)
+    return not (torch.is_grad_enabled() and img.requires_grad) and not _observed(img)
 
 
 def _on_tv_kernels(img: torch.Tensor, eps: float) -> bool:
@@ -175,8 +187,9 @@ def _on_tv_kernels(img: torch.Tensor, eps: float) -> bool:
 def _elementwise(x: torch.Tensor, y: torch.Tensor, per_geom: torch.Tensor, *scalars) -> bool:
     """Whether the residual and update kernels take (x, y) with ``per_geom`` for every item: no
     broadcasting but that, and plain numbers as scalars."""
-    return (all(isinstance(s, (int, float)) for s in scalars) and per_geom.numel() <= 0xffffff00 and _plain(x) and _plain(y) and _plain(per_geom) and x.shape == y.shape and x.shape[-3:] == per_geom.shape
-            and x.device == y.device == per_geom.device)
+    return (all(isinstance(s, (int, float)) for s in scalars) and per_geom.numel() <= 0xffffff00
+            and x.shape == y.shape and x.shape[-3:] == per_geom.shape and x.device == y.device == per_geom.device
+            and _plain(x) and _plain(y) and _plain(per_geom))
 
 
 def _residual(p, ax, a, weighted: bool, eps: float = 0.0):
