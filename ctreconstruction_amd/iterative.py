@@ -151,12 +151,13 @@ def _normalise_pad(dtv: torch.Tensor, eps: float) -> torch.Tensor:
 
 def _observed(img: torch.Tensor) -> bool:
     """Whether something maps, differentiates forward, traces or intercepts torch's work on ``img``, which a
-    kernel called by address would pass by.  torch has no public form for some of these questions: where it
-    cannot answer one, the answer is yes."""
+    kernel called by address would pass by.  A default device (``torch.set_default_device``) does not count.
+    torch has no public form for some of these questions: where it cannot answer one, the answer is yes."""
     if torch.compiler.is_compiling() or torch.jit.is_tracing():
         return True
     try:
-        if torch.overrides._get_current_function_mode_stack():
+        modes = torch.overrides._get_current_function_mode_stack()
+        if any(type(m).__module__ != "torch.utils._device" for m in modes):
             return True
         if torch.utils._python_dispatch._get_current_dispatch_mode() is not None:
             return True

@@ -1,5 +1,5 @@
 """Which calls the total-variation, residual and update kernels take: anything that watches torch's work on a
-tensor keeps the torch expressions, and so does a torch that cannot tell."""
+tensor keeps the torch expressions, a default device does not, and so does a torch that cannot tell."""
 import pytest
 import torch
 from torch.autograd import forward_ad
@@ -28,6 +28,10 @@ class DispatchMode(TorchDispatchMode):
 def test_what_counts_as_observed():
     x = torch.zeros(3)
     assert not IT._observed(x)
+    with torch.device("cpu"):
+        assert not IT._observed(x)
+        with FunctionMode():
+            assert IT._observed(x)
     for mode in (FunctionMode(), DispatchMode()):
         with mode:
             assert IT._observed(x)
@@ -54,6 +58,21 @@ def _scan():
     N.lib()
     geom = ctr.ScanGeometry(make_params(NumberOfImage=[24, 20, 16], NumberOfViews=10, NumberOfDetectorPixels=[40, 30]))
     return geom, torch.rand(geom.proj_shape, generator=torch.Generator().manual_seed(0)).cuda()
+
+
+@pytest.mark.gpu
+def test_a_default_device_keeps_the_kernels(monkeypatch):
+    geom, proj = _scan()
+    x0 = torch.zeros(geom.vol_shape, device="cuda")
+    ref = IT.asd_pocs(proj, geom, n_outer=1, na=1, ng=3, x0=x0)
+    calls, plain = [], IT._plain
+    monkeypatch.setattr(IT, "_plain", lambda t: calls.append(plain(t)) or calls[-1])
+    torch.set_default_device("cuda")
+    try:
+        got = IT.asd_pocs(proj, geom, n_outer=1, na=1, ng=3, x0=x0)
+    finally:
+        torch.set_default_device(None)
+    assert calls and all(calls) and torch.equal(got, ref)
 
 
 @pytest.mark.gpu
