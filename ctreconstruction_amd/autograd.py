@@ -1,11 +1,11 @@
 """The DD projector as a differentiable torch operator.
 
 ``DDProjectorFunction`` computes y = A x with the HIP forward projector; its backward is the
-hand-written matched backprojector A^T (``ctr_dd_backproject`` in adjoint mode), so gradients
-of any loss of A x flow through the project's own kernels.  ``DDBackprojectorFunction`` is the
-transpose pair (y -> A^T y, backward A).  Both accept one volume [nz, ny, nx] or a batch
-[B, nz, ny, nx] (projections [nView, nv, nu] or [B, nView, nv, nu]); the items of a batch share
-launches on the current stream.
+hand-written matched backprojector A^T (``ctr_dd_backproject`` in adjoint mode,
+``ctr_dd_adjoint_batch`` for a batch), so gradients of any loss of A x flow through the project's
+own kernels.  ``DDBackprojectorFunction`` is the transpose pair (y -> A^T y, backward A).  Both
+accept one volume [nz, ny, nx] or a batch [B, nz, ny, nx] (projections [nView, nv, nu] or
+[B, nView, nv, nu]); the items of a batch share launches on the current stream.
 """
 from __future__ import annotations
 
@@ -15,28 +15,23 @@ from . import projector as P
 from .geometry import ScanGeometry
 
 
-def _batched(fn, x: torch.Tensor, item_shape, out_shape, geom):
+def _apply(one, many, x: torch.Tensor, item_shape, geom: ScanGeometry) -> torch.Tensor:
     x = x.contiguous()
     if tuple(x.shape) == tuple(item_shape):
-        return fn(x, geom)
-    if x.dim() == len(item_shape) + 1 and tuple(x.shape[1:]) == tuple(item_shape):
-        out = torch.empty((x.shape[0],) + tuple(out_shape), dtype=torch.float32, device=x.device)
-        for b in range(x.shape[0]):
-            fn(x[b], geom, out=out[b])
-        return out
+        return one(x, geom)
+    if x.dim() == 4 and tuple(x.shape[1:]) == tuple(item_shape):
+        return many(x, geom)
     raise ValueError(f"expected shape {tuple(item_shape)} or [B, *{tuple(item_shape)}], got {tuple(x.shape)}")
 
 
 def forward_batch(vol: torch.Tensor, geom: ScanGeometry) -> torch.Tensor:
-    if vol.dim() == 4 and tuple(vol.shape[1:]) == tuple(geom.vol_shape):
-        return P.dd_forward_batch(vol.contiguous(), geom)
-    return _batched(P.dd_forward, vol, geom.vol_shape, geom.proj_shape, geom)
+    """A x of one volume or of every volume of a batch."""
+    return _apply(P.dd_forward, P.dd_forward_batch, vol, geom.vol_shape, geom)
 
 
 def adjoint_batch(proj: torch.Tensor, geom: ScanGeometry) -> torch.Tensor:
-    if proj.dim() == 4 and tuple(proj.shape[1:]) == tuple(geom.proj_shape):
-        return P.dd_adjoint_batch(proj.contiguous(), geom)
-    return _batched(P.dd_adjoint, proj, geom.proj_shape, geom.vol_shape, geom)
+    """A^T y of one scan or of every scan of a batch."""
+    return _apply(P.dd_adjoint, P.dd_adjoint_batch, proj, geom.proj_shape, geom)
 
 
 class DDProjectorFunction(torch.autograd.Function):

@@ -70,7 +70,8 @@ def _gradient_operands(x: torch.Tensor, gout: torch.Tensor):
 
 
 def conv3x3_wgrad(x: torch.Tensor, gout: torch.Tensor, with_bias: bool = True):
-    """(grad_weight [Cout,3,3,Cin] float32, grad_bias [Cout] float32) summed over all pixels."""
+    """(grad_weight [Cout,3,3,Cin] float32, grad_bias [Cout] float32) summed over all pixels: the weight
+    half of :func:`conv3x3_backward`, for callers that need no input gradient (and no weights) or no bias."""
     n, h, w, cin, cout = _gradient_operands(x, gout)
     lib = N.lib()
     gw = torch.empty((cout, 3, 3, cin), dtype=torch.float32, device=x.device)
@@ -83,7 +84,8 @@ def conv3x3_wgrad(x: torch.Tensor, gout: torch.Tensor, with_bias: bool = True):
 
 
 def flip_transpose(w_bf16: torch.Tensor) -> torch.Tensor:
-    """Weights of the input-gradient convolution: w'[ci, ky, kx, co] = w[co, 2-ky, 2-kx, ci]."""
+    """Weights of the input-gradient convolution: w'[ci, ky, kx, co] = w[co, 2-ky, 2-kx, ci], for callers
+    that take that gradient by :func:`conv3x3_forward` (:func:`conv3x3_backward` flips them itself)."""
     return torch.flip(w_bf16, dims=(1, 2)).permute(3, 1, 2, 0).contiguous()
 
 
