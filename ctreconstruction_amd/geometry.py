@@ -13,6 +13,7 @@ from __future__ import annotations
 import math
 
 import numpy as np
+import torch
 
 from . import _native as N
 
@@ -128,22 +129,23 @@ class ScanGeometry:
         return b"".join((bytes(self.ctypes_struct()), np.float64(self.dtheta).tobytes(),
                          np.ascontiguousarray(self.angles).tobytes(), np.ascontiguousarray(self.branch).tobytes()))
 
-    def device_views(self, device):
+    def device_views(self, device, stream=None):
         """(angles float64, branch int32) device tensors, uploaded once per device and again when the
-        arrays have changed.  Their memory outlives the work of every stream that asked for them."""
-        import torch
-        key, contents = str(device), (self.angles.tobytes(), self.branch.tobytes())
-        stream = torch.cuda.current_stream(device)
-        hit = self._device_cache.get(key)
+        arrays have changed.  Their memory outlives the work of every stream that asked for them
+        (``stream``: the current one, where the caller has it at hand)."""
+        if stream is None:
+            stream = torch.cuda.current_stream(device)
+        contents = (self.angles.tobytes(), self.branch.tobytes())
+        hit = self._device_cache.get(device)
         if hit is None or hit[0] != contents:
             # copies from pageable memory: finished when they return
             ang = torch.from_numpy(np.array(self.angles, dtype=np.float64)).to(device)
             br = torch.from_numpy(np.array(self.branch, dtype=np.int32)).to(device)
-            hit = self._device_cache[key] = (contents, stream, ang, br)
-        elif hit[1] != stream:
-            for t in hit[2:]:
+            hit = self._device_cache[device] = (contents, stream.cuda_stream, (ang, br))
+        elif hit[1] != stream.cuda_stream:
+            for t in hit[2]:
                 t.record_stream(stream)
-        return hit[2:]
+        return hit[2]
 
     def __getstate__(self):
         """Copies and pickles upload their own views."""

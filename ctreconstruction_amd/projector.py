@@ -52,11 +52,12 @@ def dd_forward(vol: torch.Tensor, geom: ScanGeometry, out: torch.Tensor | None =
     _require(out, geom.proj_shape, "proj")
     lib = N.lib()
     g = geom.ctypes_struct()
-    ang, br = geom.device_views(dev)
+    stream = torch.cuda.current_stream(dev)
+    ang, br = geom.device_views(dev, stream)
     nbytes = lib.ctr_dd_forward_workspace_bytes(ctypes.byref(g))
     ws = _workspace(nbytes, dev)
     N.check(lib.ctr_dd_forward(ctypes.byref(g), _ptr(ang), _ptr(br), _ptr(vol), _ptr(out),
-                               _ptr(ws), nbytes, _stream(dev)), "ctr_dd_forward")
+                               _ptr(ws), nbytes, ctypes.c_void_p(stream.cuda_stream)), "ctr_dd_forward")
     return out
 
 
@@ -75,7 +76,8 @@ def dd_forward_batch(vol: torch.Tensor, geom: ScanGeometry) -> torch.Tensor:
     _require(vol, (batch,) + tuple(geom.vol_shape), "vol")
     lib = N.lib()
     g = geom.ctypes_struct()
-    ang, br = geom.device_views(dev)
+    stream = torch.cuda.current_stream(dev)
+    ang, br = geom.device_views(dev, stream)
     size = lambda n: lib.ctr_dd_forward_batch_workspace_bytes(ctypes.byref(g), n)  # noqa: E731
     most = max(1, min(batch, 4096, _FORWARD_TABLES // max(size(2) - size(1), 1)))
     launches = -(-batch // most)
@@ -84,8 +86,8 @@ def dd_forward_batch(vol: torch.Tensor, geom: ScanGeometry) -> torch.Tensor:
     ws = _workspace(nbytes, dev)
     for b in range(0, batch, per):
         n = min(per, batch - b)
-        N.check(lib.ctr_dd_forward_batch(ctypes.byref(g), _ptr(ang), _ptr(br), _ptr(vol[b]), _ptr(out[b]), n, _ptr(ws),
-                                         nbytes, _stream(dev)), "ctr_dd_forward_batch")
+        N.check(lib.ctr_dd_forward_batch(ctypes.byref(g), _ptr(ang), _ptr(br), _ptr(vol[b]), _ptr(out[b]), n,
+                                         _ptr(ws), nbytes, ctypes.c_void_p(stream.cuda_stream)), "ctr_dd_forward_batch")
     return out
 
 
@@ -154,7 +156,8 @@ def dd_backproject(proj: torch.Tensor, geom: ScanGeometry, mode: str = "ref", sc
     _require(out, geom.vol_shape, "vol")
     lib = N.lib()
     g = geom.ctypes_struct()
-    ang, br = geom.device_views(dev)
+    stream = torch.cuda.current_stream(dev)
+    ang, br = geom.device_views(dev, stream)
     m = N.BP_MODES[mode]
     nbytes = lib.ctr_dd_backproject_workspace_bytes(ctypes.byref(g), m)
     ws = _workspace(nbytes, dev)
@@ -162,7 +165,7 @@ def dd_backproject(proj: torch.Tensor, geom: ScanGeometry, mode: str = "ref", sc
         scale = 1.0 if mode == "adjoint" else geom.dtheta
     N.check(lib.ctr_dd_backproject(ctypes.byref(g), _ptr(ang), _ptr(br), _ptr(proj), _ptr(out), m,
                                    float(scale), float(zero_tol), int(bool(accumulate)), _ptr(ws),
-                                   nbytes, _stream(dev)), "ctr_dd_backproject")
+                                   nbytes, ctypes.c_void_p(stream.cuda_stream)), "ctr_dd_backproject")
     return out
 
 
@@ -186,7 +189,8 @@ def dd_adjoint_batch(proj: torch.Tensor, geom: ScanGeometry) -> torch.Tensor:
     geom.check_supported()
     lib = N.lib()
     g = geom.ctypes_struct()
-    ang, br = geom.device_views(dev)
+    stream = torch.cuda.current_stream(dev)
+    ang, br = geom.device_views(dev, stream)
     most = max(1, min(batch, 4096, _ADJOINT_TABLES // (4 * proj[0].numel())))
     launches = -(-batch // most)
     per = -(-batch // launches)
@@ -195,8 +199,9 @@ def dd_adjoint_batch(proj: torch.Tensor, geom: ScanGeometry) -> torch.Tensor:
     nbytes = max(size(n) for n in set(sizes))   # fewer scans may be split into more parts
     ws = _workspace(nbytes, dev)
     for i, n in enumerate(sizes):
-        N.check(lib.ctr_dd_adjoint_batch(ctypes.byref(g), _ptr(ang), _ptr(br), _ptr(proj[i * per]), _ptr(out[i * per]), n,
-                                         1.0, _ptr(ws), nbytes, _stream(dev)), "ctr_dd_adjoint_batch")
+        N.check(lib.ctr_dd_adjoint_batch(ctypes.byref(g), _ptr(ang), _ptr(br), _ptr(proj[i * per]), _ptr(out[i * per]),
+                                         n, 1.0, _ptr(ws), nbytes, ctypes.c_void_p(stream.cuda_stream)),
+                "ctr_dd_adjoint_batch")
     return out
 
 
