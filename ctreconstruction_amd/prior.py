@@ -112,7 +112,7 @@ def conv3x3_backward(x: torch.Tensor, w_bf16: torch.Tensor, gout: torch.Tensor, 
 class Conv3x3Function(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias, need_input_grad):
-        wb = weight.detach().to(BF16).contiguous()
+        wb = weight.detach().to(BF16)  # either direction makes it contiguous
         ctx.save_for_backward(x, wb)
         ctx.need_input_grad = need_input_grad
         return conv3x3_forward(x, wb, bias.detach())
@@ -120,7 +120,9 @@ class Conv3x3Function(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gout):
         x, wb = ctx.saved_tensors
-        return (*conv3x3_backward(x, wb, gout.to(BF16), ctx.need_input_grad), None)
+        if gout.dtype is not BF16:
+            gout = gout.to(BF16)
+        return (*conv3x3_backward(x, wb, gout, ctx.need_input_grad), None)
 
 
 class ResidualPrior(torch.nn.Module):
