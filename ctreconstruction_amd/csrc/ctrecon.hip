@@ -4,16 +4,18 @@
 //   fp_prepare_kernel           per-view DD footprint tables, FP64 -> FP32 (index space), and
 //                               vol[z][y][x] -> z-prefix tables [y][x][k] and [x][y][k]
 //   dd_forward_kernel           one wavefront per (2 views, 4 detector columns, 63 rows)
+//   dd_forward_thin_kernel      detectors of at most four rows: one lane per detector column
 //   dd_forward_zslab_kernel     z-slab views (non-circular geometries), FP64 loops per cell
 //   bp_geometry_kernel          per-view backprojection constants, FP64 -> FP32; clears the flags
 //   dd_backproject_tile_kernel  one workgroup per 16 x 16 x ZC voxel tile and view split, windows in LDS
+//   bp_slice_kernel             FDK backprojection of a single slice, gathered per pixel
 //   sum_parts_kernel            sums the view splits' partial volumes in a fixed order (splits.h)
 //   adj_geometry_kernel         footprint tables and constants of the inverse central projection
 //   adj_prepare_kernel          row prefix sums of projections times path length; detector windows of
 //                               every (view, column tile)
 //   dd_adjoint_kernel           exact transpose of the forward projector, gathered per voxel, windows in LDS
 //   spectrum_kernel             filter magnitude from the Ram-Lak cosine series, FP64
-//   twiddle_kernel              Stockham twiddles, stage-major, FP64 -> FP32
+//   twiddle_kernel              Stockham twiddles, stage-major, and the scaled spectrum, FP64 -> FP32
 //   fdk_filter_kernel           cosine weight + LDS Stockham FFT convolution, two rows per FFT
 //
 // Reference semantics are cited at each kernel (leehoy/CTReconstruction paths).
@@ -814,7 +816,8 @@ __global__ void __launch_bounds__(64 * kFpWaves * SPLIT, CTR_FP_MIN_WAVES) dd_fo
 // column's footprint over its width times the slab's magnification, the z integral of a line up to
 // the edge interpolated in the prefix table, FP64 sums over the slabs.  Neighbouring columns cross
 // neighbouring lines, so a wavefront's table reads are one short run while the lines are short.
-// Bound by VALU issue (290 cycles per wavefront and slab for a single row).  Measured: 256^2, 360 views
+// Bound by the wait for the lanes' table reads (the texture data unit busy 0.65 of the cycles) beside
+// VALU issue at 0.17 per SIMD-cycle (290 cycles per wavefront and slab for a single row).  Measured: 256^2, 360 views
 // of 512 columns: 1404 us by dd_forward_kernel (2 of 64 lanes at work), 88 us here; 256^2 x 64 and 256^3,
 // 360 views of 512 x 4 and x 3 cells: 1330 and 1362 us by that kernel, 610 and 560 us here, where each
 // lane's table reads touch a line of their own: more rows are left to that kernel.  Four slabs' reads
@@ -1110,8 +1113,11 @@ constexpr int kMaxRows = 19;                // rows per sub-chunk on the row-int
 // the last, and the registers for as many.  Measured, with one shape (the first) before: 256^3 x 360
 // views of 1024 x 768 cells, 1.9 cells per voxel, 80.6 -> 9.7 ms (Fine); 320 x 320 x 200 x 480 views,
 // 1.2 cells, 81.4 -> 11.2 ms (Medium; Fine 12.6); 192 x 192 x 100 x 300, 1.05 cells, 3.15 -> 1.42 ms
-// (Medium; Fine 1.50); 128^3 x 180, 1.0 cells, 0.51 -> 0.42 ms (Whole; Medium 0.52).  2048-cell windows
-// for Whole: 136 registers, three groups per CU, 18 % slower on a 151 x 163 x 107 helix.
+// (Medium; Fine 1.50); 128^3 x 180, 1.0 cells, 0.51 -> 0.42 ms (Whole; Medium 0.52).  Large volumes that
+// leave the first shape for a few straddling, short or cut sub-chunks, 512 x 512 from 720 views of
+// 1024 x 768: 496 slices 114.0 -> 72.6, 500 slices 114.2 -> 72.3, 400 slices 76.8 -> 59.3, 512 slices from 500
+// rows 75.3 -> 71.1, on a helix 78.2 -> 70.6 ms (Whole; 62.5 where all are plain).  2048-cell windows for
+// Whole: 136 registers, three groups per CU, 18 % slower on a 151 x 163 x 107 helix.
 template <int ZC_, int SUB_, int CAP_, int TAPS_>
 struct BpShape {
     static constexpr int ZC = ZC_, SUB = SUB_, CAP = CAP_, TAPS = TAPS_;
@@ -1620,7 +1626,7 @@ __device__ inline void bp_column_view(const BpView& v, const float* __restrict__
 // part or whole) to kBpRest, which adds those contributions; kBpAll does everything.
 // blockIdx.y is the view split: split s takes the views [s * views_per, (s + 1) * views_per) of
 // its tile and, where there is more than one, writes its sums to its own copy of the volume in
-// `parts`, which sum_parts_kernel adds up in split order (see bp_split).
+// `parts`, which sum_parts_kernel adds up in split order (see bp_plan).
 // GENERAL: the fast pass takes every sub-chunk that fits (bp_column_view_fast).
 template <int ZC, int KIND, typename S, bool GENERAL>
 __global__ void __launch_bounds__(256) dd_backproject_tile_kernel(
@@ -1819,8 +1825,8 @@ __global__ void __launch_bounds__(256) dd_backproject_tile_kernel(
 // The backprojection of a single slice (2-D fans): a column's row integral would serve one voxel,
 // so the footprint's few cells are gathered from memory (a wavefront's 8 x 8 pixels read neighbouring
 // cells, and a slice's views stay in L2) without windows or barriers.  Overlap weights as in
-// bp_column_view, weights below zero_tol dropped.  Bound by VALU issue (about 120 instructions per
-// pixel and view, half of them the four corners).  Measured: 256^2 x 360 views of a curved detector
+// bp_column_view, weights below zero_tol dropped.  Bound by VALU issue (0.293 per SIMD-cycle, about 120
+// instructions per pixel and view, half of them the four corners).  Measured: 256^2 x 360 views of a curved detector
 // 344 us by the tile kernel, 95 us here; 512^2 x 720 views 0.69 ms (three taps read at once instead of
 // one by one: 0.73).
 __global__ void __launch_bounds__(256) bp_slice_kernel(
@@ -1898,8 +1904,9 @@ constexpr int kAdjViewStride = 16;
 constexpr int kAdjCols = 127;  // most window columns
 
 // Work shape: TZ voxels per work-item, CAP floats per LDS window: fewer voxels where the detector is
-// finer (adj_choose: the tallest whose windows fit).  Bound by VALU issue (eight instructions and one
-// two-word LDS read per voxel boundary and candidate column, 2-3 columns per voxel).  Measured
+// finer (adj_choose: the tallest whose windows fit).  Bound by VALU issue (0.327 per SIMD-cycle, LDS busy
+// 0.46: eight instructions and one two-word LDS read per voxel boundary and candidate column, 2-3
+// columns per voxel).  Measured
 // against one 8-byte gather from the texture path per boundary: 128^3 x 180 views 1154 -> 234 us,
 // 256^3 x 60 views 1808 -> 525 us.
 template <int TZ_, int CAP_>
@@ -2848,8 +2855,8 @@ int static_scratch(void** out) {
     return CTR_OK;
 }
 
-// Work shape of the FDK backprojection (BpCoarse, BpFine, BpFinest) and whether its fast pass holds
-// the general voxel loop, from what one voxel, one sub-chunk and one tile project to.
+// Work shape of the FDK backprojection, and with it whether its fast pass holds the general voxel loop (all but
+// BpCoarse), from what one voxel, one sub-chunk and one tile project to.
 //
 // The common-case pass needs a sub-chunk's rows in its table, a footprint's columns in registers
 // and a tile's window in LDS; what does not fit is left to the completing pass, which gathers from
@@ -2928,7 +2935,8 @@ size_t bp_base_bytes(const ctr_geometry* g, BpKind shape) {
 // 241 views, 4.16 -> 3.89 ms at 256^3 x 360 views (2048 tiles: a nearly empty last wave).  2560 and
 // 10240 groups are up to 10 % slower on those than 5120 (too few in flight; more copies to add).
 // A split keeps at least kBpMinViews views (64^3 x 90: 98 us with 4, 116 with 8, 160 with 16).  The
-// copies take at most kBpTargetGroups tiles' worth of memory (168 MB).
+// copies take less than twice kBpTargetGroups tiles' worth of memory (335 MB; a volume of 5119 tiles
+// has two): the count is rounded up.
 constexpr int kBpTargetGroups = 5120;
 constexpr int kBpMinViews = 4;
 
@@ -3434,8 +3442,8 @@ int ctr_dd_backproject_static(const ctr_geometry* g, const double* angles, const
     if (!angles || !proj || !vol) return CTR_ERR_INVALID;
     void* ws = nullptr;
     if ((st = static_scratch(&ws))) return st;
-    // the same launches as ctr_dd_backproject: the per-view table is written by a kernel and
-    // the flags are cleared by a fill kernel on `stream` before use
+    // the same launches as ctr_dd_backproject: bp_geometry_kernel writes the per-view table and clears
+    // the flags on `stream` before use
     return bp_fdk(g, angles, proj, vol, mode, scale, zero_tol, accumulate, ws, bp_plan(g, kStaticScratchBytes),
                   (hipStream_t)stream);
 }

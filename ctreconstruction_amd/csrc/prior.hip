@@ -503,7 +503,7 @@ __global__ void __launch_bounds__(kPThreads) conv3x3_fwd_persistent_kernel(
 // cleared.  An instance of its own: in the common one that took 0.8 us of 33 at 16 x 128 x 128, whose
 // tiles are whole (103 x 54 x 140, 3 -> 64 channels, with it: 92.9 -> 95.8 us).
 // Bound by the staging: a tile's 75 KB take longer to arrive and be stored than its MFMAs (a
-// workgroup per CU, 2.8 TB/s).  Measured at 16 x 128 x 128, 64 -> 64 channels: 28 us, 690 TFLOP/s
+// workgroup per CU, 2.8 TB/s).  Measured at 16 x 128 x 128, 64 -> 64 channels: 27 us, 714 TFLOP/s
 // (118 us with one workgroup per (pixel chunk, tap) that wrote transposed copies of both operands to
 // LDS); at 103 x 54 x 140, 3 -> 64 channels 77 us (97 us without SPLIT, 450 us before).
 constexpr int kGTileH = 8, kGTileW = 32;

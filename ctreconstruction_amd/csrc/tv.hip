@@ -9,8 +9,10 @@
 //
 // A step is three launches: tv_pass_kernel<kTvNorm> sums g^2 per workgroup, tv_norm_kernel adds the
 // sums up per volume, and tv_pass_kernel evaluates g again and applies it.  g is recomputed rather
-// than stored: a pass reads the volume once (its planes stay in the caches) and is bound by VALU
-// issue, about as long as the 2 x 4 bytes per voxel that storing and rereading g would add.
+// than stored: a pass reads the volume about twice from beyond L2 (its planes stay in the caches) and is
+// bound by the vector memory path in front of them (seven reads per voxel: texture data unit busy 0.70-0.78,
+// address unit 0.59-0.69 of the cycles, VALU issue 0.17-0.19 per SIMD-cycle), about as long as the 2 x 4
+// bytes per voxel that storing and rereading g would add.
 // Measured per step, 8 x 128^3: about 950 us as some 25 torch elementwise and reduction kernels, 82 us
 // here (31 + 5 + 46).
 
