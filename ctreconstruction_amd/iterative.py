@@ -149,10 +149,10 @@ def _normalise_pad(dtv: torch.Tensor, eps: float) -> torch.Tensor:
     return torch.nn.functional.pad(dtv / norm, (1, 1, 1, 1, 1, 1))
 
 
-def _observed(img: torch.Tensor) -> bool:
-    """Whether something maps, differentiates forward, traces or intercepts torch's work on ``img``, which a
-    kernel called by address would pass by.  A default device (``torch.set_default_device``) does not count.
-    torch has no public form for some of these questions: where it cannot answer one, the answer is yes."""
+def _observed(*tensors: torch.Tensor) -> bool:
+    """Whether something maps, differentiates forward, traces or intercepts torch's work on one of ``tensors``,
+    which a kernel called by address would pass by.  A default device (``torch.set_default_device``) does not
+    count.  torch has no public form for some of these questions: where it cannot answer one, the answer is yes."""
     if torch.compiler.is_compiling() or torch.jit.is_tracing():
         return True
     try:
@@ -161,21 +161,26 @@ def _observed(img: torch.Tensor) -> bool:
             return True
         if torch.utils._python_dispatch._get_current_dispatch_mode() is not None:
             return True
-        if torch._C._functorch.is_functorch_wrapped_tensor(img):
+        if any(map(torch._C._functorch.is_functorch_wrapped_tensor, tensors)):
             return True
-        return torch.autograd.forward_ad.unpack_dual(img).tangent is not None
+        return any(torch.autograd.forward_ad.unpack_dual(t).tangent is not None for t in tensors)
     except (AttributeError, ImportError):
         return True
 
 
-def _plain(img: torch.Tensor) -> bool:
-    """Whether a kernel may take ``img``: a contiguous float32 batch of volumes (or projections) on the
-    GPU that nothing differentiates or observes (the torch expressions serve everything else)."""
-    if type(img) is not torch.Tensor or img.device.type != "cuda" or img.dtype != torch.float32:
-        return False
-    if img.dim() < 3 or not img.is_contiguous() or img.numel() == 0 or img.shape[:-3].numel() > 65535:
-        return False
-    return not (torch.is_grad_enabled() and img.requires_grad) and not _observed(img)
+def _plain(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel may take ``tensors``: contiguous float32 batches of volumes (or projections) on the
+    current GPU that nothing differentiates or observes (the torch expressions serve everything else,
+    other GPUs among it: a default stream's handle does not name its device)."""
+    gpu = torch.cuda.current_device() if torch.cuda.is_initialized() else None
+    for t in tensors:
+        if type(t) is not torch.Tensor or not t.is_cuda or t.dtype is not torch.float32 or t.get_device() != gpu:
+            return False
+        if t.dim() < 3 or not t.is_contiguous() or t.numel() == 0 or t.shape[:-3].numel() > 65535:
+            return False
+        if t.requires_grad and torch.is_grad_enabled():
+            return False
+    return not _observed(*tensors)
 
 
 def _on_tv_kernels(img: torch.Tensor, eps: float) -> bool:
@@ -190,7 +195,7 @@ def _elementwise(x: torch.Tensor, y: torch.Tensor, per_geom: torch.Tensor, *scal
     broadcasting but that, and plain numbers as scalars."""
     return (all(isinstance(s, (int, float)) for s in scalars) and per_geom.numel() <= 0xffffff00
             and x.shape == y.shape and x.shape[-3:] == per_geom.shape and x.device == y.device == per_geom.device
-            and _plain(x) and _plain(y) and _plain(per_geom))
+            and _plain(x, y, per_geom))
 
 
 def _residual(p, ax, a, weighted: bool, eps: float = 0.0):

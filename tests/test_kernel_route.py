@@ -66,7 +66,7 @@ def test_a_default_device_keeps_the_kernels(monkeypatch):
     x0 = torch.zeros(geom.vol_shape, device="cuda")
     ref = IT.asd_pocs(proj, geom, n_outer=1, na=1, ng=3, x0=x0)
     calls, plain = [], IT._plain
-    monkeypatch.setattr(IT, "_plain", lambda t: calls.append(plain(t)) or calls[-1])
+    monkeypatch.setattr(IT, "_plain", lambda *t: calls.append(plain(*t)) or calls[-1])
     torch.set_default_device("cuda")
     try:
         got = IT.asd_pocs(proj, geom, n_outer=1, na=1, ng=3, x0=x0)
